@@ -18,7 +18,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_NAME = "librnn_kernel_amd.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 SOURCES = ["rka_capi.hip", "gemm_f32.hip", "gru_recurrence.hip", "gru_rec_tiled.hip", "gru_rec_reg.hip",
-           "gru_rec_bwd1.hip", "gru_rec_fwd1.hip", "train_ops.hip", "probes.hip"]
+           "gru_rec_bwd1.hip", "gru_rec_fwd1.hip", "gru_rec_wide.hip", "train_ops.hip", "probes.hip"]
 ARCH = "gfx950"
 # Flags of single sources on top of compile_flags().  The machine-scheduler
 # strategy is an option per translation unit: the one-row kernels that

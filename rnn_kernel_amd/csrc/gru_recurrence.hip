@@ -6,7 +6,10 @@
 // launch of a grid that is resident on an idle GPU; a batch whose grid is
 // not resident runs as several launches over batch slices):
 //   register-resident (gru_rec_reg.hip)  hidden <= 256, W_hh slice in VGPRs;
-//   LDS-tiled         (gru_rec_tiled.hip) any hidden whose tile fits LDS.
+//   wide              (gru_rec_wide.hip) hidden 257 to 768, likewise, four
+//                     rows and 32 units per workgroup;
+//   LDS-tiled         (gru_rec_tiled.hip) any hidden whose tile fits LDS
+//                     (on request, or where the others' grid is not resident).
 #include "rec_common.h"
 
 #include <atomic>
@@ -94,20 +97,27 @@ int choose_rec_config(int dir, int batch, int hidden, const DeviceInfo& dev, Rec
         clear_error();
         return 0;
     }
+    if (wide_takes(hidden) && wide_choose(dir, batch, hidden, dev, cfg) == 0) {
+        clear_error();
+        return 0;
+    }
     return tiled_choose(dir, batch, hidden, dev, 0, 0, cfg);
 }
 
 namespace {
-// Two exchange slots of [B, 4H] words (the largest user is the backward's
-// [B, 3H] gate gradients), one start-up XCD word per workgroup, then a
-// 256-byte trailer holding the abort flag.
-size_t slots_bytes(int batch, int hidden) {
-    return align_up((size_t)2 * batch * 4 * hidden * sizeof(unsigned long long), 256);
+// Two exchange slots of [B, 4H] words (the largest user among the kernels
+// that exchange rows is the backward's [B, 3H] gate gradients) or, if more,
+// the words of the wide kernels, then one start-up XCD word per workgroup and
+// a 256-byte trailer holding the abort flag.
+size_t slots_bytes(int dir, int batch, int hidden) {
+    size_t words = (size_t)2 * batch * 4 * hidden;
+    if (wide_takes(hidden)) words = std::max(words, wide_exchange_words(dir, batch, hidden));
+    return align_up(words * sizeof(unsigned long long), 256);
 }
 constexpr size_t kXccBytes = (size_t)rec::MAX_XCC_BLOCKS * sizeof(unsigned long long);
 }  // namespace
 
-size_t rec_workspace_bytes(int batch, int hidden) { return slots_bytes(batch, hidden) + kXccBytes + 256; }
+size_t rec_workspace_bytes(int dir, int batch, int hidden) { return slots_bytes(dir, batch, hidden) + kXccBytes + 256; }
 
 namespace {
 
@@ -126,6 +136,9 @@ __global__ void fill_u64_kernel(unsigned long long* __restrict__ slots, size_t n
     if (blockIdx.x == 0 && threadIdx.x == 0) *abort_flag = 0;
 }
 
+// Whether a configuration is the wide kernels' (register-resident past 256).
+bool is_wide(const RecConfig& c, int H) { return c.kind == REC_REGISTER && wide_takes(H); }
+
 // Launches the recurrence of direction `dir` over the whole batch: one
 // launch per batch slice of c.batch_per_launch rows (pointers offset to the
 // slice's rows).  Slice k uses its own part of the exchange slots (words
@@ -133,6 +146,8 @@ __global__ void fill_u64_kernel(unsigned long long* __restrict__ slots, size_t n
 // backward) and start-up XCD words tagged with k, so consecutive time ranges
 // of a chunked backward continue each slice on the same, once-zeroed
 // workspace: tags are (steps done before this range) * launches + k + 1.
+// The wide backward's slices use the same words, each with a step-tag base of
+// its own (k T).
 int launch_slices(int dir, const RecConfig& c, rec::Args a, unsigned long long* xcc_base, hipStream_t stream) {
     const int B = a.B, T = a.T, H = a.H;
     const size_t W = (size_t)(dir == 0 ? 1 : 3) * H;
@@ -154,11 +169,15 @@ int launch_slices(int dir, const RecConfig& c, rec::Args a, unsigned long long* 
         s.h0 = off(a.h0, (size_t)H);
         s.y = off(a.y, (size_t)T * H);
         s.reserve = off(a.reserve, (size_t)T * 4 * H);
-        s.exch = const_cast<unsigned long long*>(exch0) + 2 * (size_t)r0 * W;
+        const bool wide = is_wide(c, H);
+        s.exch = const_cast<unsigned long long*>(exch0) + (wide && dir == 1 ? 0 : 2 * (size_t)r0 * W);
+        if (wide && dir == 1) s.tag_base = (unsigned)k * (unsigned)T;
         const size_t blocks = (size_t)grid_groups(cs, cs.groups) * cs.slices;
         s.xcc_words = blocks <= (size_t)rec::MAX_XCC_BLOCKS && !g_agent_stores.load() ? xcc_base : nullptr;
         s.xcc_tag = (unsigned)((size_t)(T - a.t_end) * c.launches + k + 1);
-        if (cs.kind == REC_REGISTER) {
+        if (wide) {
+            RKA_RETURN_IF_ERR(wide_launch(dir, cs, s, stream));
+        } else if (cs.kind == REC_REGISTER) {
             RKA_RETURN_IF_ERR(reg_launch(dir, cs, s, stream));
         } else {
             RKA_RETURN_IF_ERR(tiled_launch(dir, cs, s, stream));
@@ -193,7 +212,8 @@ int launch_at(int dir, rec::Args& a, const RecState& st, bool zero_ws, hipStream
     // holds [B, H] words in the forward and [B, 3H] in the backward.  A range
     // launch that continues the previous one keeps its slots (tags grow).
     if (zero_ws) {
-        const size_t n_slots = (size_t)2 * a.B * (dir == 0 ? 1 : 3) * a.H;
+        const size_t n_slots =
+            is_wide(c, a.H) ? wide_exchange_words(dir, a.B, a.H) : (size_t)2 * a.B * (dir == 0 ? 1 : 3) * a.H;
         const size_t blocks = (size_t)grid_groups(c, c.groups) * c.slices;
         const size_t n_xcc = blocks <= (size_t)rec::MAX_XCC_BLOCKS ? blocks : 0;
         const size_t n = n_slots + n_xcc;
@@ -207,13 +227,13 @@ int launch_at(int dir, rec::Args& a, const RecState& st, bool zero_ws, hipStream
 }
 
 int launch(int dir, rec::Args& a, void* ws, size_t ws_bytes, bool zero_ws, hipStream_t stream) {
-    const size_t need = rec_workspace_bytes(a.B, a.H);
+    const size_t need = rec_workspace_bytes(dir, a.B, a.H);
     if (ws == nullptr || ws_bytes < need)
         return fail(RKA_ERR_WORKSPACE_TOO_SMALL, "recurrence workspace too small: need " + std::to_string(need) +
                                                      " bytes, got " + std::to_string(ws_bytes));
     char* base = reinterpret_cast<char*>(ws);
     const RecState st{reinterpret_cast<unsigned long long*>(base),
-                      reinterpret_cast<unsigned long long*>(base + slots_bytes(a.B, a.H)),
+                      reinterpret_cast<unsigned long long*>(base + slots_bytes(dir, a.B, a.H)),
                       reinterpret_cast<int*>(base + need - 256)};
     return launch_at(dir, a, st, zero_ws, stream);
 }

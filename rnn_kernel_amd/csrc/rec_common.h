@@ -71,7 +71,8 @@ struct Args {
     // that share exchange memory across calls (the allocation-free forward)
     // take a different base per call, so a word left or written by another
     // call never matches; with a private, freshly zeroed workspace it is 0
-    // (the backward, which has no allocation-free entry point, ignores it).
+    // (the backward has no allocation-free entry point; its wide form takes
+    // a base per batch slice, whose launches share the exchange words).
     unsigned tag_base = 0;
     // Failure injection for tests (-1: off): the workgroup with this block
     // index publishes every word into the other step-parity slot, where its
@@ -325,5 +326,13 @@ int tiled_launch(int dir, const RecConfig& c, const rec::Args& a, hipStream_t st
 // Register-resident kernels (W_hh slice in VGPRs; hidden size <= 256).
 int reg_choose(int dir, int B, int H, const DeviceInfo& dev, int fixed_units, int fixed_rows, RecConfig* cfg);
 int reg_launch(int dir, const RecConfig& c, const rec::Args& a, hipStream_t stream);
+
+// Register-resident kernels for hidden sizes 257 to 768 (four rows and 32
+// units per workgroup).
+bool wide_takes(int H);
+int wide_choose(int dir, int B, int H, const DeviceInfo& dev, RecConfig* cfg);
+int wide_launch(int dir, const RecConfig& c, const rec::Args& a, hipStream_t stream);
+// 64-bit exchange words a call needs (both slots).
+size_t wide_exchange_words(int dir, int B, int H);
 
 }  // namespace rka

@@ -4,6 +4,7 @@
 // gemm_f32.hip and gru_recurrence.hip.
 #include "rka_internal.h"
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -66,7 +67,7 @@ FwdLayout fwd_layout(int B, int T, int I, int H) {
     FwdLayout l{};
     l.gx = 0;
     l.rec = align_up((size_t)B * T * 3 * H * sizeof(float), 256);
-    l.total = l.rec + rec_workspace_bytes(B, H);
+    l.total = l.rec + rec_workspace_bytes(0, B, H);
     return l;
 }
 
@@ -83,7 +84,7 @@ BwdLayout bwd_layout(int B, int T, int I, int H) {
     l.ks_ih = choose_ksplit(3 * H, I, K, 128, 3);
     l.g = 0;
     l.rec = align_up((size_t)B * T * 4 * H * sizeof(float), 256);
-    l.part_hh = l.rec + align_up(rec_workspace_bytes(B, H), 256);
+    l.part_hh = l.rec + align_up(rec_workspace_bytes(1, B, H), 256);
     l.part_ih = l.part_hh + align_up(splitk_partial_floats(3 * H, H, l.ks_hh) * sizeof(float), 256);
     l.total = l.part_ih + align_up(splitk_partial_floats(3 * H, I, l.ks_ih) * sizeof(float), 256);
     return l;
@@ -176,7 +177,7 @@ size_t rka_gru_backward_workspace_bytes(int batch, int seq_len, int input_size, 
 
 size_t rka_gru_recurrence_workspace_bytes(int batch, int hidden_size) {
     if (batch < 1 || hidden_size < 1) return 0;
-    return rec_workspace_bytes(batch, hidden_size);
+    return std::max(rec_workspace_bytes(0, batch, hidden_size), rec_workspace_bytes(1, batch, hidden_size));
 }
 
 int rka_gru_forward(const float* x, const float* h0, const float* w_ih, const float* w_hh,
@@ -201,7 +202,7 @@ int rka_gru_forward(const float* x, const float* h0, const float* w_ih, const fl
     // the GEMM also clears the recurrence's exchange state (slots, start-up
     // XCD words, abort flag), which saves the recurrence its fill launch
     unsigned long long* rec_state = reinterpret_cast<unsigned long long*>(ws + l.rec);
-    const size_t rec_words = rec_workspace_bytes(B, H) / sizeof(unsigned long long);
+    const size_t rec_words = rec_workspace_bytes(0, B, H) / sizeof(unsigned long long);
     {
         StageScope scope(0, s);
         RKA_RETURN_IF_ERR(gemm_direct(B * T, 3 * H, I, a, b, b_ih, gx, 3 * H, s, SegMap{}, rec_state, rec_words));

@@ -166,7 +166,7 @@ void set_rec_agent_stores(bool on);
 // the library was loaded (synchronises the device).
 int rec_abort_count(unsigned long long* count);
 
-size_t rec_workspace_bytes(int batch, int hidden);
+size_t rec_workspace_bytes(int dir, int batch, int hidden);
 int eval_gate_functions(const float* x, float* sig, float* th, int n, hipStream_t stream);
 
 // zero_ws false: the workspace's recurrence state was cleared by an earlier
