@@ -8,13 +8,18 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace rka {
 namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMaxReduceBlocks = 2048;   // partial sums of a loss reduction
-constexpr int kHeadBlocks = 512;         // row ranges of the head's dw reduction
+// Elements one block reduces by itself, without the second launch (back to back
+// on MI355X 3.5 us from 16 to 16384 elements, against 5.8 us for the two
+// launches):
+constexpr size_t kMseOneBlock = 16384;
+constexpr int kHeadBlocks = 1024;        // row ranges of the head's dw reduction at most
 
 // Sum over the block's threads in a fixed order: each wavefront's 64 values
 // by a butterfly of lane exchanges, then the four wavefront sums in order
@@ -56,10 +61,12 @@ __device__ __forceinline__ float4 load_streaming(const float4* p) {
 // elements.  Vector form (chunk a multiple of 4, both operands 16-byte
 // aligned): thread t takes float4 t, t + 256, ... of the range into four
 // running sums (one per component), combined as (s0 + s1) + (s2 + s3);
-// scalar form: elements t, t + 256, ... into one sum.
+// scalar form: elements t, t + 256, ... into one sum.  A single block (loss
+// set) writes the mean itself.
 __global__ __launch_bounds__(kThreads) void mse_partial_kernel(const float* __restrict__ pred,
                                                                const float* __restrict__ target, size_t n,
-                                                               size_t chunk, int vec, float* __restrict__ partial) {
+                                                               size_t chunk, int vec, float* __restrict__ partial,
+                                                               float* __restrict__ loss) {
     __shared__ float scratch[kThreads / 64];
     const size_t beg = (size_t)blockIdx.x * chunk;
     const size_t end = beg + chunk < n ? beg + chunk : n;
@@ -91,7 +98,12 @@ __global__ __launch_bounds__(kThreads) void mse_partial_kernel(const float* __re
         }
     }
     const float s = block_sum_waves(acc, scratch);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s;
+    if (threadIdx.x == 0) {
+        if (loss)
+            loss[0] = s / (float)n;
+        else
+            partial[blockIdx.x] = s;
+    }
 }
 
 // loss[0] = (sum of the nb <= kMaxReduceBlocks partials, thread t summing
@@ -146,75 +158,221 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // Blocks of the loss reduction and the range of each (a multiple of 4).
 int mse_blocks(size_t n, size_t* chunk) {
     const size_t nb = std::min<size_t>(kMaxReduceBlocks, (n + 4095) / 4096);
-    const size_t b = nb < 1 ? 1 : nb;
+    const size_t b = nb < 1 || n <= kMseOneBlock ? 1 : nb;
     *chunk = ((n + b - 1) / b + 3) / 4 * 4;
     return (int)((n + *chunk - 1) / *chunk);
 }
 
 // ----------------------------------------------------------------- head ---
-// pred[r] = sum_h out[r, h] w[h] + b[0]; one wavefront per row, lane l
-// summing h = l, l + 64, ... in order, then a fixed butterfly across lanes.
+// A team of TEAM lanes (a power of two) takes a row, four columns a lane: VEC
+// columns 4 l .. 4 l + 3 as one float4 (hidden a multiple of 4, rows 16-byte
+// aligned), else columns l + TEAM j.  Up to 256 columns a team covers the row
+// (narrow heads then keep all 64 lanes busy with 64 / TEAM rows); wider rows go
+// 256 columns at a time.  Both passes are HBM-bound and keep kHeadUnroll rows
+// per team in flight.
+constexpr int kHeadUnroll = 4;
+
+template <int TEAM, bool VEC>
+__device__ __forceinline__ int head_col(int l, int j) {
+    return VEC ? 4 * l + j : l + TEAM * j;
+}
+
+// Four columns (from c0) of a row; zero past hidden.
+template <int TEAM, bool VEC>
+__device__ __forceinline__ float4 head_load(const float* __restrict__ row, int c0, int l, int hidden) {
+    if constexpr (VEC) {
+        const int c = c0 + 4 * l;
+        return c < hidden ? *reinterpret_cast<const float4*>(row + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    } else {
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int c = c0 + head_col<TEAM, VEC>(l, j);
+            v[j] = c < hidden ? row[c] : 0.f;
+        }
+        return make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+
+// pred[r] = sum_h out[r, h] w[h] + b[0]: each lane sums its columns in order,
+// then a fixed butterfly across the team.  B = 256, T = 1024, hidden = 256 on
+// MI355X: 92 -> 60 us (4.5 TB/s; one row per wavefront with 4-byte loads before).
+template <int TEAM, bool VEC>
 __global__ __launch_bounds__(kThreads) void head_forward_kernel(const float* __restrict__ out,
                                                                 const float* __restrict__ w,
                                                                 const float* __restrict__ b, int rows, int hidden,
                                                                 float* __restrict__ pred) {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const float* o = out + (size_t)row * hidden;
-    float acc = 0.f;
-    for (int h = lane; h < hidden; h += 64) acc = fmaf(o[h], w[h], acc);
+    constexpr int RPB = kThreads / TEAM;  // rows per block and pass
+    const int l = threadIdx.x % TEAM;
+    const size_t r0 = (size_t)blockIdx.x * RPB * kHeadUnroll + threadIdx.x / TEAM;
+    const size_t last = (size_t)rows - 1;
+    float acc[kHeadUnroll];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-    if (lane == 0) pred[row] = acc + b[0];
-}
-
-// dout[r, h] = dpred[r] w[h] (if dout), and per row range of block k:
-// partial[k][h] = sum_r dpred[r] out[r, h], partial[k][hidden] = sum_r dpred[r]
-// (rows in order, thread t owning h = t, t + 256, ...).
-__global__ __launch_bounds__(kThreads) void head_backward_partial_kernel(
-    const float* __restrict__ out, const float* __restrict__ w, const float* __restrict__ dpred, int rows,
-    int hidden, int rows_per_block, float* __restrict__ dout, float* __restrict__ partial) {
-    const int r0 = blockIdx.x * rows_per_block;
-    const int r1 = min(rows, r0 + rows_per_block);
-    float* part = partial + (size_t)blockIdx.x * (hidden + 1);
-    for (int h = threadIdx.x; h <= hidden; h += kThreads) {
-        const bool bias = h == hidden;
-        const float wh = bias ? 0.f : w[h];
-        float acc = 0.f;
-#pragma unroll 8
-        for (int r = r0; r < r1; ++r) {
-            const float g = dpred[r];
-            if (bias) {
-                acc += g;
-            } else {
-                const size_t idx = (size_t)r * hidden + h;
-                acc = fmaf(g, out[idx], acc);
-                if (dout) dout[idx] = g * wh;
-            }
+    for (int k = 0; k < kHeadUnroll; ++k) acc[k] = 0.f;
+    for (int c0 = 0; c0 < hidden; c0 += 4 * TEAM) {
+        const float4 wv = head_load<TEAM, VEC>(w, c0, l, hidden);
+        float4 o[kHeadUnroll];
+#pragma unroll
+        for (int k = 0; k < kHeadUnroll; ++k) {
+            const size_t r = r0 + k * RPB < last ? r0 + k * RPB : last;
+            o[k] = head_load<TEAM, VEC>(out + r * hidden, c0, l, hidden);
         }
-        part[h] = acc;
+#pragma unroll
+        for (int k = 0; k < kHeadUnroll; ++k)
+            acc[k] = fmaf(o[k].w, wv.w, fmaf(o[k].z, wv.z, fmaf(o[k].y, wv.y, fmaf(o[k].x, wv.x, acc[k]))));
+    }
+#pragma unroll
+    for (int k = 0; k < kHeadUnroll; ++k) {
+#pragma unroll
+        for (int off = TEAM / 2; off > 0; off >>= 1) acc[k] += __shfl_xor(acc[k], off, TEAM);
+        const size_t r = r0 + k * RPB;
+        if (l == 0 && r <= last) pred[r] = acc[k] + b[0];
     }
 }
 
-// dw[h] = sum_k partial[k][h] (k in order); db[0] = sum_k partial[k][hidden]
+// dout[r, h] = dpred[r] w[h] (if dout), and per row range of block x:
+// part[h] = sum_r dpred[r] out[r, h], part[hidden] = sum_r dpred[r], where part
+// is partial + x (hidden + 1), or, with one block (partial NULL), dw and db
+// themselves.  Team k of the block takes rows k, k + RPB, ... of the range in
+// order; the block's teams are added in LDS in a fixed order.  blockIdx.y: the
+// 256 columns a team takes.  Same shape: 298 -> 88 us (6.1 TB/s; before, 512
+// blocks, and the bias sum was a second serial pass of one thread over the rows).
+template <int TEAM, bool VEC>
+__global__ __launch_bounds__(kThreads) void head_backward_partial_kernel(
+    const float* __restrict__ out, const float* __restrict__ w, const float* __restrict__ dpred, int rows,
+    int hidden, int rows_per_block, float* __restrict__ dout, float* __restrict__ partial, float* __restrict__ dw,
+    float* __restrict__ db) {
+    constexpr int RPB = kThreads / TEAM;
+    __shared__ float lds[RPB][4 * TEAM];
+    __shared__ float lds_b[RPB];
+    const int l = threadIdx.x % TEAM, team = threadIdx.x / TEAM;
+    const size_t r0 = (size_t)blockIdx.x * rows_per_block;
+    const size_t r1 = r0 + rows_per_block < (size_t)rows ? r0 + rows_per_block : (size_t)rows;
+    float* part = partial ? partial + (size_t)blockIdx.x * (hidden + 1) : nullptr;
+    for (int c0 = blockIdx.y * 4 * TEAM; c0 < hidden; c0 += gridDim.y * 4 * TEAM) {
+        const float4 wv = head_load<TEAM, VEC>(w, c0, l, hidden);
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        float accb = 0.f;
+        for (size_t r = r0 + team; r < r1; r += RPB * kHeadUnroll) {
+            float g[kHeadUnroll];
+            float4 o[kHeadUnroll];
+#pragma unroll
+            for (int k = 0; k < kHeadUnroll; ++k) {
+                const size_t rr = r + k * RPB < r1 ? r + k * RPB : r1 - 1;
+                g[k] = dpred[rr];
+                o[k] = head_load<TEAM, VEC>(out + rr * hidden, c0, l, hidden);
+            }
+#pragma unroll
+            for (int k = 0; k < kHeadUnroll; ++k) {
+                const size_t rk = r + k * RPB;
+                if (rk >= r1) break;
+                acc.x = fmaf(g[k], o[k].x, acc.x);
+                acc.y = fmaf(g[k], o[k].y, acc.y);
+                acc.z = fmaf(g[k], o[k].z, acc.z);
+                acc.w = fmaf(g[k], o[k].w, acc.w);
+                accb += g[k];
+                if (dout) {
+                    float* d = dout + rk * hidden + c0;
+                    const float v[4] = {g[k] * wv.x, g[k] * wv.y, g[k] * wv.z, g[k] * wv.w};
+                    if constexpr (VEC) {
+                        if (c0 + 4 * l < hidden)
+                            *reinterpret_cast<float4*>(d + 4 * l) = make_float4(v[0], v[1], v[2], v[3]);
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const int c = head_col<TEAM, VEC>(l, j);
+                            if (c0 + c < hidden) d[c] = v[j];
+                        }
+                    }
+                }
+            }
+        }
+        const float a4[4] = {acc.x, acc.y, acc.z, acc.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) lds[team][head_col<TEAM, VEC>(l, j)] = a4[j];
+        if (l == 0) lds_b[team] = accb;
+        __syncthreads();
+        for (int c = threadIdx.x; c < 4 * TEAM && c0 + c < hidden; c += kThreads) {
+            float sum = lds[0][c];
+#pragma unroll 4
+            for (int k = 1; k < RPB; ++k) sum += lds[k][c];
+            (part ? part : dw)[c0 + c] = sum;
+        }
+        if (threadIdx.x == 0 && c0 == 0) {
+            float sum = lds_b[0];
+            for (int k = 1; k < RPB; ++k) sum += lds_b[k];
+            (part ? part + hidden : db)[0] = sum;
+        }
+        __syncthreads();
+    }
+}
+
+// dw[h] = sum_k partial[k][h]; db[0] = sum_k partial[k][hidden].  A block takes
+// 16 columns with 16 threads each: thread p sums the partials p, p + 16, ... in
+// order (eight loads in flight), then the sixteen are added in order.  Same
+// shape: 119 -> 4.9 us (before, one thread per column over 512 partials).
+constexpr int kFinishCols = 16;
 __global__ __launch_bounds__(kThreads) void head_backward_finish_kernel(const float* __restrict__ partial, int nb,
                                                                         int hidden, float* __restrict__ dw,
                                                                         float* __restrict__ db) {
-    const int h = blockIdx.x * kThreads + threadIdx.x;
-    if (h > hidden) return;
+    constexpr int P = kThreads / kFinishCols;
+    __shared__ float lds[P][kFinishCols + 1];
+    const int c = threadIdx.x % kFinishCols, p = threadIdx.x / kFinishCols;
+    const int h = blockIdx.x * kFinishCols + c;
     float acc = 0.f;
-    for (int k = 0; k < nb; ++k) acc += partial[(size_t)k * (hidden + 1) + h];
+    if (h <= hidden) {
+#pragma unroll 8
+        for (int k = p; k < nb; k += P) acc += partial[(size_t)k * (hidden + 1) + h];
+    }
+    lds[p][c] = acc;
+    __syncthreads();
+    if (p != 0 || h > hidden) return;
+    float sum = lds[0][c];
+#pragma unroll
+    for (int k = 1; k < P; ++k) sum += lds[k][c];
     if (h < hidden)
-        dw[h] = acc;
+        dw[h] = sum;
     else
-        db[0] = acc;
+        db[0] = sum;
 }
 
-int head_blocks(int rows, int* rows_per_block) {
-    const int nb = std::max(1, std::min(kHeadBlocks, rows));
-    *rows_per_block = (rows + nb - 1) / nb;
-    return (rows + *rows_per_block - 1) / *rows_per_block;
+// Lanes per row: the fewest (from 4) whose four columns each cover it.
+int head_team(int hidden) {
+    int team = 4;
+    while (team < 64 && 4 * team < hidden) team *= 2;
+    return team;
+}
+
+bool head_vec(int hidden, const void* a, const void* b, const void* c) {
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c);
+    return hidden % 4 == 0 && (bits & 15u) == 0;
+}
+
+// Row ranges of the backward: at least four passes of a block's teams each,
+// so that small heads end in few partials (one: no second pass).
+int head_blocks(int rows, int hidden, int* rows_per_block) {
+    const int pass = kThreads / head_team(hidden) * kHeadUnroll;
+    const int least = 4 * pass;
+    *rows_per_block = std::max(least, ((rows - 1) / kHeadBlocks + pass) / pass * pass);
+    return (rows - 1) / *rows_per_block + 1;
+}
+
+// Calls f(team, vec) with both as integral constants.
+template <typename F>
+void with_head_form(int hidden, bool vec, F f) {
+    auto pick = [&](auto team) {
+        if (vec)
+            f(team, std::true_type{});
+        else
+            f(team, std::false_type{});
+    };
+    switch (head_team(hidden)) {
+        case 4: pick(std::integral_constant<int, 4>{}); break;
+        case 8: pick(std::integral_constant<int, 8>{}); break;
+        case 16: pick(std::integral_constant<int, 16>{}); break;
+        case 32: pick(std::integral_constant<int, 32>{}); break;
+        default: pick(std::integral_constant<int, 64>{}); break;
+    }
 }
 
 // ---------------------------------------------------------------- AdamW ---
@@ -283,10 +441,13 @@ int rka_mse_forward(const float* pred, const float* target, float* loss, void* w
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     float* partial = reinterpret_cast<float*>(workspace);
     const int vec = (aligned16(pred) && aligned16(target)) ? 1 : 0;
-    hipLaunchKernelGGL(mse_partial_kernel, dim3(nb), dim3(kThreads), 0, s, pred, target, n, chunk, vec, partial);
+    hipLaunchKernelGGL(mse_partial_kernel, dim3(nb), dim3(kThreads), 0, s, pred, target, n, chunk, vec, partial,
+                       nb == 1 ? loss : nullptr);
     RKA_RETURN_IF_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mse_finish_kernel, dim3(1), dim3(kThreads), 0, s, partial, nb, n, loss);
-    RKA_RETURN_IF_HIP(hipGetLastError());
+    if (nb > 1) {
+        hipLaunchKernelGGL(mse_finish_kernel, dim3(1), dim3(kThreads), 0, s, partial, nb, n, loss);
+        RKA_RETURN_IF_HIP(hipGetLastError());
+    }
     return 0;
 }
 
@@ -306,9 +467,12 @@ int rka_head_forward(const float* out, const float* w, const float* b, float* pr
                      void* stream) {
     if (rows < 1 || hidden < 1 || !out || !w || !b || !pred)
         return fail(RKA_ERR_INVALID_ARGUMENT, "head_forward: bad arguments");
-    const int per_block = kThreads / 64;
-    hipLaunchKernelGGL(head_forward_kernel, dim3((rows + per_block - 1) / per_block), dim3(kThreads), 0,
-                       reinterpret_cast<hipStream_t>(stream), out, w, b, rows, hidden, pred);
+    with_head_form(hidden, head_vec(hidden, out, w, out), [&](auto team, auto vec) {
+        constexpr int kRows = kThreads / decltype(team)::value * kHeadUnroll;
+        hipLaunchKernelGGL((head_forward_kernel<decltype(team)::value, decltype(vec)::value>),
+                           dim3((unsigned)((rows - 1) / kRows + 1)), dim3(kThreads), 0,
+                           reinterpret_cast<hipStream_t>(stream), out, w, b, rows, hidden, pred);
+    });
     RKA_RETURN_IF_HIP(hipGetLastError());
     return 0;
 }
@@ -316,7 +480,7 @@ int rka_head_forward(const float* out, const float* w, const float* b, float* pr
 size_t rka_head_backward_workspace_bytes(int rows, int hidden) {
     if (rows < 1 || hidden < 1) return 0;
     int rpb = 0;
-    const int nb = head_blocks(rows, &rpb);
+    const int nb = head_blocks(rows, hidden, &rpb);
     return (size_t)nb * (hidden + 1) * sizeof(float);
 }
 
@@ -325,17 +489,23 @@ int rka_head_backward(const float* out, const float* w, const float* dpred, floa
     if (rows < 1 || hidden < 1 || !out || !w || !dpred || !dw || !db)
         return fail(RKA_ERR_INVALID_ARGUMENT, "head_backward: bad arguments");
     int rpb = 0;
-    const int nb = head_blocks(rows, &rpb);
+    const int nb = head_blocks(rows, hidden, &rpb);
     if (!workspace || workspace_bytes < (size_t)nb * (hidden + 1) * sizeof(float))
         return fail(RKA_ERR_WORKSPACE_TOO_SMALL, "head_backward: workspace too small");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    float* partial = reinterpret_cast<float*>(workspace);
-    hipLaunchKernelGGL(head_backward_partial_kernel, dim3(nb), dim3(kThreads), 0, s, out, w, dpred, rows, hidden, rpb,
-                       dout, partial);
+    float* partial = nb > 1 ? reinterpret_cast<float*>(workspace) : nullptr;
+    with_head_form(hidden, head_vec(hidden, out, w, dout), [&](auto team, auto vec) {
+        constexpr int kTeam = decltype(team)::value;
+        const dim3 grid((unsigned)nb, (unsigned)std::min((hidden - 1) / (4 * kTeam) + 1, 65535));
+        hipLaunchKernelGGL((head_backward_partial_kernel<kTeam, decltype(vec)::value>), grid, dim3(kThreads), 0, s, out,
+                           w, dpred, rows, hidden, rpb, dout, partial, dw, db);
+    });
     RKA_RETURN_IF_HIP(hipGetLastError());
-    hipLaunchKernelGGL(head_backward_finish_kernel, dim3((hidden + 1 + kThreads - 1) / kThreads), dim3(kThreads), 0,
-                       s, partial, nb, hidden, dw, db);
-    RKA_RETURN_IF_HIP(hipGetLastError());
+    if (nb > 1) {
+        hipLaunchKernelGGL(head_backward_finish_kernel, dim3((unsigned)(hidden / kFinishCols + 1)), dim3(kThreads), 0, s,
+                           partial, nb, hidden, dw, db);
+        RKA_RETURN_IF_HIP(hipGetLastError());
+    }
     return 0;
 }
 
