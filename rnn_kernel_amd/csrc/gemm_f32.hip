@@ -28,6 +28,7 @@
 // reduction, so results are deterministic run to run; up to 8 columns past
 // their last 128-column panel are summed on the VALU instead of in a tile.
 #include <atomic>
+#include <type_traits>
 
 #include "rka_internal.h"
 
@@ -1006,6 +1007,9 @@ __global__ __launch_bounds__(NT) void gemm_direct_reduce_kernel(GemmArgs p, Redu
     gemm_tile<AK, BKM, false, false, false, kDirectBK, UA>(p, bx, by, 0, smem);
 }
 
+// ------------------------------------------------------- small products ---
+#include "gemm_small.h"
+
 // ------------------------------------------------- narrow last columns ---
 // A split-K product whose n is whole 128-column panels plus w <= kNarrowMax
 // columns (the weight gradients at odd hidden sizes: n = H = 129) runs its
@@ -1191,6 +1195,76 @@ int launch_gemm(GemmArgs args, int ksplit, bool av, bool bv, hipStream_t stream)
 
 std::atomic<int> g_gemm_tiles{RKA_GEMM_TILES_AUTO};
 
+// Tiles a direct product runs in.
+enum DirectTile { TILE_128, TILE_128x64, TILE_64, TILE_32 };
+using Tile128x64 = SmallTile<128, 64, 64, 32, 16>;
+using Tile64 = SmallTile<64, 64, 32, 32, 16>;
+using Tile32 = SmallTile<32, 32, 32, 32, 64>;
+
+// The tile with the least work on the busiest CU: tiles per CU, rounded up,
+// times the tile's area, times the measured cost of a unit of area (large
+// products that divide evenly: the 128x128 ring 1, 128x64 1.02, 64x64 1.07,
+// 32x32 1.30; the ring's register path for operands that are not 16-byte
+// aligned 1.45).  Rounding up is what decides: 8192 x 2304 (k = 768) is 4.5
+// 128x128 tiles per CU, 8192 x 128 a quarter.  Measured on MI355X (us, 128 /
+// 128x64 / 64 / 32): 32768 x 768, k = 256: 113 / 115 / 118 / 154; 8192 x 2304,
+// k = 768: 271 / 246 / 257 / 319; 8192 x 128, k = 768: 59 / 36 / 23 / 20;
+// 32768 x 129, k = 387 (not aligned): 77 / 53 / 55 / 73; 64 x 768, k = 256:
+// 22 / 13 / 9.0 / 4.3; 1 x 256, k = 768: 55 / 35 / 21 / 8.2.
+DirectTile direct_tile(const GemmArgs& g) {
+    if (g_gemm_tiles.load(std::memory_order_relaxed) != RKA_GEMM_TILES_AUTO || g.a.kmajor) return TILE_128;
+    auto cost = [&](int tm, int tn, double unit) {
+        const long long tiles = (long long)((g.m + tm - 1) / tm) * ((g.n + tn - 1) / tn);
+        return (double)((tiles + 255) / 256) * tm * tn * unit;
+    };
+    DirectTile best = TILE_128;
+    double least = cost(128, 128, g.a_vec && g.b_vec ? 1.0 : 1.45);
+    auto consider = [&](DirectTile t, double c) {
+        if (c < least) {
+            best = t;
+            least = c;
+        }
+    };
+    consider(TILE_128x64, cost(128, 64, 1.02));
+    consider(TILE_64, cost(64, 64, 1.07));
+    consider(TILE_32, cost(32, 32, 1.30));
+    return best;
+}
+
+template <int AK, int BKM, typename S, bool VEC>
+int launch_small_t(GemmArgs args, const ReduceJob* j0, const ReduceJob* j1, long reducers, hipStream_t stream) {
+    args.tiles_m = (args.m + S::TM - 1) / S::TM;
+    const long long tiles = (long long)args.tiles_m * ((args.n + S::TN - 1) / S::TN);
+    if (tiles + reducers > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
+    args.tiles = (int)tiles;
+    const dim3 grid((unsigned)(tiles + reducers));
+    if (j0)
+        hipLaunchKernelGGL((gemm_small_reduce_kernel<AK, BKM, S, VEC>), grid, dim3(NT), 0, stream, args, *j0, *j1);
+    else
+        hipLaunchKernelGGL((gemm_small_kernel<AK, BKM, S, VEC>), grid, dim3(NT), 0, stream, args);
+    RKA_RETURN_IF_HIP(hipGetLastError());
+    return 0;
+}
+
+// A direct product of a row-major A in `tile`s (not TILE_128), with the
+// reductions j0, j1 (both or neither) in `reducers` workgroups after them.
+int launch_small(DirectTile tile, const GemmArgs& args, const ReduceJob* j0, const ReduceJob* j1, long reducers,
+                 hipStream_t stream) {
+    auto with = [&](auto bk, auto shape) {
+        constexpr int B = decltype(bk)::value;
+        using S = decltype(shape);
+        if (args.a_vec && args.b_vec) return launch_small_t<0, B, S, true>(args, j0, j1, reducers, stream);
+        return launch_small_t<0, B, S, false>(args, j0, j1, reducers, stream);
+    };
+    auto run = [&](auto bk) {
+        if (tile == TILE_32) return with(bk, Tile32{});
+        if (tile == TILE_64) return with(bk, Tile64{});
+        return with(bk, Tile128x64{});
+    };
+    if (args.a.kmajor) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: small tiles take a row-major A");
+    return args.b.kmajor ? run(std::integral_constant<int, 1>{}) : run(std::integral_constant<int, 0>{});
+}
+
 }  // namespace
 
 int set_gemm_tiles(int mode) {
@@ -1221,6 +1295,12 @@ int gemm_direct(int m, int n, int k, const GemmOperand& a, const GemmOperand& b,
     args.c_seg = c_seg;
     args.zero = zero;
     args.zero_words = zero ? zero_words : 0;
+    if (!(a.seg.len || b.seg.len || c_seg.len || a.shift_T > 0 || b.shift_T > 0)) {
+        args.a_vec = vec_ok(a, m, k) ? 1 : 0;
+        args.b_vec = vec_ok(b, n, k) ? 1 : 0;
+        const DirectTile tile = direct_tile(args);
+        if (tile != TILE_128) return launch_small(tile, args, nullptr, nullptr, 0, stream);
+    }
     return launch_gemm<false>(args, 1, vec_ok(a, m, k), vec_ok(b, n, k), stream);
 }
 
@@ -1409,6 +1489,8 @@ int gemm_direct_reduce_pair(int m, int n, int k, const GemmOperand& a, const Gem
     if ((long long)args.tiles + reducers > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
     const dim3 grid((unsigned)(args.tiles + reducers));
     const ReduceJob j0 = reduce_job(p0), j1 = reduce_job(p1);
+    const DirectTile tile = direct_tile(args);
+    if (tile != TILE_128) return launch_small(tile, args, &j0, &j1, reducers, stream);
     if (!a.kmajor && !b.kmajor)
         launch_direct_reduce<0, 0>(args, j0, j1, grid, stream);
     else if (!a.kmajor)

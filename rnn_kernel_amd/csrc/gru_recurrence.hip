@@ -117,6 +117,10 @@ size_t slots_bytes(int dir, int batch, int hidden) {
 constexpr size_t kXccBytes = (size_t)rec::MAX_XCC_BLOCKS * sizeof(unsigned long long);
 }  // namespace
 
+size_t rec_forward_state_offset(int batch, int hidden) {
+    return slots_bytes(0, batch, hidden) - align_up((size_t)2 * batch * hidden * sizeof(unsigned long long), 256);
+}
+
 size_t rec_workspace_bytes(int dir, int batch, int hidden) { return slots_bytes(dir, batch, hidden) + kXccBytes + 256; }
 
 namespace {
@@ -232,7 +236,9 @@ int launch(int dir, rec::Args& a, void* ws, size_t ws_bytes, bool zero_ws, hipSt
         return fail(RKA_ERR_WORKSPACE_TOO_SMALL, "recurrence workspace too small: need " + std::to_string(need) +
                                                      " bytes, got " + std::to_string(ws_bytes));
     char* base = reinterpret_cast<char*>(ws);
-    const RecState st{reinterpret_cast<unsigned long long*>(base),
+    // the forward's words end where the start-up XCD words begin, so that its
+    // state is one range of the workspace
+    const RecState st{reinterpret_cast<unsigned long long*>(dir == 0 ? base + rec_forward_state_offset(a.B, a.H) : base),
                       reinterpret_cast<unsigned long long*>(base + slots_bytes(dir, a.B, a.H)),
                       reinterpret_cast<int*>(base + need - 256)};
     return launch_at(dir, a, st, zero_ws, stream);

@@ -201,8 +201,9 @@ int rka_gru_forward(const float* x, const float* h0, const float* w_ih, const fl
     GemmOperand b{w_ih, I, 0, 0, nullptr};
     // the GEMM also clears the recurrence's exchange state (slots, start-up
     // XCD words, abort flag), which saves the recurrence its fill launch
-    unsigned long long* rec_state = reinterpret_cast<unsigned long long*>(ws + l.rec);
-    const size_t rec_words = rec_workspace_bytes(0, B, H) / sizeof(unsigned long long);
+    const size_t rec_off = rec_forward_state_offset(B, H);
+    unsigned long long* rec_state = reinterpret_cast<unsigned long long*>(ws + l.rec + rec_off);
+    const size_t rec_words = (rec_workspace_bytes(0, B, H) - rec_off) / sizeof(unsigned long long);
     {
         StageScope scope(0, s);
         RKA_RETURN_IF_ERR(gemm_direct(B * T, 3 * H, I, a, b, b_ih, gx, 3 * H, s, SegMap{}, rec_state, rec_words));

@@ -167,6 +167,9 @@ void set_rec_agent_stores(bool on);
 int rec_abort_count(unsigned long long* count);
 
 size_t rec_workspace_bytes(int dir, int batch, int hidden);
+// Where the state that a forward launch reads before it writes it (exchange
+// words, start-up XCD words, abort flag) begins; it ends with the workspace.
+size_t rec_forward_state_offset(int batch, int hidden);
 int eval_gate_functions(const float* x, float* sig, float* th, int n, hipStream_t stream);
 
 // zero_ws false: the workspace's recurrence state was cleared by an earlier
