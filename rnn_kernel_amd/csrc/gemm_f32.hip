@@ -27,8 +27,11 @@
 // The weight gradients (K = B*T rows) use split-K with a fixed-order
 // reduction, so results are deterministic run to run; up to 8 columns past
 // their last 128-column panel are summed on the VALU instead of in a tile.
+#include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <type_traits>
+#include <utility>
 
 #include "rka_internal.h"
 
@@ -303,6 +306,8 @@ struct GemmArgs {
     SegMap c_seg;          // direct mode: output row map
     unsigned long long* zero;  // direct mode: words cleared on the side (nullable)
     size_t zero_words;
+    int rot;               // split mode with c set (one slice): row rotation of c and colsum
+    float* colsum;
     int narrow;            // last columns left to gemm_narrow_kernel (0: none)
 };
 
@@ -921,6 +926,7 @@ struct ReduceJob {
     size_t items, total;  // row items (float4 or float), then m column sums
 };
 
+template <int TEAM>
 __device__ __forceinline__ void reduce_item(const ReduceJob& j, size_t idx, int member) {
     const int m = j.m, n = j.n, ksplit = j.ksplit;
     if (idx < j.items) {
@@ -931,7 +937,7 @@ __device__ __forceinline__ void reduce_item(const ReduceJob& j, size_t idx, int 
             const int col = 4 * (int)(idx % per_row);
             const float* pp = j.partial + (size_t)src * n + col;
             float4 s4 = make_float4(0.f, 0.f, 0.f, 0.f);
-            for (int z = member; z < ksplit; z += kTeam) {
+            for (int z = member; z < ksplit; z += TEAM) {
                 const float4 v = *reinterpret_cast<const float4*>(pp + (size_t)z * m * n);
                 s4.x += v.x;
                 s4.y += v.y;
@@ -939,19 +945,19 @@ __device__ __forceinline__ void reduce_item(const ReduceJob& j, size_t idx, int 
                 s4.w += v.w;
             }
 #pragma unroll
-            for (int off = 1; off < kTeam; off <<= 1) {
-                s4.x += __shfl_xor(s4.x, off, kTeam);
-                s4.y += __shfl_xor(s4.y, off, kTeam);
-                s4.z += __shfl_xor(s4.z, off, kTeam);
-                s4.w += __shfl_xor(s4.w, off, kTeam);
+            for (int off = 1; off < TEAM; off <<= 1) {
+                s4.x += __shfl_xor(s4.x, off, TEAM);
+                s4.y += __shfl_xor(s4.y, off, TEAM);
+                s4.z += __shfl_xor(s4.z, off, TEAM);
+                s4.w += __shfl_xor(s4.w, off, TEAM);
             }
             if (member == 0) *reinterpret_cast<float4*>(j.c + (size_t)o * j.ldc + col) = s4;
         } else {
             const int col = (int)(idx % per_row);
             float sum = 0.f;
-            for (int z = member; z < ksplit; z += kTeam) sum += j.partial[((size_t)z * m + src) * n + col];
+            for (int z = member; z < ksplit; z += TEAM) sum += j.partial[((size_t)z * m + src) * n + col];
 #pragma unroll
-            for (int off = 1; off < kTeam; off <<= 1) sum += __shfl_xor(sum, off, kTeam);
+            for (int off = 1; off < TEAM; off <<= 1) sum += __shfl_xor(sum, off, TEAM);
             if (member == 0) j.c[(size_t)o * j.ldc + col] = sum;
         }
     } else {
@@ -959,9 +965,9 @@ __device__ __forceinline__ void reduce_item(const ReduceJob& j, size_t idx, int 
         const int src = j.rot ? (o + j.rot) % m : o;
         const float* cpart = j.partial + (size_t)ksplit * m * n;
         float sum = 0.f;
-        for (int z = member; z < ksplit; z += kTeam) sum += cpart[(size_t)z * m + src];
+        for (int z = member; z < ksplit; z += TEAM) sum += cpart[(size_t)z * m + src];
 #pragma unroll
-        for (int off = 1; off < kTeam; off <<= 1) sum += __shfl_xor(sum, off, kTeam);
+        for (int off = 1; off < TEAM; off <<= 1) sum += __shfl_xor(sum, off, TEAM);
         if (member == 0) j.colsum[o] = sum;
     }
 }
@@ -969,19 +975,30 @@ __device__ __forceinline__ void reduce_item(const ReduceJob& j, size_t idx, int 
 // The reductions of one or two split-K products by `blocks` workgroups of
 // 256 threads (this one is number `block`): team items [0, j0.total) belong
 // to the first, the rest to the second (j1.total = 0 for one product).  A
-// team's idx is uniform over its kTeam lanes, so the shuffles stay within
-// one job.
-__device__ __forceinline__ void reduce_range(const ReduceJob& j0, const ReduceJob& j1, int block, int blocks) {
-    constexpr int kTeamsPerBlock = 256 / kTeam;
-    const int member = threadIdx.x % kTeam;
+// team's idx is uniform over its lanes, so the shuffles stay within one job.
+template <int TEAM>
+__device__ __forceinline__ void reduce_range_t(const ReduceJob& j0, const ReduceJob& j1, int block, int blocks) {
+    constexpr int kTeamsPerBlock = 256 / TEAM;
+    const int member = threadIdx.x % TEAM;
     const size_t teams = (size_t)blocks * kTeamsPerBlock;
     const size_t total = j0.total + j1.total;
-    for (size_t idx = (size_t)block * kTeamsPerBlock + threadIdx.x / kTeam; idx < total; idx += teams) {
+    for (size_t idx = (size_t)block * kTeamsPerBlock + threadIdx.x / TEAM; idx < total; idx += teams) {
         if (idx < j0.total)
-            reduce_item(j0, idx, member);
+            reduce_item<TEAM>(j0, idx, member);
         else
-            reduce_item(j1, idx - j0.total, member);
+            reduce_item<TEAM>(j1, idx - j0.total, member);
     }
+}
+
+// Teams of eight lanes, or as many as there are slices where those are fewer.
+__device__ __forceinline__ void reduce_range(const ReduceJob& j0, const ReduceJob& j1, int block, int blocks) {
+    const int ks = max(j0.ksplit, j1.ksplit);
+    if (ks > 4)
+        reduce_range_t<kTeam>(j0, j1, block, blocks);
+    else if (ks > 1)
+        reduce_range_t<4>(j0, j1, block, blocks);
+    else
+        reduce_range_t<1>(j0, j1, block, blocks);
 }
 
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(ReduceJob j0, ReduceJob j1) {
@@ -999,7 +1016,8 @@ __global__ __launch_bounds__(NT) void gemm_direct_reduce_kernel(GemmArgs p, Redu
     static_assert(NT == 256, "reduction teams assume 256-thread workgroups");
     __shared__ __attribute__((aligned(16))) float smem[gemm_smem_floats<AK, kDirectBK>()];
     if ((int)blockIdx.x >= p.tiles) {
-        reduce_range(j0, j1, (int)blockIdx.x - p.tiles, (int)gridDim.x - p.tiles);
+        // (large products: many slices)
+        reduce_range_t<kTeam>(j0, j1, (int)blockIdx.x - p.tiles, (int)gridDim.x - p.tiles);
         return;
     }
     int bx, by;
@@ -1308,6 +1326,139 @@ size_t splitk_partial_floats(int m, int n, int ksplit) {
     return (size_t)ksplit * m * n + (size_t)ksplit * m;
 }
 
+namespace {
+// Slices of one of the pair's products in 128x128 tiles, or in the 192x256
+// tiles where those divide evenly: each product is sized for half the CUs at
+// three resident workgroups per CU.
+int ring_ksplit(int m, int n, int k) { return choose_ksplit(m, n, k, 128, 3); }
+
+// Whether the pair's items in 192x256 tiles divide evenly over the CUs.
+bool big_pair_divides(int m, int n0, int n1, int k, int num_cus) {
+    using T = BigTile<3, 4>;
+    long long items = 0;
+    for (int n : {n0, n1}) {
+        const int ks = ring_ksplit(m, n, k);
+        if (m % T::BM != 0 || n % T::BN != 0 || k % (ks * kSplitBK) != 0) return false;
+        items += (long long)(m / T::BM) * (n / T::BN) * ks;
+    }
+    return num_cus > 0 && items % num_cus == 0;
+}
+
+struct PairPlan {
+    DirectTile tile;  // TILE_64, TILE_128x64 or TILE_128 (the ring)
+    int ks0, ks1;
+};
+
+// Tile and slices of the weight-gradient pair (m = 3H gate rows, n0 and n1
+// columns, k = B T) outside the 192x256 tiles.  Both products take the same
+// slices, so that every workgroup has the same work; the candidates are
+// multiples of 8 (a slice's tiles then share an XCD, split_coords) and fewer
+// than 8, each slice at least four 16-deep stages and at most 2048 values long
+// (the length of a chain of float32 additions).  Taken is the least of
+//   workgroups per CU x (stages + 2) x (time of a stage at that many)
+//   + the partial sums, written and read again,
+// where up to four workgroups share a CU and a part of one counts whole.  A
+// stage of a 64x64 tile was measured at 0.75, 0.5, 0.38 and 0.35 us for one,
+// two, three and four or more workgroups per CU (its MFMAs alone take 0.21); a
+// 128x64 tile takes 1.85 times that and the 128x128 ring, a candidate where
+// every extent divides by 128, 3.24 times.  Measured on MI355X (pair, us; 128x128
+// ring, now): m = 576, n = 192 + 192, k = 32768: 218, 158; 192, 64 + 64, 32768:
+// 50, 25; 384, 128 + 128, 32768: 84, 75; 387, 129 + 129, 32768: 163, 151; 384, 128 +
+// 64, 51200: 120, 86; 768, 256 + 128, 8192: 61, 58.
+PairPlan make_pair_plan(int m, int n0, int n1, int k) {
+    PairPlan best{TILE_128x64, ring_ksplit(m, n0, k), ring_ksplit(m, n1, k)};
+    if (big_pair_divides(m, n0, n1, k, 256)) return best;  // the same slices if its operands are not aligned
+    constexpr int kMaxSlices = 256;
+    constexpr double kStage[4] = {0.75, 0.5, 0.38, 0.35};
+    const int most = std::min(kMaxSlices, std::max(1, k / (4 * kSplitBK)));
+    const int least = std::min(most, (k + 2047) / 2048);
+    double least_cost = 1e30;
+    for (const DirectTile tile : {TILE_64, TILE_128x64, TILE_128}) {
+        if (tile == TILE_128 && (m % 128 || n0 % 128 || n1 % 128)) continue;
+        const int tm = tile == TILE_64 ? 64 : 128, tn = tile == TILE_128 ? 128 : 64;
+        const double unit = tile == TILE_64 ? 1.0 : tile == TILE_128x64 ? 1.85 : 3.24;
+        const double tiles = (double)((m + tm - 1) / tm) * ((n0 + tn - 1) / tn + (n1 + tn - 1) / tn);
+        for (int ks = 1; ks <= most; ks += ks < 8 ? 1 : 8) {
+            if (ks < least && ks + 8 <= most) continue;
+            const double per_cu = tiles * ks / 256;
+            const double rounds = per_cu <= 4 ? std::ceil(per_cu) : per_cu + 0.5;
+            const int stages = ((k + ks - 1) / ks + kSplitBK - 1) / kSplitBK;
+            const double stage = kStage[std::min((int)rounds, 4) - 1] * unit;
+            const double sums = ks == 1 ? 0.0 : 0.5e-6 * 4.0 * ks * m * ((double)n0 + n1);  // ~4 TB/s each way
+            const double cost = rounds * (stages + 2) * stage + sums;
+            if (cost < least_cost) {
+                least_cost = cost;
+                best = PairPlan{tile, ks, ks};
+            }
+        }
+    }
+    return best;
+}
+
+// The plan of the thread's last shape is kept (a call asks for it three times).
+PairPlan plan_pair(int m, int n0, int n1, int k) {
+    thread_local int key[4] = {0, 0, 0, 0};
+    thread_local PairPlan plan{};
+    if (key[0] != m || key[1] != n0 || key[2] != n1 || key[3] != k) {
+        plan = make_pair_plan(m, n0, n1, k);
+        key[0] = m;
+        key[1] = n0;
+        key[2] = n1;
+        key[3] = k;
+    }
+    return plan;
+}
+
+// Whether the pair's launch writes the results itself (one slice each, outside
+// the 128x128 ring), so that there is nothing to reduce.
+bool pair_is_direct(const SplitProduct& p0, const SplitProduct& p1) {
+    return p0.ksplit == 1 && p1.ksplit == 1 && p0.b.shift_T > 0 && p0.colsum && p1.colsum &&
+           g_gemm_tiles.load(std::memory_order_relaxed) == RKA_GEMM_TILES_AUTO;
+}
+
+template <typename S>
+int launch_small_pair(const SplitProduct& p0, const SplitProduct& p1, GemmArgs a0, GemmArgs a1, hipStream_t stream) {
+    long long items = 0;
+    for (GemmArgs* g : {&a0, &a1}) {
+        g->narrow = 0;
+        g->tiles_m = (g->m + S::TM - 1) / S::TM;
+        g->tiles = g->tiles_m * ((g->n + S::TN - 1) / S::TN);
+        items += (long long)g->tiles * g->ksplit;
+    }
+    if (items > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
+    const dim3 grid((unsigned)items);
+    if (pair_is_direct(p0, p1)) {
+        for (const auto& pa : {std::make_pair(&p0, &a0), std::make_pair(&p1, &a1)}) {
+            pa.second->c = pa.first->c;
+            pa.second->ldc = pa.first->ldc;
+            pa.second->rot = pa.first->rot;
+            pa.second->colsum = pa.first->colsum;
+            pa.second->c_vec = pa.first->ldc % 4 == 0 && aligned16(pa.first->c) ? 1 : 0;
+        }
+    }
+    if (a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec)
+        hipLaunchKernelGGL((gemm_small_pair_kernel<S, true, true>), grid, dim3(NT), 0, stream, a0, a1);
+    else
+        hipLaunchKernelGGL((gemm_small_pair_kernel<S, true, false>), grid, dim3(NT), 0, stream, a0, a1);
+    RKA_RETURN_IF_HIP(hipGetLastError());
+    return 0;
+}
+}  // namespace
+
+void choose_pair_ksplit(int m, int n0, int n1, int k, int* ks0, int* ks1) {
+    PairPlan p = plan_pair(m, n0, n1, k);
+    if (g_gemm_tiles.load(std::memory_order_relaxed) != RKA_GEMM_TILES_AUTO)
+        p = PairPlan{TILE_128, ring_ksplit(m, n0, k), ring_ksplit(m, n1, k)};
+    *ks0 = p.ks0;
+    *ks1 = p.ks1;
+}
+
+void pair_ksplit_bound(int m, int n0, int n1, int k, int* ks0, int* ks1) {
+    const PairPlan p = plan_pair(m, n0, n1, k);
+    *ks0 = std::max(p.ks0, ring_ksplit(m, n0, k));
+    *ks1 = std::max(p.ks1, ring_ksplit(m, n1, k));
+}
+
 int choose_ksplit(int m, int n, int k, int num_cus, int wgs_per_cu) {
     const int tiles = ((m + BM - 1) / BM) * ((n - narrow_cols(n) + BN - 1) / BN);
     const int target = wgs_per_cu > 0 ? wgs_per_cu * (num_cus > 0 ? num_cus : 256) : (num_cus > 0 ? num_cus : 256) / 2;
@@ -1391,9 +1542,16 @@ int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, hi
     if (p1.b.shift_T > 0) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: only the first product of a pair is remapped");
     const bool seg = a0.a.seg.len || a0.b.seg.len || a1.a.seg.len || a1.b.seg.len;
     if (seg) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: pair products take whole operands");
+    const bool ring = g_gemm_tiles.load(std::memory_order_relaxed) != RKA_GEMM_TILES_AUTO || p0.b.shift_T == 0;
     bool launched = false;
     RKA_RETURN_IF_ERR(try_big_pair(a0, a1, p0.b.shift_T > 0, stream, &launched));
     if (launched) return 0;
+    if (!ring) {
+        const PairPlan plan = plan_pair(p0.m, p0.n, p1.n, p0.k);
+        if (plan.tile == TILE_64) return launch_small_pair<Tile64>(p0, p1, a0, a1, stream);
+        if (plan.tile == TILE_128x64 || !(a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec) || pair_is_direct(p0, p1))
+            return launch_small_pair<Tile128x64>(p0, p1, a0, a1, stream);
+    }
     const dim3 grid(a0.tiles * a0.ksplit + a1.tiles * a1.ksplit);
     const bool ua = !(a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec);
     if (p0.b.shift_T > 0) {
@@ -1447,6 +1605,7 @@ int splitk_reduce(const SplitProduct& p, hipStream_t stream) {
 }
 
 int splitk_reduce_pair(const SplitProduct& p0, const SplitProduct& p1, hipStream_t stream) {
+    if (pair_is_direct(p0, p1)) return 0;
     return launch_reduce(reduce_job(p0), reduce_job(p1), stream);
 }
 
@@ -1485,12 +1644,18 @@ int gemm_direct_reduce_pair(int m, int n, int k, const GemmOperand& a, const Gem
     finish_args<false>(args, 1, vec_ok(a, m, k), vec_ok(b, n, k));
     // one reducing workgroup per CU: with the product's tiles at up to two
     // per CU they run beside them, in the third workgroup slot
-    const long reducers = dev->num_cus > 0 ? dev->num_cus : 256;
+    const long reducers = pair_is_direct(p0, p1) ? 0 : dev->num_cus > 0 ? dev->num_cus : 256;
     if ((long long)args.tiles + reducers > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
     const dim3 grid((unsigned)(args.tiles + reducers));
     const ReduceJob j0 = reduce_job(p0), j1 = reduce_job(p1);
     const DirectTile tile = direct_tile(args);
-    if (tile != TILE_128) return launch_small(tile, args, &j0, &j1, reducers, stream);
+    if (tile != TILE_128) {
+        if (reducers == 0) return launch_small(tile, args, nullptr, nullptr, 0, stream);
+        // smaller workgroups than the ring's: up to four reducing ones per CU
+        const size_t want = ((j0.total + j1.total) * kTeam + NT - 1) / NT;
+        const long most = 4 * reducers;
+        return launch_small(tile, args, &j0, &j1, (long)std::min<size_t>(want, most), stream);
+    }
     if (!a.kmajor && !b.kmajor)
         launch_direct_reduce<0, 0>(args, j0, j1, grid, stream);
     else if (!a.kmajor)

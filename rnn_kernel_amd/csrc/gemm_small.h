@@ -55,7 +55,7 @@ struct SmallTile {
 template <int KMAJOR, int R, int BK, bool VEC, int NV>
 struct SmallLoader {
     static constexpr int NL = VEC ? NV : 4 * NV;
-    const char* base;      // operand at (r0, 0), wave-uniform
+    const char* base;      // operand at (r0, kbeg), wave-uniform
     size_t stage_bytes;    // bytes from one stage to the next
     unsigned kunit;        // bytes per k
     unsigned row[NL], kk[NL];
@@ -70,9 +70,10 @@ struct SmallLoader {
         return KMAJOR ? x / R : x % BK;
     }
 
-    __device__ __forceinline__ SmallLoader(const GemmOperand& op, int rows, int r0, int tid) {
+    __device__ __forceinline__ SmallLoader(const GemmOperand& op, int rows, int r0, int kbeg, int klen, int tid) {
+        (void)klen;
         const size_t ld = (size_t)op.ld;
-        base = reinterpret_cast<const char*>(op.ptr + (KMAJOR ? (size_t)r0 : (size_t)r0 * ld));
+        base = reinterpret_cast<const char*>(op.ptr + (KMAJOR ? (size_t)kbeg * ld + r0 : (size_t)r0 * ld + kbeg));
         kunit = KMAJOR ? 4u * (unsigned)op.ld : 4u;
         stage_bytes = (size_t)BK * (KMAJOR ? 4 * ld : 4);
         const int last = rows - r0 - (VEC && KMAJOR ? 4 : 1);  // last row (row group) of the tile
@@ -83,11 +84,11 @@ struct SmallLoader {
             kk[j] = (unsigned)k_of(x) * kunit;
         }
     }
-    // stage kb of nkb, or the last one again past it
-    __device__ __forceinline__ void load(int kb, int nkb, int kend, float4 (&v)[NV]) const {
+    // stage kb of the nkb that klen values make, or the last one again past it
+    __device__ __forceinline__ void load(int kb, int nkb, int klen, float4 (&v)[NV]) const {
         const int st = min(kb, nkb - 1);
         const char* p = base + (size_t)st * stage_bytes;
-        const unsigned lim = (unsigned)(kend - st * BK - (VEC && !KMAJOR ? 4 : 1)) * kunit;
+        const unsigned lim = (unsigned)(klen - st * BK - (VEC && !KMAJOR ? 4 : 1)) * kunit;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             if constexpr (VEC) {
@@ -99,6 +100,69 @@ struct SmallLoader {
                     e[c] = *reinterpret_cast<const float*>(p + (row[4 * j + c] + min(kk[4 * j + c], lim)));
                 v[j] = make_float4(e[0], e[1], e[2], e[3]);
             }
+        }
+    }
+};
+
+// The same for the k-major [h0 ; y[:, :-1]] operand (GemmOperand::shift_T): k =
+// b T + t reads row k - 1 of ptr, or row b of shift_first where t = 0.  Stages
+// are loaded in order, so each element carries its t and b and one stage on is
+// an addition (a division only where a sequence ends).
+template <int R, int BK, bool VEC, int NV>
+struct ShiftLoader {
+    using Plain = SmallLoader<1, R, BK, VEC, NV>;
+    static constexpr int NL = Plain::NL;
+    const float* ptr;
+    const float* first;
+    size_t ld;
+    int T, left;           // left: k values from this stage's start to the end of the range
+    int row[NL], t[NL], b[NL], k[NL];
+
+    __device__ __forceinline__ ShiftLoader(const GemmOperand& op, int rows, int r0, int kbeg, int klen, int tid)
+        : ptr(op.ptr), first(op.shift_first), ld((size_t)op.ld), T(op.shift_T), left(klen) {
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            const int x = tid + NT * j;
+            row[j] = min(r0 + Plain::row_of(x), rows - (VEC ? 4 : 1));
+            k[j] = kbeg + Plain::k_of(x);
+            b[j] = k[j] / T;
+            t[j] = k[j] - b[j] * T;
+        }
+    }
+    // the next stage; elements past the range read row 0 of shift_first
+    __device__ __forceinline__ void load(int, int, int, float4 (&v)[NV]) {
+        float e[NL][VEC ? 4 : 1];
+#pragma unroll
+        for (int j = 0; j < NL; ++j) {
+            const bool in = Plain::k_of((int)threadIdx.x + NT * j) < left;
+            const bool start = !in || t[j] == 0;
+            const float* src = start ? first : ptr;
+            const size_t line = !in ? 0 : start ? (size_t)b[j] : (size_t)(k[j] - 1);
+            src += line * ld + row[j];
+            if constexpr (VEC) {
+                const float4 u = *reinterpret_cast<const float4*>(src);
+                e[j][0] = u.x;
+                e[j][1] = u.y;
+                e[j][2] = u.z;
+                e[j][3] = u.w;
+            } else {
+                e[j][0] = *src;
+            }
+            k[j] += BK;
+            t[j] += BK;
+            if (t[j] >= T) {
+                const int q = t[j] / T;
+                b[j] += q;
+                t[j] -= q * T;
+            }
+        }
+        left -= BK;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            if constexpr (VEC)
+                v[j] = make_float4(e[j][0], e[j][1], e[j][2], e[j][3]);
+            else
+                v[j] = make_float4(e[4 * j][0], e[4 * j + 1][0], e[4 * j + 2][0], e[4 * j + 3][0]);
         }
     }
 };
@@ -163,8 +227,11 @@ __device__ __forceinline__ void small_frag(const float* lds, int row0, int k, in
     }
 }
 
-template <int AK, int BKM, typename S, bool VEC>
-__device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, float* smem) {
+// One tile (bx, by); SPLIT: the partial products of k slice bz, with the column
+// sums of A (the bias gradients) in the first column of tiles.
+template <int AK, int BKM, typename S, bool VEC, bool SPLIT = false, bool BSHIFT = false>
+__device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, int bz, float* smem) {
+    static_assert(!SPLIT || (AK == 1 && BKM == 1 && S::WK == 1), "split-K products take k-major operands");
     constexpr int TM = S::TM, TN = S::TN, BK = S::BK, MB = S::MB, NB = S::NB;
     constexpr int NVA = TM * BK / (4 * NT), NVB = TN * BK / (4 * NT);
     constexpr int AF = S::template floats<AK, TM>(), BF = S::template floats<BKM, TN>();
@@ -174,12 +241,16 @@ __device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, fl
     const int wk = wave % S::WK, wm = wave / S::WK % S::WM, wn = wave / (S::WK * S::WM);
     const int i = lane & 15, g = lane >> 4;
     const int m0 = bx * TM, n0 = by * TN;
-    const int nkb = (p.k + BK - 1) / BK;
+    const int kbeg = SPLIT ? bz * p.kchunk : 0;
+    const int klen = SPLIT ? max(0, min(p.k - kbeg, p.kchunk)) : p.k;
+    const int nkb = (klen + BK - 1) / BK;
+    const bool colsum = SPLIT && p.want_colsum && by == 0;
+    float cs = 0.f;
     // the columns a thread stores are the same in every row it stores
     static_assert(NT % (TN / 4) == 0, "a thread's columns");
     const int scol = 4 * (tid % (TN / 4)), sn = n0 + scol;
     float bias[4] = {0.f, 0.f, 0.f, 0.f};
-    if (p.bias) {
+    if (!SPLIT && p.bias) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) bias[q] = p.bias[min(sn + q, p.n - 1)];
     }
@@ -188,12 +259,14 @@ __device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, fl
     for (int x = 0; x < MB; ++x)
 #pragma unroll
         for (int y = 0; y < NB; ++y) acc[x][y] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const SmallLoader<AK, TM, BK, VEC, NVA> la(p.a, p.m, m0, tid);
-    const SmallLoader<BKM, TN, BK, VEC, NVB> lb(p.b, p.n, n0, tid);
+    const SmallLoader<AK, TM, BK, VEC, NVA> la(p.a, p.m, m0, kbeg, klen, tid);
+    using LoaderB =
+        std::conditional_t<BSHIFT, ShiftLoader<TN, BK, VEC, NVB>, SmallLoader<BKM, TN, BK, VEC, NVB>>;
+    LoaderB lb(p.b, p.n, n0, kbeg, klen, tid);
     float4 ra[2][NVA], rb[2][NVB];
     auto load = [&](int kb, int st) {
-        la.load(kb, nkb, p.k, ra[st]);
-        lb.load(kb, nkb, p.k, rb[st]);
+        la.load(kb, nkb, klen, ra[st]);
+        lb.load(kb, nkb, klen, rb[st]);
     };
     // stage kb: registers to LDS, the loads of stage kb + 2 into the same
     // registers, one barrier (the other LDS buffer's readers are past it), MFMAs
@@ -201,10 +274,16 @@ __device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, fl
         constexpr int ST = decltype(st)::value;
         float* as = smem + ST * (AF + BF);
         float* bs = as + AF;
-        small_store<AK, TM, BK, VEC>(as, p.k, kb * BK, tid, ra[ST]);
-        small_store<BKM, TN, BK, VEC>(bs, p.k, kb * BK, tid, rb[ST]);
+        small_store<AK, TM, BK, VEC>(as, klen, kb * BK, tid, ra[ST]);
+        small_store<BKM, TN, BK, VEC>(bs, klen, kb * BK, tid, rb[ST]);
         load(kb + 2, ST);
         __syncthreads();
+        if constexpr (SPLIT) {
+            if (colsum && tid < TM) {
+#pragma unroll
+                for (int kk = 0; kk < BK; ++kk) cs += as[kk * LDA + tid];
+            }
+        }
 #pragma unroll
         for (int q = 0; q < S::NG; ++q) {
             const int k = 16 * (S::NG * wk + q);
@@ -263,13 +342,29 @@ __device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, fl
         }
         const float c[4] = {v.x + bias[0], v.y + bias[1], v.z + bias[2], v.w + bias[3]};
         if (m >= p.m || sn >= p.n) continue;
-        float* dst = p.c + (size_t)m * p.ldc + sn;
+        float* dst;
+        if constexpr (SPLIT) {
+            // one slice: the sums are the result, its rows rotated (out[o] = C[(o + rot) % m])
+            dst = p.c ? p.c + (size_t)(m >= p.rot ? m - p.rot : m - p.rot + p.m) * p.ldc + sn
+                      : p.partial + ((size_t)(p.z_off + bz) * p.m + m) * p.n + sn;
+        } else {
+            dst = p.c + (size_t)m * p.ldc + sn;
+        }
         if (p.c_vec && sn + 3 < p.n) {
             *reinterpret_cast<float4*>(dst) = make_float4(c[0], c[1], c[2], c[3]);
         } else {
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 if (sn + q < p.n) dst[q] = c[q];
+        }
+    }
+    if constexpr (SPLIT) {
+        if (colsum && tid < TM && m0 + tid < p.m) {
+            const int m = m0 + tid;
+            if (p.c)
+                p.colsum[m >= p.rot ? m - p.rot : m - p.rot + p.m] = cs;
+            else
+                (p.partial + (size_t)p.ksplit_total * p.m * p.n)[(size_t)(p.z_off + bz) * p.m + m] = cs;
         }
     }
 }
@@ -280,7 +375,7 @@ __global__ __launch_bounds__(NT) void gemm_small_kernel(GemmArgs p) {
     for (size_t i = (size_t)blockIdx.x * NT + threadIdx.x; i < p.zero_words; i += (size_t)gridDim.x * NT) p.zero[i] = 0ull;
     int bx, by;
     direct_coords(p, blockIdx.x, bx, by);
-    small_tile<AK, BKM, S, VEC>(p, bx, by, smem);
+    small_tile<AK, BKM, S, VEC>(p, bx, by, 0, smem);
 }
 
 // The same with the reductions of one or two split-K products in the
@@ -294,5 +389,20 @@ __global__ __launch_bounds__(NT) void gemm_small_reduce_kernel(GemmArgs p, Reduc
     }
     int bx, by;
     direct_coords(p, blockIdx.x, bx, by);
-    small_tile<AK, BKM, S, VEC>(p, bx, by, smem);
+    small_tile<AK, BKM, S, VEC>(p, bx, by, 0, smem);
+}
+
+// The two split-K weight-gradient products in one launch (gemm_f32_pair_kernel).
+template <typename S, bool SHIFT0, bool VEC>
+__global__ __launch_bounds__(NT, S::TM == 64 ? 4 : 2) void gemm_small_pair_kernel(GemmArgs p0, GemmArgs p1) {
+    __shared__ __attribute__((aligned(16))) float smem[S::template smem<1, 1>()];
+    const int blocks0 = p0.tiles * p0.ksplit;
+    int bx, by, bz;
+    if ((int)blockIdx.x < blocks0) {
+        split_coords(p0, blockIdx.x, bx, by, bz);
+        small_tile<1, 1, S, VEC, true, SHIFT0>(p0, bx, by, bz, smem);
+    } else {
+        split_coords(p1, blockIdx.x - blocks0, bx, by, bz);
+        small_tile<1, 1, S, VEC, true, false>(p1, bx, by, bz, smem);
+    }
 }

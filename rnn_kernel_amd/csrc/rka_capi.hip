@@ -78,15 +78,14 @@ struct BwdLayout {
 BwdLayout bwd_layout(int B, int T, int I, int H) {
     BwdLayout l{};
     const int K = B * T;
-    // the two products share one launch (gemm_splitk_pair), so each is sized
-    // for half the CUs at three resident workgroups per CU
-    l.ks_hh = choose_ksplit(3 * H, H, K, 128, 3);
-    l.ks_ih = choose_ksplit(3 * H, I, K, 128, 3);
+    choose_pair_ksplit(3 * H, H, I, K, &l.ks_hh, &l.ks_ih);
+    int most_hh = 0, most_ih = 0;
+    pair_ksplit_bound(3 * H, H, I, K, &most_hh, &most_ih);
     l.g = 0;
     l.rec = align_up((size_t)B * T * 4 * H * sizeof(float), 256);
     l.part_hh = l.rec + align_up(rec_workspace_bytes(1, B, H), 256);
-    l.part_ih = l.part_hh + align_up(splitk_partial_floats(3 * H, H, l.ks_hh) * sizeof(float), 256);
-    l.total = l.part_ih + align_up(splitk_partial_floats(3 * H, I, l.ks_ih) * sizeof(float), 256);
+    l.part_ih = l.part_hh + align_up(splitk_partial_floats(3 * H, H, most_hh) * sizeof(float), 256);
+    l.total = l.part_ih + align_up(splitk_partial_floats(3 * H, I, most_ih) * sizeof(float), 256);
     return l;
 }
 

@@ -120,6 +120,11 @@ int set_gemm_tiles(int mode);
 // (0: half a workgroup per CU, for products that share the GPU with a
 // concurrently running recurrence); a multiple of 8 from 8 up.
 int choose_ksplit(int m, int n, int k, int num_cus, int wgs_per_cu);
+// Slices of the weight-gradient pair's products (m rows, n0 and n1 columns) at
+// the current tile choice, and the most over every choice (rka_set_gemm_tiles),
+// which sizes the workspace.
+void choose_pair_ksplit(int m, int n0, int n1, int k, int* ks0, int* ks1);
+void pair_ksplit_bound(int m, int n0, int n1, int k, int* ks0, int* ks1);
 
 // ----------------------------------------------------------- recurrence ---
 enum RecKind { REC_AUTO = 0, REC_TILED = 1, REC_REGISTER = 2 };

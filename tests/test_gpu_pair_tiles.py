@@ -1,0 +1,65 @@
+"""The weight-gradient products where their tile or number of slices changes,
+against float64 sums of the gate gradients that the library itself returns:
+one slice (the results written by the products' own launch), few, and a
+multiple of 8; sequences shorter than a 16-deep stage and of one step (the
+[h0 ; y[:, :-1]] rows); a last slice shorter than the others; aligned and
+unaligned rows; 64x64 and 128x64 tiles and the ring."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 1, 1), (2, 3, 5, 7), (127, 1, 16, 20), (128, 1, 12, 64), (9, 14, 33, 65), (5, 100, 100, 100),
+          (40, 25, 64, 128), (7, 300, 129, 129), (16, 520, 128, 256), (33, 331, 16, 64), (16, 2000, 256, 256)]
+
+
+@pytest.mark.parametrize("B,T,I,H", SHAPES)
+@pytest.mark.parametrize("need_dx", [True, False])
+def test_weight_gradients_match_float64(gpu, hip_lib, B, T, I, H, need_dx):
+    from rnn_kernel_amd import _lib
+
+    print(f"pair B={B} T={T} I={I} H={H} dx={need_dx}", flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(B + T + I + H)
+
+    def randn(*shape):
+        return torch.randn(*shape, generator=gen, device=gpu)
+
+    x, h0, y, dy, dhn = randn(B, T, I), randn(B, H), torch.tanh(randn(B, T, H)), randn(B, T, H), randn(B, H)
+    w_ih, w_hh = 0.1 * randn(3 * H, I), 0.1 / H ** 0.5 * randn(3 * H, H)
+    res = torch.sigmoid(randn(B, T, H, 4))
+    stream = torch.cuda.current_stream().cuda_stream
+    g, dh0 = torch.empty(B, T, 4, H, device=gpu), torch.empty(B, H, device=gpu)
+    nb = hip_lib.rka_gru_recurrence_workspace_bytes(B, H)
+    ws = torch.empty(nb, dtype=torch.uint8, device=gpu)
+    _lib.check(hip_lib.rka_gru_recurrence_backward(dy.data_ptr(), dhn.data_ptr(), res.data_ptr(), h0.data_ptr(),
+                                                   y.data_ptr(), w_hh.data_ptr(), g.data_ptr(), dh0.data_ptr(),
+                                                   ws.data_ptr(), nb, B, T, H, stream), "recurrence_backward")
+    nan = float("nan")
+    dx = torch.full((B, T, I), nan, device=gpu)
+    dw_ih, dw_hh = torch.full((3 * H, I), nan, device=gpu), torch.full((3 * H, H), nan, device=gpu)
+    db_ih, db_hh = torch.full((3 * H,), nan, device=gpu), torch.full((3 * H,), nan, device=gpu)
+    nb = hip_lib.rka_gru_backward_workspace_bytes(B, T, I, H)
+    ws = torch.empty(nb, dtype=torch.uint8, device=gpu)
+    _lib.check(hip_lib.rka_gru_backward(x.data_ptr(), h0.data_ptr(), w_ih.data_ptr(), w_hh.data_ptr(), y.data_ptr(),
+                                        res.data_ptr(), dy.data_ptr(), dhn.data_ptr(), dx.data_ptr() if need_dx else None,
+                                        dh0.data_ptr(), dw_ih.data_ptr(), dw_hh.data_ptr(), db_ih.data_ptr(),
+                                        db_hh.data_ptr(), ws.data_ptr(), nb, B, T, I, H, stream), "backward")
+    # G = (da_n, dr^, dz^, dn^) per step
+    G = g.double().view(B * T, 4 * H)
+    g_ih = G[:, H:]
+    g_hh = torch.cat([G[:, H:3 * H], G[:, :H]], dim=1)
+    hprev = torch.cat([h0[:, None], y[:, :-1]], dim=1).double().reshape(B * T, H)
+    # a float32 sum of n products, in chains of at most 2048 and their sum, is
+    # within (2048 + 256) 2^-24 of the sum of the products' magnitudes
+    n = min(B * T, 2304)
+    for name, out, a, b in (("dw_ih", dw_ih, g_ih, x.double().reshape(B * T, I)), ("dw_hh", dw_hh, g_hh, hprev),
+                            ("db_ih", db_ih, g_ih, None), ("db_hh", db_hh, g_hh, None)):
+        if b is None:
+            ref, mag = a.sum(0), a.abs().sum(0)
+        else:
+            ref, mag = a.t().contiguous() @ b, a.abs().t().contiguous() @ b.abs()
+        assert bool(((out.double() - ref).abs() <= n * 2.0 ** -24 * mag + 1e-30).all()), name
+    if need_dx:
+        ref = (g_ih @ w_ih.double()).view(B, T, I)
+        mag = (g_ih.abs() @ w_ih.double().abs()).view(B, T, I)
+        assert bool(((dx.double() - ref).abs() <= 3 * H * 2.0 ** -24 * mag + 1e-30).all())
