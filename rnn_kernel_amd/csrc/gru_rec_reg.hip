@@ -16,7 +16,7 @@ namespace {
 constexpr int fwd_waves1(int S) { return S == 4 ? 16 : 8; }
 
 template <int S>
-const void* local_ptr(int dir, int rows, bool io, bool full) {
+const void* local_ptr(int dir, int rows, bool io, bool full, bool stage) {
     if (dir == 1) {
         if (rows == 1) {
             // whole slices at three and four slices: the instances built with
@@ -38,13 +38,23 @@ const void* local_ptr(int dir, int rows, bool io, bool full) {
     switch (rows) {
         case 1:
             if (full) {
-                if constexpr (S == 4) return rec_fwd1_kernel();
-                return io ? reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, true, NW, true>)
-                          : reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, false, fwd_waves1(S), true>);
+                if constexpr (S == 4) {
+                    return rec_fwd1_kernel();
+                } else {
+                    return stage ? reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, true, NW, true, true>)
+                                 : reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, true, NW, true, false>);
+                }
             }
-            return io ? reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, true>)
-                      : reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, false, fwd_waves1(S)>);
-        case 2: return reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 2, false>);
+            if constexpr (S == 4) {
+                return stage ? reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, false, 16, false, true>)
+                             : reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, false, 16>);
+            } else {
+                return stage ? reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, true, NW, false, true>)
+                             : reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 1, true>);
+            }
+        case 2:
+            return stage ? reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 2, false, NW, false, true>)
+                       : reinterpret_cast<const void*>(&gru_fwd_local_kernel<S, 2, false>);
         default:
             return full ? reinterpret_cast<const void*>(&gru_fwd_mfma4_kernel<S, true>)
                         : reinterpret_cast<const void*>(&gru_fwd_mfma4_kernel<S>);
@@ -62,15 +72,16 @@ int block_threads(int dir, int rows, int slices) {
 }
 
 // The local-slice kernels: S slices, 1, 2 or 4 batch rows per workgroup.
-// full: H = 64 * slices (the one-row forward has instances for it).
-const void* kernel_ptr(int dir, int cap, int rows, int slices, bool full = false) {
+// full: H = 64 * slices (the one-row forward has instances for it); stage:
+// the forward reads W_hh through LDS.
+const void* kernel_ptr(int dir, int cap, int rows, int slices, bool full = false, bool stage = true) {
     (void)cap;
     const bool io = uses_io(dir, rows, slices);
     switch (slices) {
-        case 1: return local_ptr<1>(dir, rows, io, full);
-        case 2: return local_ptr<2>(dir, rows, io, full);
-        case 3: return local_ptr<3>(dir, rows, io, full);
-        default: return local_ptr<4>(dir, rows, io, full);
+        case 1: return local_ptr<1>(dir, rows, io, full, stage);
+        case 2: return local_ptr<2>(dir, rows, io, full, stage);
+        case 3: return local_ptr<3>(dir, rows, io, full, stage);
+        default: return local_ptr<4>(dir, rows, io, full, stage);
     }
 }
 
@@ -147,9 +158,15 @@ int reg_launch(int dir, const RecConfig& c, const rec::Args& a, hipStream_t stre
     // whole slices: the forward always takes the compile-time-H instances;
     // the one-row backward only on grids of 128 or more workgroups (c2: 434
     // -> 427 us per launch; at 64 workgroups, c5, 3.44 -> 3.54 ms per step)
-    bool full = a.H == 64 * c.slices;
+    bool full = a.H == 64 * c.slices && (dir == 1 || prm.wvec != 0);
     if (dir == 1 && c.rows == 1 && (long)c.groups * c.slices < 128) full = false;
-    const void* k = kernel_ptr(dir, cap, c.rows, c.slices, full);
+    // The forward reads W_hh through LDS where its rows are aligned float4: 7 to
+    // 15 us less per launch at two to four slices, 2 at one.  At one and three
+    // slices the step loop behind it came out 0.004 and 0.014 us slower per step
+    // (H = 64, 192: 0.446 vs 0.442, 0.718 vs 0.704), which outweighs that from
+    // some 700 steps on.
+    const bool stage = prm.wvec != 0 && (c.slices % 2 == 0 || c.rows != 1 || a.T <= 600);
+    const void* k = kernel_ptr(dir, cap, c.rows, c.slices, full, stage);
     if (k == nullptr) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "register recurrence: no kernel for this row count");
     const unsigned blocks = (unsigned)(grid_groups(c, c.groups) * c.slices);
     if (dir == 0) {

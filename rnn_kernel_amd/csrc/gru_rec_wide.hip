@@ -68,7 +68,11 @@ __global__ __launch_bounds__(NTH) void gru_fwd_wide_kernel(
     static_assert(KP % 8 == 0, "whole poll registers");
     constexpr int NPR = 8 * KP / 64;   // polled words per lane: 2 KP k of four rows
     constexpr int HRS = 2 * KP + 4;    // LDS row of a wavefront's h values
-    __shared__ __attribute__((aligned(16))) float part[2][NW][3][WR][WU];  // [parity][wave][gate][row][unit]
+    // [parity][wave][gate][row][unit]; the same memory holds W_hh's chunks
+    // before the loop
+    constexpr int kPart = 2 * NW * 3 * WR * WU, kChunk = 16 * (16 * KP + 4);
+    __shared__ __attribute__((aligned(16))) float shared0[kPart > kChunk ? kPart : kChunk];
+    float (&part)[2][NW][3][WR][WU] = *reinterpret_cast<float (*)[2][NW][3][WR][WU]>(shared0);
     __shared__ __attribute__((aligned(16))) float hrem[NW][WR][HRS];
     __shared__ int s_abort;
     __shared__ int s_local;
@@ -84,24 +88,61 @@ __global__ __launch_bounds__(NTH) void gru_fwd_wide_kernel(
     const int u = s * WU + ul;  // the lane's unit, as A row and as owner
     const int k0 = (2 * wave + hf) * KP;
 
+    // W_hh in chunks of one gate's 16 units (half of the slice) and every k,
+    // read in whole rows and handed out through LDS: a lane's KP values lie in
+    // one row, so its own loads would fetch 64 rows' lines per instruction,
+    // each several times (a launch of one step: 23.7 -> 20.8 us at H = 768)
     float wa[3][KP];
-    const bool vec = (H & 3) == 0 && (reinterpret_cast<uintptr_t>(w_hh) & 15u) == 0;
+    {
+        constexpr int NV = KP / 8;  // float4 of a chunk per thread
+        constexpr int KT = 16 * KP;
+        const bool vec = (H & 3) == 0 && (reinterpret_cast<uintptr_t>(w_hh) & 15u) == 0;
+        float4 r[2][NV];
+        auto load = [&](int c, float4 (&d)[NV]) {  // chunk c: gate c / 2, units 16 (c % 2) ..
 #pragma unroll
-    for (int g = 0; g < 3; ++g) {
-        const float* src = w_hh + ((size_t)g * H + (u < H ? u : 0)) * H;
+            for (int v = 0; v < NV; ++v) {
+                const int x = (int)threadIdx.x + NTH * v;
+                const int un = WU * s + 16 * (c % 2) + x / (KT / 4), k = 4 * (x % (KT / 4));
+                const float* src = w_hh + ((size_t)(c / 2) * H + un) * H + k;
+                if (vec) {
+                    const bool in = un < H && k < H;
+                    const float4 t = *reinterpret_cast<const float4*>(in ? src : w_hh);
+                    d[v] = make_float4(in ? t.x : 0.f, in ? t.y : 0.f, in ? t.z : 0.f, in ? t.w : 0.f);
+                } else {
+                    float e[4];
 #pragma unroll
-        for (int i = 0; i < KP; i += 4) {
-            const int k = k0 + i;
-            if (vec) {
-                const float4 v = u < H && k < H ? *reinterpret_cast<const float4*>(src + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-                wa[g][i] = v.x;
-                wa[g][i + 1] = v.y;
-                wa[g][i + 2] = v.z;
-                wa[g][i + 3] = v.w;
-            } else {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) wa[g][i + c] = u < H && k + c < H ? src[k + c] : 0.f;
+                    for (int q = 0; q < 4; ++q) {
+                        const bool in = un < H && k + q < H;
+                        const float t = *(in ? src + q : w_hh);
+                        e[q] = in ? t : 0.f;
+                    }
+                    d[v] = make_float4(e[0], e[1], e[2], e[3]);
+                }
             }
+        };
+        float (&chunk)[16][KT + 4] = *reinterpret_cast<float (*)[16][KT + 4]>(shared0);
+        load(0, r[0]);
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            if (c + 1 < 6) load(c + 1, r[(c + 1) & 1]);
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                const int x = (int)threadIdx.x + NTH * v;
+                *reinterpret_cast<float4*>(&chunk[x / (KT / 4)][4 * (x % (KT / 4))]) = r[c & 1][v];
+            }
+            __syncthreads();
+            const bool mine = ul / 16 == c % 2;
+#pragma unroll
+            for (int i = 0; i < KP; i += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(&chunk[ul % 16][k0 + i]);
+                float* d = &wa[c / 2][i];
+                const bool keep = c % 2 == 1 && !mine;
+                d[0] = keep ? d[0] : v.x;
+                d[1] = keep ? d[1] : v.y;
+                d[2] = keep ? d[2] : v.z;
+                d[3] = keep ? d[3] : v.w;
+            }
+            __syncthreads();
         }
     }
 

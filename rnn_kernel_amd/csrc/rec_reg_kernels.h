@@ -70,6 +70,52 @@ struct RegParams {
     int stall_block;                      // test failure injection (rec::Args::stall_block)
 };
 
+// Reads the W_hh entries of a forward workgroup (units [64 s, 64 s + 64), every
+// k, three gates) in chunks of 64 units x 64 k, one per slot j (the slice (s +
+// j) mod S) and gate g, with whole rows of consecutive lanes, and hands each to
+// take(j, g, chunk) in LDS ([unit][k], zero past H), from which the lanes pick
+// theirs.  A lane's own entries are 16 or 32 bytes of one row in 64 different
+// rows per load; read straight from memory that fetched every line several
+// times over: a launch of one step at H = 256 took 25 us, now 8 to 10 (MI355X,
+// B = 1 to 64; 14 -> 7.6 at H = 128; four rows, B = 200: 28 -> 16).  Called by
+// the NL compute threads (any others of the workgroup take its 3 S barriers).
+// Every load is issued before the first chunk
+// is written, and none under a branch (out-of-range ones read w_hh[0]).  For
+// rows that can be read as aligned float4 (RegParams::wvec); otherwise the lanes
+// read their own entries one by one, which measured faster than staging them
+// (H = 129, one step: 13.5 vs 15.2 us).
+constexpr int kWhhChunks = 2 * 64 * 68;  // floats of its two buffers
+template <int S, int NL, typename F>
+__device__ __forceinline__ void stage_whh(const float* __restrict__ w_hh, int H, int s, float (&buf)[2][64][68],
+                                          F take) {
+    constexpr int NV = 1024 / NL;  // float4 of a chunk per thread
+    float4 r[3 * S][NV];
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int c = 0; c < 3 * S; ++c) {
+        const int j = c / 3, g = c % 3;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int x = tid + NL * v;
+            const int u = 64 * s + x / 16, k = 64 * ((s + j) % S) + 4 * (x % 16);
+            const float* src = w_hh + ((size_t)g * H + u) * H + k;
+            const bool in = u < H && k < H;
+            const float4 t = *reinterpret_cast<const float4*>(in ? src : w_hh);
+            r[c][v] = make_float4(in ? t.x : 0.f, in ? t.y : 0.f, in ? t.z : 0.f, in ? t.w : 0.f);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 3 * S; ++c) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int x = tid + NL * v;
+            *reinterpret_cast<float4*>(&buf[c & 1][x / 16][4 * (x % 16)]) = r[c][v];
+        }
+        __syncthreads();
+        take(c / 3, c % 3, buf[c & 1]);
+    }
+}
+
 // Forward recurrence, S = ceil(H / 64) slices of 64 units (one workgroup
 // each) and R batch rows per workgroup, with the workgroup's own slice of
 // h_{t-1} taken from LDS (S = 1: no exchange at all).  Every wavefront runs
@@ -102,7 +148,10 @@ struct RegParams {
 // wavefront (registers or LDS-DMA, one to three steps ahead) measured 0.53
 // to 0.57 ms, while the same copies from L2-resident addresses measured
 // 0.455 ms.
-template <int S, int R, bool IO, int NWF = NW, bool FULL = false>
+// STAGE: W_hh through stage_whh (rows of aligned float4); an instance of its
+// own, because the step loop of the other one is compiled differently with
+// the staging in front of it (H = 129: 0.70 vs 0.68 us per step).
+template <int S, int R, bool IO, int NWF = NW, bool FULL = false, bool STAGE = FULL>
 __global__ __launch_bounds__(IO ? NWF * 64 + 64 : NWF * 64) void gru_fwd_local_kernel(
     const float* __restrict__ gx, const float* __restrict__ h0, const float* __restrict__ w_hh,
     const float* __restrict__ b_hh, float* __restrict__ y, float* __restrict__ hn,
@@ -171,6 +220,9 @@ __global__ __launch_bounds__(IO ? NWF * 64 + 64 : NWF * 64) void gru_fwd_local_k
                 for (int c = 0; c < 5; ++c) o[c] = io_out[t & 1][c][lane];
             };
             const rec::WaitCtl wc{abort_flag, p.abort_count, p.spin_limit};
+            if constexpr (STAGE) {
+                for (int c = 0; c < 3 * S; ++c) __syncthreads();  // stage_whh's
+            }
             (void)rec::group_on_one_xcd(p.xcc_words, gc.first, gc.stride, p.S, p.xcc_tag, wc, &s_local);
             int t_stop = T;
             for (int t = 0; t < T; ++t) {
@@ -202,32 +254,47 @@ __global__ __launch_bounds__(IO ? NWF * 64 + 64 : NWF * 64) void gru_fwd_local_k
 
     // slot j's W_hh entries in w?[KH j .. KH j + KH - 1]
     float wr[KH * S], wz[KH * S], wn[KH * S];
-    const bool vec = p.wvec != 0;
+    if constexpr (STAGE) {
+        __shared__ __attribute__((aligned(16))) float wbuf[2][64][68];
+        stage_whh<S, NWF * 64>(w_hh, H, s, wbuf, [&](int j, int g, const float (&w)[64][68]) {
+            float* d = (g == 0 ? wr : g == 1 ? wz : wn) + KH * j;
 #pragma unroll
-    for (int j = 0; j < S; ++j) {
+            for (int i = 0; i < KH; i += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(&w[fu][KP * Q + KH * hf + i]);
+                d[i] = v.x;
+                d[i + 1] = v.y;
+                d[i + 2] = v.z;
+                d[i + 3] = v.w;
+            }
+        });
+    } else {
+        const bool vec = p.wvec != 0;
 #pragma unroll
-        for (int i = 0; i < KH; i += 4) {
-            const int k = kof(j, i);
-            const float* pr = w_hh + (size_t)uf * H + k;
-            const float* pz = pr + (size_t)H * H;
-            const float* pn = pz + (size_t)H * H;
-            if (vec) {
-                const bool ok = ufvalid && k < H;
-                const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-                const float4 a = ok ? *reinterpret_cast<const float4*>(pr) : z4;
-                const float4 b = ok ? *reinterpret_cast<const float4*>(pz) : z4;
-                const float4 c = ok ? *reinterpret_cast<const float4*>(pn) : z4;
-                const int e = KH * j + i;
-                wr[e] = a.x; wr[e + 1] = a.y; wr[e + 2] = a.z; wr[e + 3] = a.w;
-                wz[e] = b.x; wz[e + 1] = b.y; wz[e + 2] = b.z; wz[e + 3] = b.w;
-                wn[e] = c.x; wn[e + 1] = c.y; wn[e + 2] = c.z; wn[e + 3] = c.w;
-            } else {
+        for (int j = 0; j < S; ++j) {
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const bool ok = ufvalid && k + c < H;
-                    wr[KH * j + i + c] = ok ? pr[c] : 0.f;
-                    wz[KH * j + i + c] = ok ? pz[c] : 0.f;
-                    wn[KH * j + i + c] = ok ? pn[c] : 0.f;
+            for (int i = 0; i < KH; i += 4) {
+                const int k = kof(j, i);
+                const float* pr = w_hh + (size_t)uf * H + k;
+                const float* pz = pr + (size_t)H * H;
+                const float* pn = pz + (size_t)H * H;
+                if (vec) {
+                    const bool ok = ufvalid && k < H;
+                    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+                    const float4 a = ok ? *reinterpret_cast<const float4*>(pr) : z4;
+                    const float4 b = ok ? *reinterpret_cast<const float4*>(pz) : z4;
+                    const float4 c = ok ? *reinterpret_cast<const float4*>(pn) : z4;
+                    const int e = KH * j + i;
+                    wr[e] = a.x; wr[e + 1] = a.y; wr[e + 2] = a.z; wr[e + 3] = a.w;
+                    wz[e] = b.x; wz[e + 1] = b.y; wz[e + 2] = b.z; wz[e + 3] = b.w;
+                    wn[e] = c.x; wn[e + 1] = c.y; wn[e + 2] = c.z; wn[e + 3] = c.w;
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        const bool ok = ufvalid && k + c < H;
+                        wr[KH * j + i + c] = ok ? pr[c] : 0.f;
+                        wz[KH * j + i + c] = ok ? pz[c] : 0.f;
+                        wn[KH * j + i + c] = ok ? pn[c] : 0.f;
+                    }
                 }
             }
         }
@@ -593,7 +660,11 @@ __global__ __launch_bounds__(NTH) void gru_fwd_mfma4_kernel(
     constexpr int WE = 32 * NR;      // polled words per wavefront: (slot, c, row)
     constexpr int NPR = WE > 64 ? 2 : 1;  // poll registers per lane
     typedef float f4 __attribute__((ext_vector_type(4)));
-    __shared__ __attribute__((aligned(16))) float part[2][NW][3][R][64];  // [parity][wave][gate][row][unit]
+    // [parity][wave][gate][row][unit]; the same memory holds W_hh's chunks
+    // before the loop
+    constexpr int kPart = 2 * NW * 3 * R * 64;
+    __shared__ __attribute__((aligned(16))) float shared0[kPart > kWhhChunks ? kPart : kWhhChunks];
+    float (&part)[2][NW][3][R][64] = *reinterpret_cast<float (*)[2][NW][3][R][64]>(shared0);
     __shared__ __attribute__((aligned(16))) float hloc[2][R][64];          // [parity][row][unit]
     __shared__ __attribute__((aligned(16))) float hrem[NW][NR > 0 ? NR : 1][R][8];  // per wave: [slot][row][c]
     __shared__ int s_abort;
@@ -613,15 +684,27 @@ __global__ __launch_bounds__(NTH) void gru_fwd_mfma4_kernel(
 
     // A operands: wa[g][8 j + c] = W_hh[g H + u][kof(j, c)] (0 past H)
     float wa[3][8 * S];
+    if (p.wvec) {
+        float (&wbuf)[2][64][68] = *reinterpret_cast<float (*)[2][64][68]>(shared0);
+        stage_whh<S, NTH>(w_hh, H, s, wbuf, [&](int j, int g, const float (&w)[64][68]) {
 #pragma unroll
-    for (int j = 0; j < S; ++j)
+            for (int i = 0; i < 8; i += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(&w[lane][8 * wave + i]);
+                wa[g][8 * j + i] = v.x;
+                wa[g][8 * j + i + 1] = v.y;
+                wa[g][8 * j + i + 2] = v.z;
+                wa[g][8 * j + i + 3] = v.w;
+            }
+        });
+    } else {
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const int k = kof(j, c);
+        for (int e = 0; e < 8 * S; ++e) {
+            const int k = kof(e / 8, e % 8);
             const bool ok = uvalid && k < H;
 #pragma unroll
-            for (int g = 0; g < 3; ++g) wa[g][8 * j + c] = ok ? w_hh[((size_t)g * H + u) * H + k] : 0.f;
+            for (int g = 0; g < 3; ++g) wa[g][e] = ok ? w_hh[((size_t)g * H + u) * H + k] : 0.f;
         }
+    }
 
     // wave r < R owns row row0 + r: its gate math, outputs and exchange words
     const int orow = row0 + (wave < R ? wave : 0);
