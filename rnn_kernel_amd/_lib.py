@@ -26,6 +26,8 @@ SIGNATURES = {
     "rka_gru_reserve_bytes": (_SZ, [_I, _I, _I]),
     "rka_gru_forward_workspace_bytes": (_SZ, [_I, _I, _I, _I]),
     "rka_gru_forward": (_I, [_P] * 9 + [_P, _SZ, _I, _I, _I, _I, _P]),
+    "rka_gru_stack_forward_workspace_bytes": (_SZ, [_I] * 5),
+    "rka_gru_stack_forward": (_I, [_I, _P, _P, _P, _P, _P, _P, _SZ, _I, _I, _I, _I, _P]),
     "rka_gru_backward_workspace_bytes": (_SZ, [_I, _I, _I, _I]),
     "rka_gru_backward": (_I, [_P] * 14 + [_P, _SZ, _I, _I, _I, _I, _P]),
     "rka_gemm_f32": (_I, [_I, _I, _I, _P, _I, _I, _P, _I, _I, _P, _P, _I, _P]),
@@ -103,6 +105,36 @@ def check(rc: int, what: str) -> None:
 def ptr(t) -> Optional[int]:
     """Device pointer of a tensor (None -> NULL)."""
     return None if t is None else t.data_ptr()
+
+
+def raw_stream(index: int) -> int:
+    """Handle of torch's current stream on CUDA device ``index`` (without
+    building a Stream object, where torch offers that)."""
+    import torch
+
+    global _raw_stream
+    if _raw_stream is None:
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                              lambda i: torch.cuda.current_stream(i).cuda_stream)
+    return _raw_stream(index)
+
+
+_raw_stream = None
+
+
+def call(index: int, name: str, *args) -> None:
+    """Entry point ``name`` with ``args`` and device ``index``'s current stream,
+    that device being current during the call; raises on a nonzero status."""
+    import torch
+
+    fn = getattr(load(), name)
+    if torch.cuda.current_device() == index:
+        rc = fn(*args, raw_stream(index))
+    else:
+        with torch.cuda.device(index):
+            rc = fn(*args, raw_stream(index))
+    if rc != 0:
+        check(rc, name)
 
 
 def profile_enable(on: bool) -> None:

@@ -3,6 +3,8 @@
 // in rec_reg_kernels.h).
 #include "rec_reg_kernels.h"
 
+#include <atomic>
+
 namespace rka {
 namespace {
 
@@ -85,6 +87,21 @@ const void* kernel_ptr(int dir, int cap, int rows, int slices, bool full = false
     }
 }
 
+// Workgroups of the kernel that a CU holds (-1: the query failed), asked once
+// per device and kernel (a query takes about a microsecond of every call).
+int blocks_per_cu(int device, int dir, int cap, int rows, int slices) {
+    static std::atomic<int> known[16][2][3][4];  // the answer + 1
+    std::atomic<int>* k =
+        device >= 0 && device < 16 ? &known[device][dir][rows == 1 ? 0 : rows == 2 ? 1 : 2][slices - 1] : nullptr;
+    if (k != nullptr && k->load(std::memory_order_relaxed) > 0) return k->load(std::memory_order_relaxed) - 1;
+    int per_cu = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel_ptr(dir, cap, rows, slices),
+                                                     block_threads(dir, rows, slices), 0) != hipSuccess)
+        return -1;
+    if (k != nullptr) k->store(per_cu + 1, std::memory_order_relaxed);
+    return per_cu;
+}
+
 // Units per workgroup and whether the register-resident kernels hold H.
 void chunk_of(int dir, int H, int* chunk, int* cap) {
     (void)dir;
@@ -121,10 +138,8 @@ int reg_choose(int dir, int batch, int hidden, const DeviceInfo& dev, int fixed_
     for (int rows : {1, 2, 4}) {
         if (rows > max_rows(dir, S) || (fixed_rows && rows != fixed_rows)) continue;
         const int G = (batch + rows - 1) / rows;
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel_ptr(dir, cap, rows, S), block_threads(dir, rows, S),
-                                                         0) != hipSuccess)
-            continue;
+        const int per_cu = blocks_per_cu(dev.device, dir, cap, rows, S);
+        if (per_cu < 0) continue;
         const long resident = (long)per_cu * dev.num_cus;
         chosen = rows;  // the last candidate (the most rows) unless one fits
         chosen_cap = resident;

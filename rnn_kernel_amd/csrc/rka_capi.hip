@@ -71,6 +71,21 @@ FwdLayout fwd_layout(int B, int T, int I, int H) {
     return l;
 }
 
+// Workspace of a stack: the layers' own (shared), then the outputs of the
+// layers before the last, two in turn.
+struct StackLayout {
+    size_t layer, y[2], total;
+};
+StackLayout stack_layout(int L, int B, int T, int I, int H) {
+    StackLayout l{};
+    l.layer = fwd_layout(B, T, I, H).total;
+    const size_t y = align_up((size_t)B * T * H * sizeof(float), 256);
+    l.y[0] = align_up(l.layer, 256);
+    l.y[1] = l.y[0] + y;
+    l.total = l.y[0] + (size_t)std::min(L - 1, 2) * y;
+    return l;
+}
+
 struct BwdLayout {
     size_t g, rec, part_hh, part_ih, total;
     int ks_hh, ks_ih;  // split-K slices
@@ -210,6 +225,37 @@ int rka_gru_forward(const float* x, const float* h0, const float* w_ih, const fl
     StageScope scope(1, s);
     return launch_rec_forward(gx, h0, w_hh, b_hh, y, hn, reserve, ws + l.rec, l.total - l.rec, B, T, H, s,
                               false);
+}
+
+size_t rka_gru_stack_forward_workspace_bytes(int num_layers, int batch, int seq_len, int input_size, int hidden_size) {
+    if (num_layers < 1 || batch < 1 || seq_len < 1 || hidden_size < 1 || input_size < 1) return 0;
+    return stack_layout(num_layers, batch, seq_len, input_size, hidden_size).total;
+}
+
+int rka_gru_stack_forward(int num_layers, const float* x, const float* h0, const float* const* weights, float* y,
+                          float* hn, void* workspace, size_t workspace_bytes, int batch, int seq_len, int input_size,
+                          int hidden_size, void* stream) {
+    clear_error();
+    if (num_layers < 1) return fail(RKA_ERR_INVALID_ARGUMENT, "rka_gru_stack_forward: num_layers must be >= 1");
+    RKA_RETURN_IF_ERR(check_dims(batch, seq_len, input_size, hidden_size));
+    if (!x || !h0 || !weights || !y || !hn)
+        return fail(RKA_ERR_INVALID_ARGUMENT, "rka_gru_stack_forward: null tensor pointer");
+    const StackLayout l = stack_layout(num_layers, batch, seq_len, input_size, hidden_size);
+    if (!workspace || workspace_bytes < l.total)
+        return fail(RKA_ERR_WORKSPACE_TOO_SMALL, "rka_gru_stack_forward: workspace needs " + std::to_string(l.total) +
+                                                     " bytes, got " + std::to_string(workspace_bytes));
+    char* ws = reinterpret_cast<char*>(workspace);
+    const size_t state = (size_t)batch * hidden_size;
+    const float* in = x;
+    for (int k = 0; k < num_layers; ++k) {
+        float* out = k + 1 == num_layers ? y : reinterpret_cast<float*>(ws + l.y[k & 1]);
+        const float* const* w = weights + 4 * k;
+        RKA_RETURN_IF_ERR(rka_gru_forward(in, h0 + k * state, w[0], w[1], w[2], w[3], out, hn + k * state, nullptr, ws,
+                                          l.layer, batch, seq_len, k == 0 ? input_size : hidden_size, hidden_size,
+                                          stream));
+        in = out;
+    }
+    return 0;
 }
 
 int rka_gru_backward(const float* x, const float* h0, const float* w_ih, const float* w_hh,

@@ -27,8 +27,8 @@ from torch import nn
 from . import _lib
 
 
-def _stream(device) -> int:
-    return torch.cuda.current_stream(device=device).cuda_stream
+def _index_of(device) -> int:
+    return device.index if device.index is not None else torch.cuda.current_device()
 
 
 def _check_tensor(t: torch.Tensor, name: str) -> None:
@@ -56,10 +56,8 @@ class HeadFunction(torch.autograd.Function):
         rows = out_c.numel() // hidden
         pred = torch.empty(out.shape[:-1], device=out.device, dtype=torch.float32)
         if rows > 0:
-            lib = _lib.load()
-            with torch.cuda.device(out.device):
-                _lib.check(lib.rka_head_forward(_lib.ptr(out_c), _lib.ptr(w_c), _lib.ptr(b_c), _lib.ptr(pred),
-                                                rows, hidden, _stream(out.device)), "rka_head_forward")
+            _lib.call(_index_of(out.device), "rka_head_forward", out_c.data_ptr(), w_c.data_ptr(), b_c.data_ptr(),
+                      pred.data_ptr(), rows, hidden)
         ctx.save_for_backward(out_c, w_c)
         return pred
 
@@ -78,11 +76,9 @@ class HeadFunction(torch.autograd.Function):
         g = grad_pred.contiguous()
         lib = _lib.load()
         ws_bytes = lib.rka_head_backward_workspace_bytes(rows, hidden)
-        with torch.cuda.device(out.device):
-            ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=out.device)
-            _lib.check(lib.rka_head_backward(_lib.ptr(out), _lib.ptr(weight), _lib.ptr(g), _lib.ptr(grad_out),
-                                             _lib.ptr(grad_w), _lib.ptr(grad_b), _lib.ptr(ws), ws_bytes, rows,
-                                             hidden, _stream(out.device)), "rka_head_backward")
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=out.device)
+        _lib.call(_index_of(out.device), "rka_head_backward", out.data_ptr(), weight.data_ptr(), g.data_ptr(),
+                  _lib.ptr(grad_out), grad_w.data_ptr(), grad_b.data_ptr(), ws.data_ptr(), ws_bytes, rows, hidden)
         return grad_out, grad_w, grad_b
 
 
@@ -129,10 +125,9 @@ class MSELossFunction(torch.autograd.Function):
         loss = torch.empty((), device=pred.device, dtype=torch.float32)
         lib = _lib.load()
         ws_bytes = lib.rka_mse_workspace_bytes(n)
-        with torch.cuda.device(pred.device):
-            ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=pred.device)
-            _lib.check(lib.rka_mse_forward(_lib.ptr(p), _lib.ptr(t), _lib.ptr(loss), _lib.ptr(ws), ws_bytes, n,
-                                           _stream(pred.device)), "rka_mse_forward")
+        ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=pred.device)
+        _lib.call(_index_of(pred.device), "rka_mse_forward", p.data_ptr(), t.data_ptr(), loss.data_ptr(), ws.data_ptr(),
+                  ws_bytes, n)
         ctx.save_for_backward(p, t)
         return loss
 
@@ -141,10 +136,8 @@ class MSELossFunction(torch.autograd.Function):
         p, t = ctx.saved_tensors
         g = grad_loss.contiguous()
         grad = torch.empty_like(p)
-        lib = _lib.load()
-        with torch.cuda.device(p.device):
-            _lib.check(lib.rka_mse_backward(_lib.ptr(p), _lib.ptr(t), _lib.ptr(g), _lib.ptr(grad), p.numel(),
-                                            _stream(p.device)), "rka_mse_backward")
+        _lib.call(_index_of(p.device), "rka_mse_backward", p.data_ptr(), t.data_ptr(), g.data_ptr(), grad.data_ptr(),
+                  p.numel())
         return grad, None
 
 
@@ -178,7 +171,6 @@ class AdamW(torch.optim.Optimizer):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
-        lib = _lib.load()
         for group in self.param_groups:
             by_step: dict = {}
             for p in group["params"]:
@@ -205,10 +197,8 @@ class AdamW(torch.optim.Optimizer):
                 m = P(*[self.state[p]["exp_avg"].data_ptr() for p in plist])
                 v = P(*[self.state[p]["exp_avg_sq"].data_ptr() for p in plist])
                 numels = (ctypes.c_size_t * n)(*[p.numel() for p in plist])
-                with torch.cuda.device(device):
-                    _lib.check(lib.rka_adamw_step(params, grads, m, v, numels, n, group["lr"], beta1, beta2,
-                                                  group["eps"], group["weight_decay"], step, _stream(device)),
-                               "rka_adamw_step")
+                _lib.call(_index_of(device), "rka_adamw_step", params, grads, m, v, numels, n, group["lr"], beta1, beta2,
+                          group["eps"], group["weight_decay"], step)
         return loss
 
 
