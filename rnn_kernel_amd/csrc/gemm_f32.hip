@@ -790,127 +790,6 @@ __global__ __launch_bounds__(NT) void gemm_f32_pair_kernel(GemmArgs p0, GemmArgs
     }
 }
 
-// ------------------------------------- large-tile weight-gradient pair ---
-// The two split-K weight-gradient products (both operands k-major) with
-// workgroups of WMW x WNW wavefronts, each wavefront computing a 64x64
-// sub-tile exactly as above (the same LDS forms and MFMA order, so every
-// partial sum equals the 128x128 kernel's bit for bit): a workgroup tile is
-// (64 WMW) x (64 WNW), one (tile, k-slice) item per workgroup and one
-// workgroup per CU.  At c2 the 3H = 768 gate rows and the 256 columns of
-// each product are four 192x256 tiles, 32 k-slices each, 256 items in all.
-// A 192x256 tile loads 28 KB of operands per 16-deep stage for 1.57 MFLOP,
-// against 16 KB for 0.52 MFLOP with 128x128 tiles; twelve wavefronts keep
-// three per SIMD, as three 128x128 workgroups per CU do.  The operand tiles
-// go straight to LDS through a ring of BigTile::D stages (five: 140 KB).
-// Measured at c2 (same box, three alternating pairs): 234.5 vs 240.5 us.
-// The same workgroups for the direct products (256x192 tiles for the
-// input projection, 128x256 for the input gradient, one workgroup per CU)
-// measured slower than three 128x128 workgroups per CU: 125 vs 120 us and
-// 126 vs 110 us.
-template <int WMW, int WNW>
-struct BigTile {
-    static constexpr int BM = 64 * WMW, BN = 64 * WNW, NW = WMW * WNW, NT = 64 * NW;
-    static constexpr int ACH = BM / 16, BCH = BN / 16, CH = ACH + BCH;  // 1 KB wave loads per stage
-    static constexpr int STAGE = 16 * (BM + BN);                        // floats per ring stage
-    // ring stages: as many as 160 KB of LDS holds, at most 6
-    static constexpr int D = 163840 / (STAGE * 4) < 6 ? 163840 / (STAGE * 4) : 6;
-    static constexpr int SMEM_BYTES = D * STAGE * 4;
-    static_assert(D >= 3, "the ring needs three stages");
-};
-
-
-// One item (split_coords(p, id)) of a split-K product of k-major operands.
-template <int WMW, int WNW, bool BSHIFT>
-__device__ __forceinline__ void big_split_item(const GemmArgs& p, int id, float* smem) {
-    using T = BigTile<WMW, WNW>;
-    constexpr int D = T::D;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave % WMW, wn = wave / WMW;
-    const int nw = (T::CH - wave + T::NW - 1) / T::NW;  // this wave's loads per stage
-    int bx, by, bz;
-    split_coords(p, id, bx, by, bz);
-    const int m0 = bx * T::BM, n0 = by * T::BN, kbeg = bz * p.kchunk;
-    const int nkb = p.kchunk / 16;
-    const bool colsum = p.want_colsum && by == 0;
-    auto issue = [&](int kb) {
-        const int k0 = kbeg + 16 * kb;
-        float* st = smem + (kb % D) * T::STAGE;
-        for (int c = wave; c < T::CH; c += T::NW) {
-            if (c < T::ACH)
-                lds_dma16(dma_src<1, false, false, false, T::BM>(p.a, m0, k0, 64 * c + lane), st + 256 * c);
-            else
-                lds_dma16(dma_src<1, BSHIFT, false, false, T::BN>(p.b, n0, k0, 64 * (c - T::ACH) + lane),
-                          st + 16 * T::BM + 256 * (c - T::ACH));
-        }
-    };
-    for (int kb = 0; kb < D - 1 && kb < nkb; ++kb) issue(kb);
-    const int i = lane & 15, g = lane >> 4;
-    floatx4 acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-    float cs = 0.f;
-    for (int kb = 0; kb < nkb; ++kb) {
-        // stage kb has landed once at most the later stages already issued
-        // (up to D - 2 of them, nw loads each) are outstanding
-        wait_vmcnt(nw * min(D - 2, nkb - 1 - kb));
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        const float* as = smem + (kb % D) * T::STAGE;
-        const float* bs = as + 16 * T::BM;
-        // operand fragments of this stage (the k forms and order of
-        // mma_tile), then the first MFMA step, so the matrix cores start
-        // before the loads into the freed stage are addressed and issued
-        float4 fa[4], fb[4];
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-            fa[x] = *reinterpret_cast<const float4*>(as + (4 * g + x) * T::BM + wm * 64 + 4 * i);
-            fb[x] = *reinterpret_cast<const float4*>(bs + (4 * g + x) * T::BN + wn * 64 + 4 * i);
-        }
-        auto mstep = [&](int j) {
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[j][a], fb[j][b], acc[a][b], 0, 0, 0);
-        };
-        __builtin_amdgcn_sched_barrier(0);
-        mstep(0);
-        __builtin_amdgcn_sched_barrier(0);
-        // the stage consumed at kb - 1 is free: every wave is past its reads
-        if (kb + D - 1 < nkb) issue(kb + D - 1);
-        if (colsum && tid < T::BM) {
-            // column sums of A (the bias gradients), in k order
-#pragma unroll
-            for (int kk = 0; kk < 16; ++kk) cs += as[kk * T::BM + tid];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        mstep(1);
-        mstep(2);
-        mstep(3);
-    }
-    store_c<1, true, false>(p, m0, n0, bz, wm, wn, lane, acc);
-    if (colsum && tid < T::BM) {
-        float* cpart = p.partial + (size_t)p.ksplit_total * p.m * p.n;
-        cpart[(size_t)(p.z_off + bz) * p.m + m0 + tid] = cs;
-    }
-}
-
-// The two weight-gradient products, one item per workgroup: items
-// [0, tiles0 * ksplit0) of the first, then the second's.
-template <int WMW, int WNW, bool SHIFT0>
-__global__ __launch_bounds__(64 * WMW * WNW) void gemm_big_pair_kernel(GemmArgs p0, GemmArgs p1) {
-    extern __shared__ __attribute__((aligned(16))) float big_smem[];
-    const int items0 = p0.tiles * p0.ksplit;
-    if ((int)blockIdx.x < items0)
-        big_split_item<WMW, WNW, SHIFT0>(p0, blockIdx.x, big_smem);
-    else
-        big_split_item<WMW, WNW, false>(p1, blockIdx.x - items0, big_smem);
-}
-
 // out[o*ldc + n] = sum_z partial[z][(o+rot)%m][n]; colsum likewise.  With
 // vec, a team of kTeam threads (consecutive lanes) sums one float4 of a row:
 // member r takes slices r, r + kTeam, ... in order, then the team's sums are
@@ -1027,6 +906,9 @@ __global__ __launch_bounds__(NT) void gemm_direct_reduce_kernel(GemmArgs p, Redu
 
 // ------------------------------------------------------- small products ---
 #include "gemm_small.h"
+
+// ------------------------------------------------------- large products ---
+#include "gemm_split.h"
 
 // ------------------------------------------------- narrow last columns ---
 // A split-K product whose n is whole 128-column panels plus w <= kNarrowMax
@@ -1214,38 +1096,46 @@ int launch_gemm(GemmArgs args, int ksplit, bool av, bool bv, hipStream_t stream)
 std::atomic<int> g_gemm_tiles{RKA_GEMM_TILES_AUTO};
 
 // Tiles a direct product runs in.
-enum DirectTile { TILE_128, TILE_128x64, TILE_64, TILE_32 };
+enum DirectTile { TILE_128, TILE_SPLIT, TILE_128x64, TILE_64, TILE_32 };
 using Tile128x64 = SmallTile<128, 64, 64, 32, 16>;
 using Tile64 = SmallTile<64, 64, 32, 32, 16>;
 using Tile32 = SmallTile<32, 32, 32, 32, 64>;
 
 // The tile with the least work on the busiest CU: tiles per CU, rounded up,
 // times the tile's area, times the measured cost of a unit of area (large
-// products that divide evenly: the 128x128 ring 1, 128x64 1.02, 64x64 1.07,
-// 32x32 1.30; the ring's register path for operands that are not 16-byte
+// products that divide evenly: the 128x128 ring 1, 128x128 split into bf16 pieces
+// 0.70, 128x64 1.02, 64x64 1.07, 32x32 1.30; the ring's register path for operands that are not 16-byte
 // aligned 1.45).  Rounding up is what decides: 8192 x 2304 (k = 768) is 4.5
 // 128x128 tiles per CU, 8192 x 128 a quarter.  Measured on MI355X (us, 128 /
-// 128x64 / 64 / 32): 32768 x 768, k = 256: 113 / 115 / 118 / 154; 8192 x 2304,
-// k = 768: 271 / 246 / 257 / 319; 8192 x 128, k = 768: 59 / 36 / 23 / 20;
+// 128x64 / 64 / 32): 32768 x 768, k = 256: 113 / 115 / 118 / 154 (split 80); 8192 x
+// 2304, k = 768: 271 / 246 / 257 / 319 (split 166); 8192 x 128, k = 768: 59 / 36 / 23 / 20;
 // 32768 x 129, k = 387 (not aligned): 77 / 53 / 55 / 73; 64 x 768, k = 256:
 // 22 / 13 / 9.0 / 4.3; 1 x 256, k = 768: 55 / 35 / 21 / 8.2.
 DirectTile direct_tile(const GemmArgs& g) {
-    if (g_gemm_tiles.load(std::memory_order_relaxed) != RKA_GEMM_TILES_AUTO || g.a.kmajor) return TILE_128;
+    if (g.a.kmajor) return TILE_128;
+    const bool vec = g.a_vec && g.b_vec;
     auto cost = [&](int tm, int tn, double unit) {
         const long long tiles = (long long)((g.m + tm - 1) / tm) * ((g.n + tn - 1) / tn);
         return (double)((tiles + 255) / 256) * tm * tn * unit;
     };
     DirectTile best = TILE_128;
-    double least = cost(128, 128, g.a_vec && g.b_vec ? 1.0 : 1.45);
+    double least = cost(128, 128, vec ? 1.0 : 1.45);
     auto consider = [&](DirectTile t, double c) {
         if (c < least) {
             best = t;
             least = c;
         }
     };
-    consider(TILE_128x64, cost(128, 64, 1.02));
-    consider(TILE_64, cost(64, 64, 1.07));
-    consider(TILE_32, cost(32, 32, 1.30));
+    if (vec) consider(TILE_SPLIT, cost(128, 128, 0.70));
+    if (g_gemm_tiles.load(std::memory_order_relaxed) == RKA_GEMM_TILES_AUTO) {
+        consider(TILE_128x64, cost(128, 64, 1.02));
+        consider(TILE_64, cost(64, 64, 1.07));
+        consider(TILE_32, cost(32, 32, 1.30));
+    } else if (best == TILE_SPLIT) {
+        // 128x128 tiles throughout: the split form where it is the choice
+        // anyway, else the ring
+        if (least > std::min(cost(128, 64, 1.02), std::min(cost(64, 64, 1.07), cost(32, 32, 1.30)))) best = TILE_128;
+    }
     return best;
 }
 
@@ -1264,6 +1154,21 @@ int launch_small_t(GemmArgs args, const ReduceJob* j0, const ReduceJob* j1, long
     return 0;
 }
 
+template <int BKM>
+int launch_split(GemmArgs args, const ReduceJob* j0, const ReduceJob* j1, long reducers, hipStream_t stream) {
+    args.tiles_m = (args.m + kSplitTile - 1) / kSplitTile;
+    const long long tiles = (long long)args.tiles_m * ((args.n + kSplitTile - 1) / kSplitTile);
+    if (tiles + reducers > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
+    args.tiles = (int)tiles;
+    const dim3 grid((unsigned)(tiles + reducers));
+    if (j0)
+        hipLaunchKernelGGL((gemm_split_reduce_kernel<BKM>), grid, dim3(NT), 0, stream, args, *j0, *j1);
+    else
+        hipLaunchKernelGGL((gemm_split_kernel<BKM>), grid, dim3(NT), 0, stream, args);
+    RKA_RETURN_IF_HIP(hipGetLastError());
+    return 0;
+}
+
 // A direct product of a row-major A in `tile`s (not TILE_128), with the
 // reductions j0, j1 (both or neither) in `reducers` workgroups after them.
 int launch_small(DirectTile tile, const GemmArgs& args, const ReduceJob* j0, const ReduceJob* j1, long reducers,
@@ -1275,6 +1180,7 @@ int launch_small(DirectTile tile, const GemmArgs& args, const ReduceJob* j0, con
         return launch_small_t<0, B, S, false>(args, j0, j1, reducers, stream);
     };
     auto run = [&](auto bk) {
+        if (tile == TILE_SPLIT) return launch_split<decltype(bk)::value>(args, j0, j1, reducers, stream);
         if (tile == TILE_32) return with(bk, Tile32{});
         if (tile == TILE_64) return with(bk, Tile64{});
         return with(bk, Tile128x64{});
@@ -1332,51 +1238,38 @@ namespace {
 // three resident workgroups per CU.
 int ring_ksplit(int m, int n, int k) { return choose_ksplit(m, n, k, 128, 3); }
 
-// Whether the pair's items in 192x256 tiles divide evenly over the CUs.
-bool big_pair_divides(int m, int n0, int n1, int k, int num_cus) {
-    using T = BigTile<3, 4>;
-    long long items = 0;
-    for (int n : {n0, n1}) {
-        const int ks = ring_ksplit(m, n, k);
-        if (m % T::BM != 0 || n % T::BN != 0 || k % (ks * kSplitBK) != 0) return false;
-        items += (long long)(m / T::BM) * (n / T::BN) * ks;
-    }
-    return num_cus > 0 && items % num_cus == 0;
-}
-
 struct PairPlan {
-    DirectTile tile;  // TILE_64, TILE_128x64 or TILE_128 (the ring)
+    DirectTile tile;  // TILE_SPLIT, TILE_64, TILE_128x64 or TILE_128 (the ring)
     int ks0, ks1;
 };
 
 // Tile and slices of the weight-gradient pair (m = 3H gate rows, n0 and n1
-// columns, k = B T) outside the 192x256 tiles.  Both products take the same
+// columns, k = B T).  Both products take the same
 // slices, so that every workgroup has the same work; the candidates are
 // multiples of 8 (a slice's tiles then share an XCD, split_coords) and fewer
-// than 8, each slice at least four 16-deep stages and at most 2048 values long
+// than 8, each slice at least four 16-deep stages and at most 4096 values long
 // (the length of a chain of float32 additions).  Taken is the least of
 //   workgroups per CU x (stages + 2) x (time of a stage at that many)
 //   + the partial sums, written and read again,
 // where up to four workgroups share a CU and a part of one counts whole.  A
 // stage of a 64x64 tile was measured at 0.75, 0.5, 0.38 and 0.35 us for one,
 // two, three and four or more workgroups per CU (its MFMAs alone take 0.21); a
-// 128x64 tile takes 1.85 times that and the 128x128 ring, a candidate where
-// every extent divides by 128, 3.24 times.  Measured on MI355X (pair, us; 128x128
+// 128x64 tile takes 1.85 times that and a split 128x128 one (operands of aligned
+// float4 rows) 2.1 times.  Measured on MI355X (pair, us; 128x128
 // ring, now): m = 576, n = 192 + 192, k = 32768: 218, 158; 192, 64 + 64, 32768:
 // 50, 25; 384, 128 + 128, 32768: 84, 75; 387, 129 + 129, 32768: 163, 151; 384, 128 +
 // 64, 51200: 120, 86; 768, 256 + 128, 8192: 61, 58.
 PairPlan make_pair_plan(int m, int n0, int n1, int k) {
-    PairPlan best{TILE_128x64, ring_ksplit(m, n0, k), ring_ksplit(m, n1, k)};
-    if (big_pair_divides(m, n0, n1, k, 256)) return best;  // the same slices if its operands are not aligned
+    PairPlan best{TILE_128x64, 1, 1};
     constexpr int kMaxSlices = 256;
     constexpr double kStage[4] = {0.75, 0.5, 0.38, 0.35};
     const int most = std::min(kMaxSlices, std::max(1, k / (4 * kSplitBK)));
-    const int least = std::min(most, (k + 2047) / 2048);
+    const int least = std::min(most, (k + 4095) / 4096);
     double least_cost = 1e30;
-    for (const DirectTile tile : {TILE_64, TILE_128x64, TILE_128}) {
-        if (tile == TILE_128 && (m % 128 || n0 % 128 || n1 % 128)) continue;
-        const int tm = tile == TILE_64 ? 64 : 128, tn = tile == TILE_128 ? 128 : 64;
-        const double unit = tile == TILE_64 ? 1.0 : tile == TILE_128x64 ? 1.85 : 3.24;
+    for (const DirectTile tile : {TILE_64, TILE_128x64, TILE_SPLIT}) {
+        if (tile == TILE_SPLIT && (n0 % 4 || n1 % 4)) continue;
+        const int tm = tile == TILE_64 ? 64 : 128, tn = tile == TILE_SPLIT ? 128 : 64;
+        const double unit = tile == TILE_64 ? 1.0 : tile == TILE_128x64 ? 1.85 : 2.1;
         const double tiles = (double)((m + tm - 1) / tm) * ((n0 + tn - 1) / tn + (n1 + tn - 1) / tn);
         for (int ks = 1; ks <= most; ks += ks < 8 ? 1 : 8) {
             if (ks < least && ks + 8 <= most) continue;
@@ -1416,17 +1309,18 @@ bool pair_is_direct(const SplitProduct& p0, const SplitProduct& p1) {
            g_gemm_tiles.load(std::memory_order_relaxed) == RKA_GEMM_TILES_AUTO;
 }
 
-template <typename S>
-int launch_small_pair(const SplitProduct& p0, const SplitProduct& p1, GemmArgs a0, GemmArgs a1, hipStream_t stream) {
+// Launches the pair in tm x tn tiles: launch(grid, first product, second).
+template <typename F>
+int launch_pair_tiles(const SplitProduct& p0, const SplitProduct& p1, GemmArgs a0, GemmArgs a1, int tm, int tn,
+                      F launch) {
     long long items = 0;
     for (GemmArgs* g : {&a0, &a1}) {
         g->narrow = 0;
-        g->tiles_m = (g->m + S::TM - 1) / S::TM;
-        g->tiles = g->tiles_m * ((g->n + S::TN - 1) / S::TN);
+        g->tiles_m = (g->m + tm - 1) / tm;
+        g->tiles = g->tiles_m * ((g->n + tn - 1) / tn);
         items += (long long)g->tiles * g->ksplit;
     }
     if (items > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
-    const dim3 grid((unsigned)items);
     if (pair_is_direct(p0, p1)) {
         for (const auto& pa : {std::make_pair(&p0, &a0), std::make_pair(&p1, &a1)}) {
             pa.second->c = pa.first->c;
@@ -1436,18 +1330,26 @@ int launch_small_pair(const SplitProduct& p0, const SplitProduct& p1, GemmArgs a
             pa.second->c_vec = pa.first->ldc % 4 == 0 && aligned16(pa.first->c) ? 1 : 0;
         }
     }
-    if (a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec)
-        hipLaunchKernelGGL((gemm_small_pair_kernel<S, true, true>), grid, dim3(NT), 0, stream, a0, a1);
-    else
-        hipLaunchKernelGGL((gemm_small_pair_kernel<S, true, false>), grid, dim3(NT), 0, stream, a0, a1);
+    launch(dim3((unsigned)items), a0, a1);
     RKA_RETURN_IF_HIP(hipGetLastError());
     return 0;
+}
+
+template <typename S>
+int launch_small_pair(const SplitProduct& p0, const SplitProduct& p1, const GemmArgs& a0, const GemmArgs& a1,
+                      hipStream_t stream) {
+    return launch_pair_tiles(p0, p1, a0, a1, S::TM, S::TN, [&](dim3 grid, const GemmArgs& x, const GemmArgs& y) {
+        if (a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec)
+            hipLaunchKernelGGL((gemm_small_pair_kernel<S, true, true>), grid, dim3(NT), 0, stream, x, y);
+        else
+            hipLaunchKernelGGL((gemm_small_pair_kernel<S, true, false>), grid, dim3(NT), 0, stream, x, y);
+    });
 }
 }  // namespace
 
 void choose_pair_ksplit(int m, int n0, int n1, int k, int* ks0, int* ks1) {
     PairPlan p = plan_pair(m, n0, n1, k);
-    if (g_gemm_tiles.load(std::memory_order_relaxed) != RKA_GEMM_TILES_AUTO)
+    if (g_gemm_tiles.load(std::memory_order_relaxed) != RKA_GEMM_TILES_AUTO && p.tile != TILE_SPLIT)
         p = PairPlan{TILE_128, ring_ksplit(m, n0, k), ring_ksplit(m, n1, k)};
     *ks0 = p.ks0;
     *ks1 = p.ks1;
@@ -1498,32 +1400,6 @@ int split_args(int m, int n, int k, const GemmOperand& a, const GemmOperand& b, 
     return 0;
 }
 
-// The weight-gradient pair in 192x256 tiles (3H = 768 gate rows in four
-// tiles, n = H or I = 256 in one), one item (tile, k-slice) per workgroup.
-// Every k-slice must be whole 16-deep stages of the same length.
-int try_big_pair(GemmArgs a0, GemmArgs a1, bool shift0, hipStream_t stream, bool* launched) {
-    *launched = false;
-    if (g_gemm_tiles.load(std::memory_order_relaxed) != RKA_GEMM_TILES_AUTO) return 0;
-    const DeviceInfo* dev = nullptr;
-    RKA_RETURN_IF_ERR(current_device_info(&dev));
-    using T = BigTile<3, 4>;
-    int items = 0;
-    for (GemmArgs* g : {&a0, &a1}) {
-        if (!g->a_vec || !g->b_vec || !g->c_vec || g->kchunk <= 0 || g->k != g->ksplit * g->kchunk) return 0;
-        if (g->m % T::BM != 0 || g->n % T::BN != 0) return 0;
-        g->tiles_m = g->m / T::BM;
-        g->tiles = g->tiles_m * (g->n / T::BN);
-        items += g->tiles * g->ksplit;
-    }
-    if (dev->num_cus <= 0 || items % dev->num_cus != 0) return 0;
-    *launched = true;
-    auto kern = shift0 ? gemm_big_pair_kernel<3, 4, true> : gemm_big_pair_kernel<3, 4, false>;
-    RKA_RETURN_IF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, T::SMEM_BYTES));
-    hipLaunchKernelGGL(kern, dim3(items), dim3(T::NT), T::SMEM_BYTES, stream, a0, a1);
-    RKA_RETURN_IF_HIP(hipGetLastError());
-    return 0;
-}
 }  // namespace
 
 int gemm_splitk_partials(int m, int n, int k, const GemmOperand& a, const GemmOperand& b, bool want_colsum,
@@ -1542,15 +1418,15 @@ int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, hi
     if (p1.b.shift_T > 0) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: only the first product of a pair is remapped");
     const bool seg = a0.a.seg.len || a0.b.seg.len || a1.a.seg.len || a1.b.seg.len;
     if (seg) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: pair products take whole operands");
-    const bool ring = g_gemm_tiles.load(std::memory_order_relaxed) != RKA_GEMM_TILES_AUTO || p0.b.shift_T == 0;
-    bool launched = false;
-    RKA_RETURN_IF_ERR(try_big_pair(a0, a1, p0.b.shift_T > 0, stream, &launched));
-    if (launched) return 0;
-    if (!ring) {
-        const PairPlan plan = plan_pair(p0.m, p0.n, p1.n, p0.k);
-        if (plan.tile == TILE_64) return launch_small_pair<Tile64>(p0, p1, a0, a1, stream);
-        if (plan.tile == TILE_128x64 || !(a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec) || pair_is_direct(p0, p1))
-            return launch_small_pair<Tile128x64>(p0, p1, a0, a1, stream);
+    if (p0.b.shift_T > 0) {
+        const bool any = g_gemm_tiles.load(std::memory_order_relaxed) == RKA_GEMM_TILES_AUTO;
+        const bool vec = a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec;
+        const DirectTile tile = plan_pair(p0.m, p0.n, p1.n, p0.k).tile;
+        if (tile == TILE_SPLIT && vec) return launch_pair_tiles(p0, p1, a0, a1, kSplitTile, kSplitTile, [&](dim3 g, const GemmArgs& x, const GemmArgs& y) {
+            hipLaunchKernelGGL(gemm_split_pair_kernel, g, dim3(NT), 0, stream, x, y);
+        });
+        if (any && tile == TILE_64) return launch_small_pair<Tile64>(p0, p1, a0, a1, stream);
+        if (any) return launch_small_pair<Tile128x64>(p0, p1, a0, a1, stream);
     }
     const dim3 grid(a0.tiles * a0.ksplit + a1.tiles * a1.ksplit);
     const bool ua = !(a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec);
@@ -1653,7 +1529,7 @@ int gemm_direct_reduce_pair(int m, int n, int k, const GemmOperand& a, const Gem
         if (reducers == 0) return launch_small(tile, args, nullptr, nullptr, 0, stream);
         // smaller workgroups than the ring's: up to four reducing ones per CU
         const size_t want = ((j0.total + j1.total) * kTeam + NT - 1) / NT;
-        const long most = 4 * reducers;
+        const long most = (tile == TILE_SPLIT ? 1 : 4) * reducers;
         return launch_small(tile, args, &j0, &j1, (long)std::min<size_t>(want, most), stream);
     }
     if (!a.kmajor && !b.kmajor)

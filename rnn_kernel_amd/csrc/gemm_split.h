@@ -1,0 +1,391 @@
+// fp32 products on the bf16 matrix cores, for the large ones: a float32 is the
+// exact sum of three bf16 values (24 mantissa bits in three rounded pieces of 8,
+// x = p0 + p1 + p2), so a product of two is nine bf16 products, each exact in
+// float32.  The three smallest (p1 q2, p2 q1, p2 q2, together below 2^-25 of
+// the product) are left out, the other six go to v_mfma_f32_32x32x16_bf16,
+// smallest first, into one float32 accumulator: six matrix instructions of 32
+// clocks per 32x32x16 block where the fp32 ones (32x32x2) take eight of 64.
+// Included by gemm_f32.hip, whose GemmArgs and tile orders it shares.
+//
+// Error against float64 (2-norm, MI355X, normal values; this / fp32 MFMA): m =
+// 32768, n = 768, k = 256: 2.4e-7 / 2.9e-7; n = 256, k = 768: 4.2e-7 / 5.0e-7;
+// k = 2304: 7.5e-7 / 8.6e-7: smaller at every size, since one instruction sums
+// sixteen products before it rounds.  A second accumulator for the five small
+// products brings 9e-8 at k = 256 but costs the third workgroup per CU (94 vs
+// 83 us), and is not used.
+//
+// What bounds it: the matrix cores and LDS about alike (a 16-deep stage of a
+// workgroup is 24 MFMAs per wavefront and 72 KB of LDS traffic).  128x128 tiles
+// of four wavefronts, 64x64 each; the operands are loaded as float32 two stages
+// ahead in registers, split there and written to LDS as three planes (48 KB for
+// two stages: three workgroups per CU).  Measured against the fp32
+// tiles they replace (us): 32768 x 768, k = 256: 113 -> 80; 8192 x 2304, k = 768:
+// 237 -> 166; 16384 x 1536, k = 512: 211 -> 141; the weight-gradient pair 768 x
+// (256 + 256), k = 32768: 229 -> 159, k = 262144: 1725 -> 1186.
+//
+// Non-finite values: the pieces of an infinity are not finite sums, so an output
+// that comes out infinite or NaN is computed again as a plain float32 dot
+// product by the lane that stored it (split_redo); finite results are never
+// touched.  A piece, or a product of two, below 2^-126 counts as zero: what
+// underflows is 2^-17 of a value, so operands or products below some 1e-33 keep
+// fewer bits.
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+
+constexpr int kSplitTile = 128;                  // tile edge
+constexpr int kPlane = kSplitTile * 8;           // dwords of a plane: 128 rows x 16 k of bf16
+constexpr int kSplitStage = 2 * 3 * kPlane;      // dwords of a stage
+
+// The three pieces of a and b, packed in pairs (a low).
+__device__ __forceinline__ void split3(float a, float b, unsigned (&p)[3]) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const bf16x2 v = {(__bf16)a, (__bf16)b};
+        p[c] = __builtin_bit_cast(unsigned, v);
+        if (c < 2) {
+            a -= __uint_as_float(p[c] << 16);
+            b -= __uint_as_float(p[c] & 0xffff0000u);
+        }
+    }
+}
+
+// LDS planes of an operand's stage.  Row-major: [row][16 k] (32 bytes a row;
+// thread x of a pass holds k 4 (x % 4) of row x / 4).  k-major: [k pair][row] of
+// dwords (thread: rows 4 (t % 32) .. + 3 at k 2 (t / 32) and the next).  Every
+// access of either is free of bank conflicts.
+template <int KMAJOR>
+__device__ __forceinline__ void split_store(unsigned* lds, int tid, const float4 (&v)[2]) {
+    if constexpr (KMAJOR == 0) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            unsigned p[3], q[3];
+            split3(v[j].x, v[j].y, p);
+            split3(v[j].z, v[j].w, q);
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                *reinterpret_cast<uintx2*>(lds + c * kPlane + (tid + NT * j) * 2) = uintx2{p[c], q[c]};
+        }
+    } else {
+        unsigned p[4][3];
+        split3(v[0].x, v[1].x, p[0]);
+        split3(v[0].y, v[1].y, p[1]);
+        split3(v[0].z, v[1].z, p[2]);
+        split3(v[0].w, v[1].w, p[3]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            *reinterpret_cast<uintx4*>(lds + c * kPlane + (tid / 32) * kSplitTile + 4 * (tid % 32)) =
+                uintx4{p[0][c], p[1][c], p[2][c], p[3][c]};
+    }
+}
+
+// A wavefront's fragments, block x and piece c: lane 32 h + i holds k 8 h .. + 7
+// of tile row row0 + 32 x + i (row-major) or row0 + 2 i + x (k-major).
+template <int KMAJOR>
+__device__ __forceinline__ void split_frag(const unsigned* lds, int row0, int i, int h, bf16x8 (&f)[2][3]) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        if constexpr (KMAJOR == 0) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+                f[x][c] = *reinterpret_cast<const bf16x8*>(lds + c * kPlane + (row0 + 32 * x + i) * 8 + 4 * h);
+        } else {
+            uintx4 a, b;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uintx2 u =
+                    *reinterpret_cast<const uintx2*>(lds + c * kPlane + (4 * h + q) * kSplitTile + row0 + 2 * i);
+                a[q] = u[0];
+                b[q] = u[1];
+            }
+            f[0][c] = __builtin_bit_cast(bf16x8, a);
+            f[1][c] = __builtin_bit_cast(bf16x8, b);
+        }
+    }
+}
+
+// The loads of one operand (both operands vec_ok).  Rows past the operand read
+// its last rows, k past the range its last k (split_tile zeroes those).
+template <int KMAJOR>
+struct SplitLoader {
+    const char* base;
+    size_t stage_bytes;
+    unsigned kunit, row[2], kk[2];
+
+    static __device__ __forceinline__ int k_of(int tid, int j) {
+        return KMAJOR ? 2 * (tid / 32) + j : 4 * (tid % 4);
+    }
+    __device__ __forceinline__ SplitLoader(const GemmOperand& op, int rows, int r0, int kbeg, int, int tid) {
+        const size_t ld = (size_t)op.ld;
+        base = reinterpret_cast<const char*>(op.ptr + (KMAJOR ? (size_t)kbeg * ld + r0 : (size_t)r0 * ld + kbeg));
+        stage_bytes = (size_t)16 * (KMAJOR ? 4 * ld : 4);
+        kunit = KMAJOR ? 4u * (unsigned)op.ld : 4u;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            row[j] = KMAJOR ? 4u * (unsigned)min(4 * (tid % 32), rows - r0 - 4)
+                            : 4u * (unsigned)op.ld * (unsigned)min((tid + NT * j) / 4, rows - r0 - 1);
+            kk[j] = (unsigned)k_of(tid, j) * kunit;
+        }
+    }
+    __device__ __forceinline__ void load(int kb, int nkb, int klen, float4 (&v)[2]) const {
+        const int st = min(kb, nkb - 1);
+        const char* p = base + (size_t)st * stage_bytes;
+        const unsigned lim = (unsigned)(klen - 16 * st - (KMAJOR ? 1 : 4)) * kunit;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) v[j] = *reinterpret_cast<const float4*>(p + (row[j] + min(kk[j], lim)));
+    }
+};
+
+// The k-major [h0 ; y[:, :-1]] operand (ShiftLoader in gemm_small.h): stages in
+// order, k past the range read row 0 of shift_first.
+struct SplitShiftLoader {
+    const float* ptr;
+    const float* first;
+    size_t ld;
+    int T, left, row, t, b, k;  // (t, b, k: of the first of the thread's two k)
+
+    __device__ __forceinline__ SplitShiftLoader(const GemmOperand& op, int rows, int r0, int kbeg, int klen, int tid)
+        : ptr(op.ptr), first(op.shift_first), ld((size_t)op.ld), T(op.shift_T), left(klen) {
+        row = min(r0 + 4 * (tid % 32), rows - 4);
+        k = kbeg + SplitLoader<1>::k_of(tid, 0);
+        b = k / T;
+        t = k - b * T;
+    }
+    __device__ __forceinline__ void load(int, int, int, float4 (&v)[2]) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const bool in = SplitLoader<1>::k_of((int)threadIdx.x, j) < left;
+            const bool wrap = t + j >= T;  // j = 1: the next sequence's first step
+            const bool start = !in || wrap || t + j == 0;
+            const float* src = start ? first : ptr;
+            const size_t line = !in ? 0 : start ? (size_t)(b + (wrap ? 1 : 0)) : (size_t)(k + j - 1);
+            v[j] = *reinterpret_cast<const float4*>(src + line * ld + row);
+        }
+        k += 16;
+        t += 16;
+        if (t >= T) {
+            const int q = t / T;
+            b += q;
+            t -= q * T;
+        }
+        left -= 16;
+    }
+};
+
+// An output as a plain float32 dot product over k in [kbeg, kbeg + klen).
+template <int AK, int BKM, bool SHIFT>
+__device__ __forceinline__ float split_dot(const GemmArgs& p, int m, int n, int kbeg, int klen) {
+    float s = 0.f;
+#pragma unroll 1
+    for (int k = kbeg; k < kbeg + klen; ++k)
+        s = fmaf(*elem_ptr<AK, false, false>(p.a, m, k), *elem_ptr<BKM, SHIFT, false>(p.b, n, k), s);
+    return s;
+}
+
+// One 128x128 tile (bx, by); SPLIT: the partial products of k slice bz, with the
+// column sums of A in the first column of tiles (as small_tile).
+template <int AK, int BKM, bool SPLIT, bool SHIFT>
+__device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, int bz, unsigned* smem) {
+    static_assert(!SPLIT || (AK == 1 && BKM == 1), "split-K products take k-major operands");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int i = lane & 31, h = lane >> 5;
+    const int m0 = bx * kSplitTile, n0 = by * kSplitTile;
+    const int kbeg = SPLIT ? bz * p.kchunk : 0;
+    const int klen = SPLIT ? max(0, min(p.k - kbeg, p.kchunk)) : p.k;
+    const int nkb = (klen + 15) / 16;
+    const bool colsum = SPLIT && p.want_colsum && by == 0;
+    float4 cs = make_float4(0.f, 0.f, 0.f, 0.f);
+
+    using LA = SplitLoader<AK>;
+    using LB = std::conditional_t<SHIFT, SplitShiftLoader, SplitLoader<BKM>>;
+    const LA la(p.a, p.m, m0, kbeg, klen, tid);
+    LB lb(p.b, p.n, n0, kbeg, klen, tid);
+    float4 ra[2][2], rb[2][2];
+    floatx16 acc[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[x][y][r] = 0.f;
+    auto zero_past = [&](auto kmajor, int rem, float4 (&v)[2]) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const bool in = SplitLoader<decltype(kmajor)::value>::k_of(tid, j) < rem;
+            v[j] = make_float4(in ? v[j].x : 0.f, in ? v[j].y : 0.f, in ? v[j].z : 0.f, in ? v[j].w : 0.f);
+        }
+    };
+    auto stage = [&](int kb, auto st) {
+        constexpr int ST = decltype(st)::value;
+        unsigned* as = smem + ST * kSplitStage;
+        unsigned* bs = as + 3 * kPlane;
+        if (klen - 16 * kb < 16) {  // the last, shorter stage
+            zero_past(std::integral_constant<int, AK>{}, klen - 16 * kb, ra[ST]);
+            zero_past(std::integral_constant<int, BKM>{}, klen - 16 * kb, rb[ST]);
+        }
+        if constexpr (SPLIT) {
+            if (colsum) {
+                cs.x += ra[ST][0].x + ra[ST][1].x;
+                cs.y += ra[ST][0].y + ra[ST][1].y;
+                cs.z += ra[ST][0].z + ra[ST][1].z;
+                cs.w += ra[ST][0].w + ra[ST][1].w;
+            }
+        }
+        split_store<AK>(as, tid, ra[ST]);
+        split_store<BKM>(bs, tid, rb[ST]);
+        la.load(kb + 2, nkb, klen, ra[ST]);
+        lb.load(kb + 2, nkb, klen, rb[ST]);
+        __syncthreads();
+        bf16x8 fa[2][3], fb[2][3];
+        split_frag<AK>(as, 64 * wm, i, h, fa);
+        split_frag<BKM>(bs, 64 * wn, i, h, fb);
+        // four independent blocks between two products of one
+        auto product = [&](int pa, int pb) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y)
+                    acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[x][pa], fb[y][pb], acc[x][y], 0, 0, 0);
+        };
+        product(2, 0);
+        product(0, 2);
+        product(1, 1);
+        product(1, 0);
+        product(0, 1);
+        product(0, 0);
+    };
+    if (nkb > 0) {
+        la.load(0, nkb, klen, ra[0]);
+        lb.load(0, nkb, klen, rb[0]);
+        la.load(1, nkb, klen, ra[1]);
+        lb.load(1, nkb, klen, rb[1]);
+        int kb = 0;
+        for (; kb + 1 < nkb; kb += 2) {
+            stage(kb, std::integral_constant<int, 0>{});
+            stage(kb + 1, std::integral_constant<int, 1>{});
+        }
+        if (kb < nkb) stage(kb, std::integral_constant<int, 0>{});
+    }
+
+    // acc[x][y][r] is C(row(x, r), col(y)): the row of register r in a block is 8
+    // (r / 4) + 4 h + r % 4, its column i
+    const bool direct = !SPLIT || p.c != nullptr;  // (SPLIT: one slice, rows rotated)
+    auto row_of = [&](int x, int r) {
+        const int lr = 8 * (r / 4) + 4 * h + r % 4;
+        return m0 + 64 * wm + (AK ? 2 * lr + x : 32 * x + lr);
+    };
+    auto col_of = [&](int y) { return n0 + 64 * wn + (BKM ? 2 * i + y : 32 * y + i); };
+    auto dst_of = [&](int m) -> float* {
+        if constexpr (SPLIT) {
+            if (!direct) return p.partial + ((size_t)(p.z_off + bz) * p.m + m) * p.n;
+            return p.c + (size_t)(m >= p.rot ? m - p.rot : m - p.rot + p.m) * p.ldc;
+        } else {
+            return p.c + (size_t)m * p.ldc;
+        }
+    };
+    float bias[2] = {0.f, 0.f};
+    if (!SPLIT && p.bias) {
+#pragma unroll
+        for (int y = 0; y < 2; ++y) bias[y] = p.bias[min(col_of(y), p.n - 1)];
+    }
+    bool odd = false;  // an output that is not finite
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = row_of(x, r);
+            const float v[2] = {acc[x][0][r] + bias[0], acc[x][1][r] + bias[1]};
+            odd = odd || !__builtin_isfinite(v[0]) || !__builtin_isfinite(v[1]);
+            if (m >= p.m) continue;
+            float* dst = dst_of(m);
+            typedef float floatx2 __attribute__((ext_vector_type(2)));
+            if (BKM && p.c_vec && col_of(1) < p.n) {
+                const floatx2 vv = {v[0], v[1]};
+                if (SPLIT)
+                    *reinterpret_cast<floatx2*>(dst + col_of(0)) = vv;
+                else
+                    __builtin_nontemporal_store(vv, reinterpret_cast<floatx2*>(dst + col_of(0)));
+            } else {
+#pragma unroll
+                for (int y = 0; y < 2; ++y) {
+                    if (col_of(y) >= p.n) continue;
+                    if (SPLIT)
+                        dst[col_of(y)] = v[y];
+                    else
+                        __builtin_nontemporal_store(v[y], dst + col_of(y));
+                }
+            }
+        }
+    if (__builtin_expect(__any(odd), 0)) {
+        // the lane reads back what it stored (past the L1) and replaces what is
+        // not finite
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll 1
+        for (int e = 0; e < 64; ++e) {
+            const int m = row_of(e >> 5, (e >> 1) & 15), n = col_of(e & 1);
+            if (m >= p.m || n >= p.n) continue;
+            float* at = dst_of(m) + n;
+            const float old = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!__builtin_isfinite(old))
+                *at = split_dot<AK, BKM, SHIFT>(p, m, n, kbeg, klen) + (!SPLIT && p.bias ? p.bias[n] : 0.f);
+        }
+    }
+    if constexpr (SPLIT) {
+        if (colsum) {
+            // rows 4 (tid % 32) .. + 3 from the eight threads that share them
+            __syncthreads();
+            float* red = reinterpret_cast<float*>(smem);  // [8][128]
+            *reinterpret_cast<float4*>(red + (tid / 32) * kSplitTile + 4 * (tid % 32)) = cs;
+            __syncthreads();
+            if (tid < kSplitTile && m0 + tid < p.m) {
+                float s = 0.f;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) s += red[q * kSplitTile + tid];
+                const int m = m0 + tid;
+                if (direct)
+                    p.colsum[m >= p.rot ? m - p.rot : m - p.rot + p.m] = s;
+                else
+                    (p.partial + (size_t)p.ksplit_total * p.m * p.n)[(size_t)(p.z_off + bz) * p.m + m] = s;
+            }
+        }
+    }
+}
+
+template <int BKM>
+__global__ __launch_bounds__(NT, 3) void gemm_split_kernel(GemmArgs p) {
+    __shared__ __attribute__((aligned(16))) unsigned smem[2 * kSplitStage];
+    for (size_t i = (size_t)blockIdx.x * NT + threadIdx.x; i < p.zero_words; i += (size_t)gridDim.x * NT) p.zero[i] = 0ull;
+    int bx, by;
+    direct_coords(p, blockIdx.x, bx, by);
+    split_tile<0, BKM, false, false>(p, bx, by, 0, smem);
+}
+
+template <int BKM>
+__global__ __launch_bounds__(NT, 3) void gemm_split_reduce_kernel(GemmArgs p, ReduceJob j0, ReduceJob j1) {
+    __shared__ __attribute__((aligned(16))) unsigned smem[2 * kSplitStage];
+    if ((int)blockIdx.x >= p.tiles) {
+        reduce_range(j0, j1, (int)blockIdx.x - p.tiles, (int)gridDim.x - p.tiles);
+        return;
+    }
+    int bx, by;
+    direct_coords(p, blockIdx.x, bx, by);
+    split_tile<0, BKM, false, false>(p, bx, by, 0, smem);
+}
+
+// The weight-gradient pair (the first product with the row remap).
+__global__ __launch_bounds__(NT, 3) void gemm_split_pair_kernel(GemmArgs p0, GemmArgs p1) {
+    __shared__ __attribute__((aligned(16))) unsigned smem[2 * kSplitStage];
+    const int blocks0 = p0.tiles * p0.ksplit;
+    int bx, by, bz;
+    if ((int)blockIdx.x < blocks0) {
+        split_coords(p0, blockIdx.x, bx, by, bz);
+        split_tile<1, 1, true, true>(p0, bx, by, bz, smem);
+    } else {
+        split_coords(p1, blockIdx.x - blocks0, bx, by, bz);
+        split_tile<1, 1, true, false>(p1, bx, by, bz, smem);
+    }
+}

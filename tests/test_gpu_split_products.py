@@ -1,0 +1,105 @@
+"""The large fp32 products on the bf16 matrix cores (three bf16 pieces per
+value): error against float64 at the edges of their tiles and over magnitudes,
+and infinities, NaN and overflow as a float32 product has them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# m, n, k (aligned rows; 256 or more 128x128 tiles, so that this form is taken):
+# partial tiles along m and n, k of a part of a stage, one, two and many
+SHAPES = [(32700, 124, 4), (32768, 128, 16), (32641, 132, 20), (16400, 252, 36), (8300, 512, 256), (16384, 256, 772)]
+
+
+def _product(gpu, hip_lib, a, b, b_kmajor, bias=None):
+    from rnn_kernel_amd import _lib
+
+    m, k = a.shape
+    n = b.shape[1] if b_kmajor else b.shape[0]
+    c = torch.full((m + 1, n), float("nan"), device=gpu)
+    rc = hip_lib.rka_gemm_f32(m, n, k, a.data_ptr(), k, 0, b.data_ptr(), b.shape[1], b_kmajor,
+                              None if bias is None else bias.data_ptr(), c.data_ptr(), n,
+                              torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "rka_gemm_f32")
+    torch.cuda.synchronize()
+    assert torch.isnan(c[m]).all()  # nothing stored past the last row
+    return c[:m]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("b_kmajor", [0, 1])
+@pytest.mark.parametrize("scale", [1.0, 1e-30, 1e15])
+def test_split_product_error(gpu, hip_lib, m, n, k, b_kmajor, scale):
+    print(f"split m={m} n={n} k={k} b_kmajor={b_kmajor} scale={scale}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    a = scale * torch.randn(m, k, generator=g, device=gpu)
+    b = torch.randn((k, n) if b_kmajor else (n, k), generator=g, device=gpu)
+    b *= torch.exp(6 * torch.randn(b.shape, generator=g, device=gpu))  # 10 decades within a sum
+    bias = scale * torch.randn(n, generator=g, device=gpu)
+    c = _product(gpu, hip_lib, a, b, b_kmajor, bias)
+    bd = b.double() if b_kmajor else b.double().t().contiguous()
+    ref = a.double() @ bd + bias.double()
+    mag = a.double().abs() @ bd.abs() + bias.double().abs()
+    # six float32 roundings per 16-deep stage and the left-out 2^-25; a piece or a
+    # product of two below the normal range (2^-126) may count as zero
+    stages = (k + 15) // 16
+    tiny = 2.0 ** -126 * (6 * k + a.double().abs().sum(1, keepdim=True) + bd.abs().sum(0))
+    assert bool(((c.double() - ref).abs() <= (6 * stages + 4) * 2.0 ** -24 * mag + tiny).all())
+
+
+@pytest.mark.parametrize("b_kmajor", [0, 1])
+def test_split_product_non_finite(gpu, hip_lib, b_kmajor):
+    """Rows with an infinity, a NaN, values that round past the largest bf16 and
+    a sum that overflows equal the float32 results; all other rows equal the
+    same product without them, bit for bit."""
+    m, n, k = 32768, 128, 64
+    g = torch.Generator(device=gpu).manual_seed(3)
+    a = torch.randn(m, k, generator=g, device=gpu)
+    b = torch.randn((k, n) if b_kmajor else (n, k), generator=g, device=gpu)
+    plain = _product(gpu, hip_lib, a, b, b_kmajor)
+    bn = b.t() if b_kmajor else b  # [n, k]
+    inf = float("inf")
+    a2 = a.clone()
+    a2[5, 7] = inf
+    a2[130, 0] = -inf
+    a2[131, 3], a2[131, 9] = inf, -inf
+    a2[200, 63] = float("nan")
+    a2[300] = 0.0
+    a2[300, 2] = 3.4e38  # finite, but its first bf16 piece is not
+    a2[400] = 3e38
+    c = _product(gpu, hip_lib, a2, b, b_kmajor)
+    touched = torch.zeros(m, dtype=torch.bool, device=gpu)
+    touched[[5, 130, 131, 200, 300, 400]] = True
+    assert torch.equal(c[~touched], plain[~touched])
+    assert torch.equal(c[5], inf * bn[:, 7].sign()) and torch.equal(c[130], -inf * bn[:, 0].sign())
+    want = torch.where(bn[:, 3].sign() == bn[:, 9].sign(), torch.full((n,), float("nan"), device=gpu), inf * bn[:, 3].sign())
+    assert torch.equal(torch.isnan(c[131]), torch.isnan(want)) and torch.equal(c[131][~torch.isnan(want)], want[~torch.isnan(want)])
+    assert torch.isnan(c[200]).all()
+    ref = a2[300, 2].double() * bn[:, 2].double()
+    fits = ref.abs() < 3.4e38
+    assert torch.allclose(c[300][fits].double(), ref[fits], rtol=1e-6) and torch.isinf(c[300][ref.abs() > 3.5e38]).all()
+    ref = (a2[400].double() @ bn.double().t().contiguous())
+    big = ref.abs() > 1e39
+    assert bool((~torch.isfinite(c[400][big])).all())
+
+
+def test_split_weight_gradients_non_finite(gpu):
+    """An infinite upstream gradient in one unit reaches that unit's weight
+    gradient rows only."""
+    from rnn_kernel_amd import GRUFunction
+
+    B, T, H = 64, 512, 256
+    g = torch.Generator(device=gpu).manual_seed(9)
+    w = [((torch.rand(*s, generator=g, device=gpu) * 2 - 1) / 16).requires_grad_(True)
+         for s in ((3 * H, H), (3 * H, H), (3 * H,), (3 * H,))]
+    x = torch.randn(B, T, H, generator=g, device=gpu)
+    dy = torch.randn(B, T, H, generator=g, device=gpu)
+    y, _ = GRUFunction.apply(x, torch.zeros(B, H, device=gpu), *w)
+    dy[3, 0, 17] = float("inf")  # the first step: its gradient goes no further back
+    y.backward(dy)
+    bad = torch.zeros(3 * H, dtype=torch.bool, device=gpu)
+    bad[[17, H + 17, 2 * H + 17]] = True
+    for p in w:
+        rows = torch.isfinite(p.grad.reshape(3 * H, -1)).all(dim=1)
+        assert bool(rows[~bad].all())
+        assert not bool(rows[bad].any())
