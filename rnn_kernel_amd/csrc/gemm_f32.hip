@@ -1095,6 +1095,9 @@ int launch_gemm(GemmArgs args, int ksplit, bool av, bool bv, hipStream_t stream)
 
 std::atomic<int> g_gemm_tiles{RKA_GEMM_TILES_AUTO};
 
+// Extents from which gemm_split.h's loads stay inside the operands.
+bool split_takes(int m, int n, int k) { return m >= 4 && n >= 4 && k >= 4; }
+
 // Tiles a direct product runs in.
 enum DirectTile { TILE_128, TILE_SPLIT, TILE_128x64, TILE_64, TILE_32 };
 using Tile128x64 = SmallTile<128, 64, 64, 32, 16>;
@@ -1104,12 +1107,12 @@ using Tile32 = SmallTile<32, 32, 32, 32, 64>;
 // The tile with the least work on the busiest CU: tiles per CU, rounded up,
 // times the tile's area, times the measured cost of a unit of area (large
 // products that divide evenly: the 128x128 ring 1, 128x128 split into bf16 pieces
-// 0.70, 128x64 1.02, 64x64 1.07, 32x32 1.30; the ring's register path for operands that are not 16-byte
-// aligned 1.45).  Rounding up is what decides: 8192 x 2304 (k = 768) is 4.5
+// 0.70, 128x64 1.02, 64x64 1.07, 32x32 1.30; operands that are not 16-byte aligned:
+// the ring's register path 1.45, split 0.75).  Rounding up is what decides: 8192 x 2304 (k = 768) is 4.5
 // 128x128 tiles per CU, 8192 x 128 a quarter.  Measured on MI355X (us, 128 /
 // 128x64 / 64 / 32): 32768 x 768, k = 256: 113 / 115 / 118 / 154 (split 80); 8192 x
 // 2304, k = 768: 271 / 246 / 257 / 319 (split 166); 8192 x 128, k = 768: 59 / 36 / 23 / 20;
-// 32768 x 129, k = 387 (not aligned): 77 / 53 / 55 / 73; 64 x 768, k = 256:
+// 32768 x 129, k = 387 (not aligned): 77 / 53 / 55 / 73 (split 46); 64 x 768, k = 256:
 // 22 / 13 / 9.0 / 4.3; 1 x 256, k = 768: 55 / 35 / 21 / 8.2.
 DirectTile direct_tile(const GemmArgs& g) {
     if (g.a.kmajor) return TILE_128;
@@ -1126,7 +1129,7 @@ DirectTile direct_tile(const GemmArgs& g) {
             least = c;
         }
     };
-    if (vec) consider(TILE_SPLIT, cost(128, 128, 0.70));
+    if (split_takes(g.m, g.n, g.k)) consider(TILE_SPLIT, cost(128, 128, vec ? 0.70 : 0.75));
     if (g_gemm_tiles.load(std::memory_order_relaxed) == RKA_GEMM_TILES_AUTO) {
         consider(TILE_128x64, cost(128, 64, 1.02));
         consider(TILE_64, cost(64, 64, 1.07));
@@ -1154,7 +1157,7 @@ int launch_small_t(GemmArgs args, const ReduceJob* j0, const ReduceJob* j1, long
     return 0;
 }
 
-template <int BKM>
+template <int BKM, bool UA>
 int launch_split(GemmArgs args, const ReduceJob* j0, const ReduceJob* j1, long reducers, hipStream_t stream) {
     args.tiles_m = (args.m + kSplitTile - 1) / kSplitTile;
     const long long tiles = (long long)args.tiles_m * ((args.n + kSplitTile - 1) / kSplitTile);
@@ -1162,9 +1165,9 @@ int launch_split(GemmArgs args, const ReduceJob* j0, const ReduceJob* j1, long r
     args.tiles = (int)tiles;
     const dim3 grid((unsigned)(tiles + reducers));
     if (j0)
-        hipLaunchKernelGGL((gemm_split_reduce_kernel<BKM>), grid, dim3(NT), 0, stream, args, *j0, *j1);
+        hipLaunchKernelGGL((gemm_split_reduce_kernel<BKM, UA>), grid, dim3(NT), 0, stream, args, *j0, *j1);
     else
-        hipLaunchKernelGGL((gemm_split_kernel<BKM>), grid, dim3(NT), 0, stream, args);
+        hipLaunchKernelGGL((gemm_split_kernel<BKM, UA>), grid, dim3(NT), 0, stream, args);
     RKA_RETURN_IF_HIP(hipGetLastError());
     return 0;
 }
@@ -1180,7 +1183,11 @@ int launch_small(DirectTile tile, const GemmArgs& args, const ReduceJob* j0, con
         return launch_small_t<0, B, S, false>(args, j0, j1, reducers, stream);
     };
     auto run = [&](auto bk) {
-        if (tile == TILE_SPLIT) return launch_split<decltype(bk)::value>(args, j0, j1, reducers, stream);
+        if (tile == TILE_SPLIT) {
+            constexpr int B = decltype(bk)::value;
+            return args.a_vec && args.b_vec ? launch_split<B, false>(args, j0, j1, reducers, stream)
+                                            : launch_split<B, true>(args, j0, j1, reducers, stream);
+        }
         if (tile == TILE_32) return with(bk, Tile32{});
         if (tile == TILE_64) return with(bk, Tile64{});
         return with(bk, Tile128x64{});
@@ -1254,11 +1261,11 @@ struct PairPlan {
 // where up to four workgroups share a CU and a part of one counts whole.  A
 // stage of a 64x64 tile was measured at 0.75, 0.5, 0.38 and 0.35 us for one,
 // two, three and four or more workgroups per CU (its MFMAs alone take 0.21); a
-// 128x64 tile takes 1.85 times that and a split 128x128 one (operands of aligned
-// float4 rows) 2.1 times.  Measured on MI355X (pair, us; 128x128
-// ring, now): m = 576, n = 192 + 192, k = 32768: 218, 158; 192, 64 + 64, 32768:
-// 50, 25; 384, 128 + 128, 32768: 84, 75; 387, 129 + 129, 32768: 163, 151; 384, 128 +
-// 64, 51200: 120, 86; 768, 256 + 128, 8192: 61, 58.
+// 128x64 tile takes 1.85 times that and a split 128x128 one 2.1 times.  Measured
+// on MI355X (pair, us; 128x128 ring, the fp32 tile chosen): m = 576, n = 192 + 192,
+// k = 32768: 218, 158; 192, 64 + 64, 32768: 50, 25; 384, 128 + 128, 32768: 84, 75;
+// 387, 129 + 129, 32768: 163, 151 (split 115); 384, 128 + 64, 51200: 120, 86; 768,
+// 256 + 128, 8192: 61, 58.
 PairPlan make_pair_plan(int m, int n0, int n1, int k) {
     PairPlan best{TILE_128x64, 1, 1};
     constexpr int kMaxSlices = 256;
@@ -1267,7 +1274,7 @@ PairPlan make_pair_plan(int m, int n0, int n1, int k) {
     const int least = std::min(most, (k + 4095) / 4096);
     double least_cost = 1e30;
     for (const DirectTile tile : {TILE_64, TILE_128x64, TILE_SPLIT}) {
-        if (tile == TILE_SPLIT && (n0 % 4 || n1 % 4)) continue;
+        if (tile == TILE_SPLIT && !(split_takes(m, n0, k) && split_takes(m, n1, k))) continue;
         const int tm = tile == TILE_64 ? 64 : 128, tn = tile == TILE_SPLIT ? 128 : 64;
         const double unit = tile == TILE_64 ? 1.0 : tile == TILE_128x64 ? 1.85 : 2.1;
         const double tiles = (double)((m + tm - 1) / tm) * ((n0 + tn - 1) / tn + (n1 + tn - 1) / tn);
@@ -1420,11 +1427,15 @@ int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, hi
     if (seg) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: pair products take whole operands");
     if (p0.b.shift_T > 0) {
         const bool any = g_gemm_tiles.load(std::memory_order_relaxed) == RKA_GEMM_TILES_AUTO;
-        const bool vec = a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec;
         const DirectTile tile = plan_pair(p0.m, p0.n, p1.n, p0.k).tile;
-        if (tile == TILE_SPLIT && vec) return launch_pair_tiles(p0, p1, a0, a1, kSplitTile, kSplitTile, [&](dim3 g, const GemmArgs& x, const GemmArgs& y) {
-            hipLaunchKernelGGL(gemm_split_pair_kernel, g, dim3(NT), 0, stream, x, y);
-        });
+        if (tile == TILE_SPLIT) {
+            const bool vec = a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec;
+            auto kern = vec ? gemm_split_pair_kernel<false> : gemm_split_pair_kernel<true>;
+            return launch_pair_tiles(p0, p1, a0, a1, kSplitTile, kSplitTile,
+                                     [&](dim3 grid, const GemmArgs& x, const GemmArgs& y) {
+                                         hipLaunchKernelGGL(kern, grid, dim3(NT), 0, stream, x, y);
+                                     });
+        }
         if (any && tile == TILE_64) return launch_small_pair<Tile64>(p0, p1, a0, a1, stream);
         if (any) return launch_small_pair<Tile128x64>(p0, p1, a0, a1, stream);
     }

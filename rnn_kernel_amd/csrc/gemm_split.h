@@ -23,6 +23,12 @@
 // 237 -> 166; 16384 x 1536, k = 512: 211 -> 141; the weight-gradient pair 768 x
 // (256 + 256), k = 32768: 229 -> 159, k = 262144: 1725 -> 1186.
 //
+// Operands without aligned float4 rows (odd sizes; UA, any row length from 4) are
+// loaded in the same float4 from 4-byte-aligned addresses.  Against the fp32
+// register-staged tiles they replace (us): 32768 x 387, k = 129: 60 -> 40; 32768 x
+// 129, k = 387: 58 -> 46; 19200 x 1533, k = 511: 308 -> 190; the pair 387 x (129 +
+// 129), k = 32768: 155 -> 115; 993 x (331 + 331), k = 8192: 152 -> 83.
+//
 // Non-finite values: the pieces of an infinity are not finite sums, so an output
 // that comes out infinite or NaN is computed again as a plain float32 dot
 // product by the lane that stored it (split_redo); finite results are never
@@ -106,62 +112,103 @@ __device__ __forceinline__ void split_frag(const unsigned* lds, int row0, int i,
     }
 }
 
-// The loads of one operand (both operands vec_ok).  Rows past the operand read
-// its last rows, k past the range its last k (split_tile zeroes those).
-template <int KMAJOR>
+// Four floats from an address that is a multiple of 4 bytes (global_load_dwordx4
+// asks for no more).
+struct __attribute__((packed, aligned(4))) Float4U {
+    float x, y, z, w;
+};
+template <bool UA>
+__device__ __forceinline__ float4 split_load4(const char* p) {
+    if constexpr (UA) {
+        const Float4U v = *reinterpret_cast<const Float4U*>(p);
+        return make_float4(v.x, v.y, v.z, v.w);
+    } else {
+        return *reinterpret_cast<const float4*>(p);
+    }
+}
+// v moved down by sh elements (sh <= 3; what moves in from past v is not used).
+__device__ __forceinline__ float4 split_shift(const float4& v, int sh) {
+    // (loaded first: loads under the selects would be merged into one of a
+    // selected address, and v would live in scratch)
+    const float x = v.x, y = v.y, z = v.z, w = v.w;
+    return make_float4(sh == 0 ? x : sh == 1 ? y : sh == 2 ? z : w, sh == 0 ? y : sh == 1 ? z : w, sh == 0 ? z : w, w);
+}
+
+// The loads of one operand.  Rows past the operand read its last rows, k past
+// the range its last k (split_tile zeroes those).  UA: rows that are not aligned
+// float4, of any length from 4: a float4 that would cross the operand's last
+// row (k-major) or the end of the range (row-major) starts early enough to end
+// there, and its values are moved down by `rsh`, or kshift(), elements.
+template <int KMAJOR, bool UA>
 struct SplitLoader {
     const char* base;
     size_t stage_bytes;
-    unsigned kunit, row[2], kk[2];
+    unsigned kunit, row[2];  // (unsigned: one uniform base and 32-bit lane offsets)
+    int rsh;
 
     static __device__ __forceinline__ int k_of(int tid, int j) {
         return KMAJOR ? 2 * (tid / 32) + j : 4 * (tid % 4);
     }
     __device__ __forceinline__ SplitLoader(const GemmOperand& op, int rows, int r0, int kbeg, int, int tid) {
         const size_t ld = (size_t)op.ld;
-        base = reinterpret_cast<const char*>(op.ptr + (KMAJOR ? (size_t)kbeg * ld + r0 : (size_t)r0 * ld + kbeg));
+        const int back = UA && KMAJOR ? min(r0, 3) : 0;  // (rows >= 4: only a later tile has fewer than 4 rows)
+        base = reinterpret_cast<const char*>(op.ptr + (KMAJOR ? (size_t)kbeg * ld + (r0 - back) : (size_t)r0 * ld + kbeg));
         stage_bytes = (size_t)16 * (KMAJOR ? 4 * ld : 4);
         kunit = KMAJOR ? 4u * (unsigned)op.ld : 4u;
+        const int r = min(4 * (tid % 32), rows - r0 - 4);
+        rsh = UA && KMAJOR ? min(4 * (tid % 32) - r, 3) : 0;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            row[j] = KMAJOR ? 4u * (unsigned)min(4 * (tid % 32), rows - r0 - 4)
+        for (int j = 0; j < 2; ++j)
+            row[j] = KMAJOR ? 4u * (unsigned)(r + back)
                             : 4u * (unsigned)op.ld * (unsigned)min((tid + NT * j) / 4, rows - r0 - 1);
-            kk[j] = (unsigned)k_of(tid, j) * kunit;
-        }
     }
-    __device__ __forceinline__ void load(int kb, int nkb, int klen, float4 (&v)[2]) const {
+    // stage kb, or the last one again past it
+    __device__ __forceinline__ void load(int kb, int nkb, int klen, int tid, float4 (&v)[2]) const {
         const int st = min(kb, nkb - 1);
         const char* p = base + (size_t)st * stage_bytes;
-        const unsigned lim = (unsigned)(klen - 16 * st - (KMAJOR ? 1 : 4)) * kunit;
+        const int lim = klen - 16 * st - (KMAJOR ? 1 : 4);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) v[j] = *reinterpret_cast<const float4*>(p + (row[j] + min(kk[j], lim)));
+        for (int j = 0; j < 2; ++j) {
+            const int k = min(k_of(tid, j), lim);
+            if constexpr (UA && !KMAJOR)  // (k may be negative)
+                v[j] = split_load4<UA>(p - 16 + (row[j] + 4u * (unsigned)(k + 4)));
+            else
+                v[j] = split_load4<UA>(p + (row[j] + (unsigned)k * kunit));
+        }
+    }
+    // the last stage of rem < 16 values: what its float4 started early by
+    static __device__ __forceinline__ int kshift(int tid, int rem) {
+        return UA && !KMAJOR ? min(max(k_of(tid, 0) - (rem - 4), 0), 3) : 0;
     }
 };
 
 // The k-major [h0 ; y[:, :-1]] operand (ShiftLoader in gemm_small.h): stages in
 // order, k past the range read row 0 of shift_first.
+template <bool UA>
 struct SplitShiftLoader {
+    using Plain = SplitLoader<1, UA>;
     const float* ptr;
     const float* first;
     size_t ld;
-    int T, left, row, t, b, k;  // (t, b, k: of the first of the thread's two k)
+    int T, left, row, rsh, t, b, k;  // (t, b, k: of the first of the thread's two k)
 
     __device__ __forceinline__ SplitShiftLoader(const GemmOperand& op, int rows, int r0, int kbeg, int klen, int tid)
         : ptr(op.ptr), first(op.shift_first), ld((size_t)op.ld), T(op.shift_T), left(klen) {
         row = min(r0 + 4 * (tid % 32), rows - 4);
-        k = kbeg + SplitLoader<1>::k_of(tid, 0);
+        rsh = UA ? min(r0 + 4 * (tid % 32) - row, 3) : 0;
+        k = kbeg + Plain::k_of(tid, 0);
         b = k / T;
         t = k - b * T;
     }
-    __device__ __forceinline__ void load(int, int, int, float4 (&v)[2]) {
+    __device__ __forceinline__ void load(int, int, int, int tid, float4 (&v)[2]) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const bool in = SplitLoader<1>::k_of((int)threadIdx.x, j) < left;
+            const bool in = Plain::k_of(tid, j) < left;
             const bool wrap = t + j >= T;  // j = 1: the next sequence's first step
             const bool start = !in || wrap || t + j == 0;
             const float* src = start ? first : ptr;
             const size_t line = !in ? 0 : start ? (size_t)(b + (wrap ? 1 : 0)) : (size_t)(k + j - 1);
-            v[j] = *reinterpret_cast<const float4*>(src + line * ld + row);
+            v[j] = split_load4<UA>(reinterpret_cast<const char*>(src + line * ld + row));
         }
         k += 16;
         t += 16;
@@ -172,6 +219,7 @@ struct SplitShiftLoader {
         }
         left -= 16;
     }
+    static __device__ __forceinline__ int kshift(int, int) { return 0; }
 };
 
 // An output as a plain float32 dot product over k in [kbeg, kbeg + klen).
@@ -186,7 +234,7 @@ __device__ __forceinline__ float split_dot(const GemmArgs& p, int m, int n, int 
 
 // One 128x128 tile (bx, by); SPLIT: the partial products of k slice bz, with the
 // column sums of A in the first column of tiles (as small_tile).
-template <int AK, int BKM, bool SPLIT, bool SHIFT>
+template <int AK, int BKM, bool SPLIT, bool SHIFT, bool UA>
 __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, int bz, unsigned* smem) {
     static_assert(!SPLIT || (AK == 1 && BKM == 1), "split-K products take k-major operands");
     const int tid = threadIdx.x, lane = tid & 63;
@@ -200,8 +248,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
     const bool colsum = SPLIT && p.want_colsum && by == 0;
     float4 cs = make_float4(0.f, 0.f, 0.f, 0.f);
 
-    using LA = SplitLoader<AK>;
-    using LB = std::conditional_t<SHIFT, SplitShiftLoader, SplitLoader<BKM>>;
+    using LA = SplitLoader<AK, UA>;
+    using LB = std::conditional_t<SHIFT, SplitShiftLoader<UA>, SplitLoader<BKM, UA>>;
     const LA la(p.a, p.m, m0, kbeg, klen, tid);
     LB lb(p.b, p.n, n0, kbeg, klen, tid);
     float4 ra[2][2], rb[2][2];
@@ -212,20 +260,40 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
         for (int y = 0; y < 2; ++y)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[x][y][r] = 0.f;
-    auto zero_past = [&](auto kmajor, int rem, float4 (&v)[2]) {
+    // the last, shorter stage: zero past the range (UA, row-major: value by value)
+    auto zero_past = [&](auto kmajor, int rem, int sh, float4 (&v)[2]) {
+        constexpr int KM = decltype(kmajor)::value;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const bool in = SplitLoader<decltype(kmajor)::value>::k_of(tid, j) < rem;
-            v[j] = make_float4(in ? v[j].x : 0.f, in ? v[j].y : 0.f, in ? v[j].z : 0.f, in ? v[j].w : 0.f);
+            const int k = SplitLoader<KM, UA>::k_of(tid, j);
+            constexpr int s = UA && !KM ? 1 : 0;
+            if constexpr (s == 1) v[j] = split_shift(v[j], sh);
+            v[j] = make_float4(k < rem ? v[j].x : 0.f, k + s < rem ? v[j].y : 0.f, k + 2 * s < rem ? v[j].z : 0.f,
+                               k + 3 * s < rem ? v[j].w : 0.f);
         }
     };
+    // tiles whose last k-major float4 would cross the operand's last row
+    const bool edge_a = UA && AK && m0 + kSplitTile > p.m, edge_b = UA && BKM && n0 + kSplitTile > p.n;
     auto stage = [&](int kb, auto st) {
         constexpr int ST = decltype(st)::value;
         unsigned* as = smem + ST * kSplitStage;
         unsigned* bs = as + 3 * kPlane;
         if (klen - 16 * kb < 16) {  // the last, shorter stage
-            zero_past(std::integral_constant<int, AK>{}, klen - 16 * kb, ra[ST]);
-            zero_past(std::integral_constant<int, BKM>{}, klen - 16 * kb, rb[ST]);
+            const int rem = klen - 16 * kb;
+            zero_past(std::integral_constant<int, AK>{}, rem, LA::kshift(tid, rem), ra[ST]);
+            zero_past(std::integral_constant<int, BKM>{}, rem, LB::kshift(tid, rem), rb[ST]);
+        }
+        if constexpr (UA && AK) {
+            if (edge_a) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) ra[ST][j] = split_shift(ra[ST][j], la.rsh);
+            }
+        }
+        if constexpr (UA && BKM) {
+            if (edge_b) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) rb[ST][j] = split_shift(rb[ST][j], lb.rsh);
+            }
         }
         if constexpr (SPLIT) {
             if (colsum) {
@@ -237,8 +305,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
         }
         split_store<AK>(as, tid, ra[ST]);
         split_store<BKM>(bs, tid, rb[ST]);
-        la.load(kb + 2, nkb, klen, ra[ST]);
-        lb.load(kb + 2, nkb, klen, rb[ST]);
+        la.load(kb + 2, nkb, klen, tid, ra[ST]);
+        lb.load(kb + 2, nkb, klen, tid, rb[ST]);
         __syncthreads();
         bf16x8 fa[2][3], fb[2][3];
         split_frag<AK>(as, 64 * wm, i, h, fa);
@@ -259,10 +327,10 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
         product(0, 0);
     };
     if (nkb > 0) {
-        la.load(0, nkb, klen, ra[0]);
-        lb.load(0, nkb, klen, rb[0]);
-        la.load(1, nkb, klen, ra[1]);
-        lb.load(1, nkb, klen, rb[1]);
+        la.load(0, nkb, klen, tid, ra[0]);
+        lb.load(0, nkb, klen, tid, rb[0]);
+        la.load(1, nkb, klen, tid, ra[1]);
+        lb.load(1, nkb, klen, tid, rb[1]);
         int kb = 0;
         for (; kb + 1 < nkb; kb += 2) {
             stage(kb, std::integral_constant<int, 0>{});
@@ -355,16 +423,16 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
     }
 }
 
-template <int BKM>
+template <int BKM, bool UA>
 __global__ __launch_bounds__(NT, 3) void gemm_split_kernel(GemmArgs p) {
     __shared__ __attribute__((aligned(16))) unsigned smem[2 * kSplitStage];
     for (size_t i = (size_t)blockIdx.x * NT + threadIdx.x; i < p.zero_words; i += (size_t)gridDim.x * NT) p.zero[i] = 0ull;
     int bx, by;
     direct_coords(p, blockIdx.x, bx, by);
-    split_tile<0, BKM, false, false>(p, bx, by, 0, smem);
+    split_tile<0, BKM, false, false, UA>(p, bx, by, 0, smem);
 }
 
-template <int BKM>
+template <int BKM, bool UA>
 __global__ __launch_bounds__(NT, 3) void gemm_split_reduce_kernel(GemmArgs p, ReduceJob j0, ReduceJob j1) {
     __shared__ __attribute__((aligned(16))) unsigned smem[2 * kSplitStage];
     if ((int)blockIdx.x >= p.tiles) {
@@ -373,19 +441,20 @@ __global__ __launch_bounds__(NT, 3) void gemm_split_reduce_kernel(GemmArgs p, Re
     }
     int bx, by;
     direct_coords(p, blockIdx.x, bx, by);
-    split_tile<0, BKM, false, false>(p, bx, by, 0, smem);
+    split_tile<0, BKM, false, false, UA>(p, bx, by, 0, smem);
 }
 
 // The weight-gradient pair (the first product with the row remap).
+template <bool UA>
 __global__ __launch_bounds__(NT, 3) void gemm_split_pair_kernel(GemmArgs p0, GemmArgs p1) {
     __shared__ __attribute__((aligned(16))) unsigned smem[2 * kSplitStage];
     const int blocks0 = p0.tiles * p0.ksplit;
     int bx, by, bz;
     if ((int)blockIdx.x < blocks0) {
         split_coords(p0, blockIdx.x, bx, by, bz);
-        split_tile<1, 1, true, true>(p0, bx, by, bz, smem);
+        split_tile<1, 1, true, true, UA>(p0, bx, by, bz, smem);
     } else {
         split_coords(p1, blockIdx.x - blocks0, bx, by, bz);
-        split_tile<1, 1, true, false>(p1, bx, by, bz, smem);
+        split_tile<1, 1, true, false, UA>(p1, bx, by, bz, smem);
     }
 }

@@ -10,7 +10,8 @@ import torch
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 1, 1, 1), (2, 3, 5, 7), (127, 1, 16, 20), (128, 1, 12, 64), (9, 14, 33, 65), (5, 100, 100, 100),
-          (40, 25, 64, 128), (7, 300, 129, 129), (16, 520, 128, 256), (33, 331, 16, 64), (16, 2001, 256, 256), (61, 500, 132, 260)]
+          (40, 25, 64, 128), (7, 300, 129, 129), (16, 520, 128, 256), (33, 331, 16, 64), (16, 2001, 256, 256), (61, 500, 132, 260),
+          (64, 512, 129, 129), (61, 500, 131, 255), (16, 2001, 257, 513)]
 
 
 @pytest.mark.parametrize("B,T,I,H", SHAPES)

@@ -6,9 +6,12 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# m, n, k (aligned rows; 256 or more 128x128 tiles, so that this form is taken):
-# partial tiles along m and n, k of a part of a stage, one, two and many
-SHAPES = [(32700, 124, 4), (32768, 128, 16), (32641, 132, 20), (16400, 252, 36), (8300, 512, 256), (16384, 256, 772)]
+# m, n, k (enough 128x128 tiles that this form is taken): partial tiles along m and
+# n, k of a part of a stage, one, two and many; then the same without aligned
+# float4 rows, where loads that would cross an operand's end start earlier: a last
+# tile of one to three columns, last stages of one to three and more k
+SHAPES = [(32700, 124, 4), (32768, 128, 16), (32641, 132, 20), (16400, 252, 36), (8300, 512, 256), (16384, 256, 772),
+          (32701, 125, 5), (32641, 127, 17), (16385, 255, 34), (8300, 510, 129), (8200, 513, 387), (8257, 643, 63)]
 
 
 def _product(gpu, hip_lib, a, b, b_kmajor, bias=None):
