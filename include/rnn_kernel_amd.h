@@ -177,12 +177,11 @@ int rka_gru_recurrence_backward(const float* dy, const float* dhn,
                                 void* stream);
 
 /* GEMM tile families (for tuning and A/B tests; affects later calls on all
- * threads).  RKA_GEMM_TILES_AUTO: the weight-gradient pair of
- * rka_gru_backward runs in 192x256 tiles, one twelve-wavefront workgroup
- * per CU, when its tiles and k-slices divide evenly over the CUs (c2, c4);
- * every other product in 128x128 tiles.  RKA_GEMM_TILES_128: 128x128 tiles
- * everywhere.  The results are the same bit for bit (each output element
- * sums its k in the same order, over the same k-slices).  No counterpart in
+ * threads).  RKA_GEMM_TILES_AUTO: the tile of each product by a cost rule
+ * (32x32 to 128x64 where 128x128 tiles would fill the CUs unevenly).
+ * RKA_GEMM_TILES_128: 128x128 tiles everywhere.  Products that the rule gives
+ * 128x128 tiles are the same bit for bit in both modes; the others differ by
+ * float32 rounding (other k-slices and summation order).  No counterpart in
  * the reference (its products are cuBLAS calls,
  * src/rnn_kernel/a100/prod/gru.py:569-578). */
 #define RKA_GEMM_TILES_AUTO 0

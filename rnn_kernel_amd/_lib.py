@@ -176,8 +176,8 @@ def set_spin_limit(polls: int) -> None:
 
 
 def set_gemm_tiles(mode: int) -> None:
-    """GEMM tile families: 0 = automatic (large persistent tiles where they
-    divide evenly), 1 = 128x128 everywhere; see rka_set_gemm_tiles."""
+    """GEMM tile families: 0 = automatic (smaller tiles where 128x128
+    would fill the CUs unevenly), 1 = 128x128 everywhere; see rka_set_gemm_tiles."""
     check(load().rka_set_gemm_tiles(mode), "rka_set_gemm_tiles")
 
 

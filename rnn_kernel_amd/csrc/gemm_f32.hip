@@ -1,11 +1,16 @@
-// fp32 GEMMs of the GRU path on gfx950 matrix cores (v_mfma_f32_16x16x4_f32).
+// fp32 GEMMs of the GRU path on gfx950 matrix cores, in three forms chosen by
+// direct_tile and plan_pair (which say why the lines lie where they do):
+//   large products: 128x128 tiles, each value in three bf16 pieces (gemm_split.h);
+//   those that would fill the CUs unevenly: register-staged tiles of 32x32 to
+//   128x64 on v_mfma_f32_16x16x4_f32 (gemm_small.h);
+//   the rest: the 128x128 ring below.
 //
-// One kernel template serves the four products of a layer:
+// The products of a layer are
 //   input projection  Gx  = X W_ih^T + b_ih        (A row-major, B row-major)
 //   input gradient    dX  = G_i W_ih               (A row-major, B k-major)
 //   weight gradients  dW  = G^T [X | Hprev]        (A k-major,  B k-major)
-// C[m,n] = sum_k A(m,k) B(n,k).  A workgroup of 4 wavefronts computes a
-// 128x128 tile; each wavefront owns a 64x64 quadrant as 4x4 MFMA 16x16
+// C[m,n] = sum_k A(m,k) B(n,k).  In the ring a workgroup of 4 wavefronts computes
+// a 128x128 tile; each wavefront owns a 64x64 quadrant as 4x4 MFMA 16x16
 // blocks; three workgroups per CU.  Tiles of 16-byte aligned operands load
 // their 16-deep operand tiles straight from global memory into a three-stage
 // LDS ring (global_load_lds_dwordx4); edge tiles clamp those loads to the
@@ -20,9 +25,10 @@
 // reads four rows at one k), a row-major one [row][k] (four k of one row;
 // swizzled in the ring, padded in the register path), and a lane's four B
 // blocks are four adjacent output columns, stored as one float4 (a
-// streaming store for the direct products).  At c2 inside the training
-// step: input projection 119 us, dx with the weight-gradient reductions
-// 110 us, the dW pair (192x256 tiles) 233 us.  Each operand layout is a
+// streaming store for the direct products).  At I = H = 256, B T = 32768 inside
+// the training step (us, ring -> the split form now taken): input projection 119
+// -> 78, dx with the weight-gradient reductions 110 -> 81, the dW pair 233 -> 153.
+// Each operand layout is a
 // template instance, so no product carries another's address arithmetic.
 // The weight gradients (K = B*T rows) use split-K with a fixed-order
 // reduction, so results are deterministic run to run; up to 8 columns past
@@ -1240,9 +1246,8 @@ size_t splitk_partial_floats(int m, int n, int ksplit) {
 }
 
 namespace {
-// Slices of one of the pair's products in 128x128 tiles, or in the 192x256
-// tiles where those divide evenly: each product is sized for half the CUs at
-// three resident workgroups per CU.
+// Slices of one of the pair's products in the ring's 128x128 tiles: each product
+// is sized for half the CUs at three resident workgroups per CU.
 int ring_ksplit(int m, int n, int k) { return choose_ksplit(m, n, k, 128, 3); }
 
 struct PairPlan {

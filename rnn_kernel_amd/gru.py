@@ -52,9 +52,10 @@ import torch.nn as nn
 from . import _lib
 
 HIDDEN_SIZE = 256            # default hidden size, as in the reference module
-# Largest hidden size accepted: the LDS-tiled backward (hidden_size > 256)
-# keeps at least 16 rows of 3H gate gradients in a workgroup's 160 KB of
-# LDS, which holds up to hidden_size 810 at batch >= 16.
+# Largest hidden size accepted.  Above 256 the wide register recurrences run (to
+# 768); the LDS-tiled family they fall back to keeps at least 16 rows of 3H gate
+# gradients in a workgroup's 160 KB of LDS, which holds up to hidden_size 810 at
+# batch >= 16.
 MAX_HIDDEN_SIZE = 768
 DEFAULT_NUM_LAYERS = 1
 
