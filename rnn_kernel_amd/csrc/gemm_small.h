@@ -88,7 +88,8 @@ struct SmallLoader {
     __device__ __forceinline__ void load(int kb, int nkb, int klen, float4 (&v)[NV]) const {
         const int st = min(kb, nkb - 1);
         const char* p = base + (size_t)st * stage_bytes;
-        const unsigned lim = (unsigned)(klen - st * BK - (VEC && !KMAJOR ? 4 : 1)) * kunit;
+        // (a stage's own k at most: klen rows of a wide operand are past 32 bits)
+        const unsigned lim = (unsigned)min(klen - st * BK - (VEC && !KMAJOR ? 4 : 1), BK) * kunit;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             if constexpr (VEC) {

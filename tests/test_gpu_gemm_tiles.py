@@ -39,3 +39,22 @@ def test_direct_product_tiles_match_float64(gpu, hip_lib, m, n, k, b_kmajor, pad
     ref = a.double() @ (b.double() if b_kmajor else b.double().t().contiguous()) + bias.double()
     assert (c[:m].double() - ref).abs().max().item() <= 1e-6 * k + 1e-5
     assert torch.isnan(c[m]).all()  # nothing stored past the last row
+
+
+@pytest.mark.parametrize("k", [1028, 1029])  # float4 and single loads of the row-major operand
+def test_direct_product_of_a_wide_k_major_operand(gpu, hip_lib, k):
+    """k rows of 2^20 floats are more than 2^32 bytes: offsets within a stage
+    must not be limited by the whole extent taken in 32 bits."""
+    from rnn_kernel_amd import _lib
+
+    m, n, ld = 64, 64, 1 << 20
+    g = torch.Generator(device=gpu).manual_seed(k)
+    a = torch.randn(m, k, generator=g, device=gpu)
+    b = torch.zeros(k, ld, device=gpu)
+    b[:, :n] = torch.randn(k, n, generator=g, device=gpu)
+    c = torch.empty(m, n, device=gpu)
+    rc = hip_lib.rka_gemm_f32(m, n, k, a.data_ptr(), k, 0, b.data_ptr(), ld, 1, None, c.data_ptr(), n,
+                              torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "rka_gemm_f32")
+    ref = a.double() @ b[:, :n].double().contiguous()
+    assert (c.double() - ref).abs().max().item() <= 1e-6 * k + 1e-5
