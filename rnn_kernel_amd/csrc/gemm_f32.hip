@@ -36,6 +36,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <limits>
 #include <type_traits>
 #include <utility>
 
@@ -1123,8 +1124,13 @@ using Tile32 = SmallTile<32, 32, 32, 32, 64>;
 DirectTile direct_tile(const GemmArgs& g) {
     if (g.a.kmajor) return TILE_128;
     const bool vec = g.a_vec && g.b_vec;
+    // A launch takes fewer than 2^32 threads, the reducing workgroups beside the
+    // tiles included: a form with too many tiles (32x32 ones from m = 2^29 on)
+    // is not taken.
+    constexpr long long kMostTiles = (1ll << 32) / NT - 8192;
     auto cost = [&](int tm, int tn, double unit) {
-        const long long tiles = (long long)((g.m + tm - 1) / tm) * ((g.n + tn - 1) / tn);
+        const long long tiles = (((long long)g.m + tm - 1) / tm) * (((long long)g.n + tn - 1) / tn);
+        if (tiles > kMostTiles) return std::numeric_limits<double>::infinity();
         return (double)((tiles + 255) / 256) * tm * tn * unit;
     };
     DirectTile best = TILE_128;

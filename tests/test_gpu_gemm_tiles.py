@@ -58,3 +58,20 @@ def test_direct_product_of_a_wide_k_major_operand(gpu, hip_lib, k):
     _lib.check(rc, "rka_gemm_f32")
     ref = a.double() @ b[:, :n].double().contiguous()
     assert (c.double() - ref).abs().max().item() <= 1e-6 * k + 1e-5
+
+
+@pytest.mark.parametrize("m,n", [((1 << 29) - 1, 3), ((1 << 30) + 33, 1)])
+def test_direct_product_of_very_many_rows(gpu, hip_lib, m, n):
+    """So many rows that 32x32 tiles (the second: 64x64 ones too) would be a
+    launch of 2^32 threads: a form of larger tiles takes the product."""
+    from rnn_kernel_amd import _lib
+
+    print(f"direct m={m} n={n}", flush=True)
+    a = torch.arange(m, device=gpu, dtype=torch.float32).remainder_(1021.0)
+    b = torch.arange(1, n + 1, device=gpu, dtype=torch.float32)
+    c = torch.empty(m, n, device=gpu)
+    rc = hip_lib.rka_gemm_f32(m, n, 1, a.data_ptr(), 1, 0, b.data_ptr(), 1, 0, None, c.data_ptr(), n,
+                              torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "rka_gemm_f32")
+    for r in range(0, m, 1 << 27):
+        assert torch.equal(c[r:r + (1 << 27)], a[r:r + (1 << 27), None] * b)
