@@ -1256,11 +1256,6 @@ namespace {
 // is sized for half the CUs at three resident workgroups per CU.
 int ring_ksplit(int m, int n, int k) { return choose_ksplit(m, n, k, 128, 3); }
 
-struct PairPlan {
-    DirectTile tile;  // TILE_SPLIT, TILE_64, TILE_128x64 or TILE_128 (the ring)
-    int ks0, ks1;
-};
-
 // Tile and slices of the weight-gradient pair (m = 3H gate rows, n0 and n1
 // columns, k = B T).  Both products take the same
 // slices, so that every workgroup has the same work; the candidates are
@@ -1278,16 +1273,16 @@ struct PairPlan {
 // 387, 129 + 129, 32768: 163, 151 (split 115); 384, 128 + 64, 51200: 120, 86; 768,
 // 256 + 128, 8192: 61, 58.
 PairPlan make_pair_plan(int m, int n0, int n1, int k) {
-    PairPlan best{TILE_128x64, 1, 1};
+    PairPlan best{PAIR_128x64, 1, 1, false};
     constexpr int kMaxSlices = 256;
     constexpr double kStage[4] = {0.75, 0.5, 0.38, 0.35};
     const int most = std::min(kMaxSlices, std::max(1, k / (4 * kSplitBK)));
     const int least = std::min(most, (k + 4095) / 4096);
     double least_cost = 1e30;
-    for (const DirectTile tile : {TILE_64, TILE_128x64, TILE_SPLIT}) {
-        if (tile == TILE_SPLIT && !(split_takes(m, n0, k) && split_takes(m, n1, k))) continue;
-        const int tm = tile == TILE_64 ? 64 : 128, tn = tile == TILE_SPLIT ? 128 : 64;
-        const double unit = tile == TILE_64 ? 1.0 : tile == TILE_128x64 ? 1.85 : 2.1;
+    for (const PairForm form : {PAIR_64, PAIR_128x64, PAIR_SPLIT}) {
+        if (form == PAIR_SPLIT && !(split_takes(m, n0, k) && split_takes(m, n1, k))) continue;
+        const int tm = form == PAIR_64 ? 64 : 128, tn = form == PAIR_SPLIT ? 128 : 64;
+        const double unit = form == PAIR_64 ? 1.0 : form == PAIR_128x64 ? 1.85 : 2.1;
         const double tiles = (double)((m + tm - 1) / tm) * ((n0 + tn - 1) / tn + (n1 + tn - 1) / tn);
         for (int ks = 1; ks <= most; ks += ks < 8 ? 1 : 8) {
             if (ks < least && ks + 8 <= most) continue;
@@ -1299,15 +1294,16 @@ PairPlan make_pair_plan(int m, int n0, int n1, int k) {
             const double cost = rounds * (stages + 2) * stage + sums;
             if (cost < least_cost) {
                 least_cost = cost;
-                best = PairPlan{tile, ks, ks};
+                best = PairPlan{form, ks, ks, ks == 1};
             }
         }
     }
     return best;
 }
 
-// The plan of the thread's last shape is kept (a call asks for it three times).
-PairPlan plan_pair(int m, int n0, int n1, int k) {
+// The plan of the thread's last shape is kept (a call and its workspace query
+// ask for it twice each).
+PairPlan auto_pair_plan(int m, int n0, int n1, int k) {
     thread_local int key[4] = {0, 0, 0, 0};
     thread_local PairPlan plan{};
     if (key[0] != m || key[1] != n0 || key[2] != n1 || key[3] != k) {
@@ -1320,17 +1316,10 @@ PairPlan plan_pair(int m, int n0, int n1, int k) {
     return plan;
 }
 
-// Whether the pair's launch writes the results itself (one slice each, outside
-// the 128x128 ring), so that there is nothing to reduce.
-bool pair_is_direct(const SplitProduct& p0, const SplitProduct& p1) {
-    return p0.ksplit == 1 && p1.ksplit == 1 && p0.b.shift_T > 0 && p0.colsum && p1.colsum &&
-           g_gemm_tiles.load(std::memory_order_relaxed) == RKA_GEMM_TILES_AUTO;
-}
-
 // Launches the pair in tm x tn tiles: launch(grid, first product, second).
 template <typename F>
-int launch_pair_tiles(const SplitProduct& p0, const SplitProduct& p1, GemmArgs a0, GemmArgs a1, int tm, int tn,
-                      F launch) {
+int launch_pair_tiles(const SplitProduct& p0, const SplitProduct& p1, bool direct, GemmArgs a0, GemmArgs a1, int tm,
+                      int tn, F launch) {
     long long items = 0;
     for (GemmArgs* g : {&a0, &a1}) {
         g->narrow = 0;
@@ -1339,7 +1328,7 @@ int launch_pair_tiles(const SplitProduct& p0, const SplitProduct& p1, GemmArgs a
         items += (long long)g->tiles * g->ksplit;
     }
     if (items > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
-    if (pair_is_direct(p0, p1)) {
+    if (direct) {
         for (const auto& pa : {std::make_pair(&p0, &a0), std::make_pair(&p1, &a1)}) {
             pa.second->c = pa.first->c;
             pa.second->ldc = pa.first->ldc;
@@ -1354,9 +1343,9 @@ int launch_pair_tiles(const SplitProduct& p0, const SplitProduct& p1, GemmArgs a
 }
 
 template <typename S>
-int launch_small_pair(const SplitProduct& p0, const SplitProduct& p1, const GemmArgs& a0, const GemmArgs& a1,
-                      hipStream_t stream) {
-    return launch_pair_tiles(p0, p1, a0, a1, S::TM, S::TN, [&](dim3 grid, const GemmArgs& x, const GemmArgs& y) {
+int launch_small_pair(const SplitProduct& p0, const SplitProduct& p1, bool direct, const GemmArgs& a0,
+                      const GemmArgs& a1, hipStream_t stream) {
+    return launch_pair_tiles(p0, p1, direct, a0, a1, S::TM, S::TN, [&](dim3 grid, const GemmArgs& x, const GemmArgs& y) {
         if (a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec)
             hipLaunchKernelGGL((gemm_small_pair_kernel<S, true, true>), grid, dim3(NT), 0, stream, x, y);
         else
@@ -1365,16 +1354,15 @@ int launch_small_pair(const SplitProduct& p0, const SplitProduct& p1, const Gemm
 }
 }  // namespace
 
-void choose_pair_ksplit(int m, int n0, int n1, int k, int* ks0, int* ks1) {
-    PairPlan p = plan_pair(m, n0, n1, k);
-    if (g_gemm_tiles.load(std::memory_order_relaxed) != RKA_GEMM_TILES_AUTO && p.tile != TILE_SPLIT)
-        p = PairPlan{TILE_128, ring_ksplit(m, n0, k), ring_ksplit(m, n1, k)};
-    *ks0 = p.ks0;
-    *ks1 = p.ks1;
+PairPlan plan_pair(int m, int n0, int n1, int k) {
+    const PairPlan p = auto_pair_plan(m, n0, n1, k);
+    // 128x128 tiles throughout: the split form where it is the choice anyway
+    if (g_gemm_tiles.load(std::memory_order_relaxed) == RKA_GEMM_TILES_AUTO || p.form == PAIR_SPLIT) return p;
+    return PairPlan{PAIR_RING, ring_ksplit(m, n0, k), ring_ksplit(m, n1, k), false};
 }
 
 void pair_ksplit_bound(int m, int n0, int n1, int k, int* ks0, int* ks1) {
-    const PairPlan p = plan_pair(m, n0, n1, k);
+    const PairPlan p = auto_pair_plan(m, n0, n1, k);
     *ks0 = std::max(p.ks0, ring_ksplit(m, n0, k));
     *ks1 = std::max(p.ks1, ring_ksplit(m, n1, k));
 }
@@ -1427,7 +1415,8 @@ int gemm_splitk_partials(int m, int n, int k, const GemmOperand& a, const GemmOp
     return launch_gemm<true>(args, ksplit, args.a_vec != 0, args.b_vec != 0, stream);
 }
 
-int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, hipStream_t stream) {
+int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan,
+                              hipStream_t stream) {
     GemmArgs a0, a1;
     RKA_RETURN_IF_ERR(split_args(p0.m, p0.n, p0.k, p0.a, p0.b, p0.colsum != nullptr, p0.partial, p0.ksplit, 0,
                                  p0.ksplit, true, &a0));
@@ -1436,19 +1425,17 @@ int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, hi
     if (p1.b.shift_T > 0) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: only the first product of a pair is remapped");
     const bool seg = a0.a.seg.len || a0.b.seg.len || a1.a.seg.len || a1.b.seg.len;
     if (seg) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: pair products take whole operands");
-    if (p0.b.shift_T > 0) {
-        const bool any = g_gemm_tiles.load(std::memory_order_relaxed) == RKA_GEMM_TILES_AUTO;
-        const DirectTile tile = plan_pair(p0.m, p0.n, p1.n, p0.k).tile;
-        if (tile == TILE_SPLIT) {
-            const bool vec = a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec;
-            auto kern = vec ? gemm_split_pair_kernel<false> : gemm_split_pair_kernel<true>;
-            return launch_pair_tiles(p0, p1, a0, a1, kSplitTile, kSplitTile,
-                                     [&](dim3 grid, const GemmArgs& x, const GemmArgs& y) {
-                                         hipLaunchKernelGGL(kern, grid, dim3(NT), 0, stream, x, y);
-                                     });
-        }
-        if (any && tile == TILE_64) return launch_small_pair<Tile64>(p0, p1, a0, a1, stream);
-        if (any) return launch_small_pair<Tile128x64>(p0, p1, a0, a1, stream);
+    if (plan.form != PAIR_RING) {
+        if (p0.b.shift_T <= 0 || !p0.colsum || !p1.colsum || p0.ksplit != plan.ks0 || p1.ksplit != plan.ks1)
+            return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: not the pair of the plan");
+        if (plan.form == PAIR_64) return launch_small_pair<Tile64>(p0, p1, plan.direct, a0, a1, stream);
+        if (plan.form == PAIR_128x64) return launch_small_pair<Tile128x64>(p0, p1, plan.direct, a0, a1, stream);
+        const bool vec = a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec;
+        auto kern = vec ? gemm_split_pair_kernel<false> : gemm_split_pair_kernel<true>;
+        return launch_pair_tiles(p0, p1, plan.direct, a0, a1, kSplitTile, kSplitTile,
+                                 [&](dim3 grid, const GemmArgs& x, const GemmArgs& y) {
+                                     hipLaunchKernelGGL(kern, grid, dim3(NT), 0, stream, x, y);
+                                 });
     }
     const dim3 grid(a0.tiles * a0.ksplit + a1.tiles * a1.ksplit);
     const bool ua = !(a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec);
@@ -1502,8 +1489,8 @@ int splitk_reduce(const SplitProduct& p, hipStream_t stream) {
     return launch_reduce(reduce_job(p), ReduceJob{}, stream);
 }
 
-int splitk_reduce_pair(const SplitProduct& p0, const SplitProduct& p1, hipStream_t stream) {
-    if (pair_is_direct(p0, p1)) return 0;
+int splitk_reduce_pair(const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan, hipStream_t stream) {
+    if (plan.direct) return 0;
     return launch_reduce(reduce_job(p0), reduce_job(p1), stream);
 }
 
@@ -1519,12 +1506,12 @@ void launch_direct_reduce(const GemmArgs& args, const ReduceJob& j0, const Reduc
 }  // namespace
 
 int gemm_direct_reduce_pair(int m, int n, int k, const GemmOperand& a, const GemmOperand& b, float* c, int ldc,
-                            const SplitProduct& p0, const SplitProduct& p1, hipStream_t stream) {
+                            const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan, hipStream_t stream) {
     if (m <= 0 || n <= 0 || k < 0) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: m and n must be positive");
     if (!a.ptr || !b.ptr || !c) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: null operand");
     RKA_RETURN_IF_ERR(check_ld(a, b));
     if (a.seg.len || b.seg.len || b.shift_T > 0) {
-        RKA_RETURN_IF_ERR(splitk_reduce_pair(p0, p1, stream));
+        RKA_RETURN_IF_ERR(splitk_reduce_pair(p0, p1, plan, stream));
         return gemm_direct(m, n, k, a, b, nullptr, c, ldc, stream);
     }
     const DeviceInfo* dev = nullptr;
@@ -1542,7 +1529,7 @@ int gemm_direct_reduce_pair(int m, int n, int k, const GemmOperand& a, const Gem
     finish_args<false>(args, 1, vec_ok(a, m, k), vec_ok(b, n, k));
     // one reducing workgroup per CU: with the product's tiles at up to two
     // per CU they run beside them, in the third workgroup slot
-    const long reducers = pair_is_direct(p0, p1) ? 0 : dev->num_cus > 0 ? dev->num_cus : 256;
+    const long reducers = plan.direct ? 0 : dev->num_cus > 0 ? dev->num_cus : 256;
     if ((long long)args.tiles + reducers > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
     const dim3 grid((unsigned)(args.tiles + reducers));
     const ReduceJob j0 = reduce_job(p0), j1 = reduce_job(p1);

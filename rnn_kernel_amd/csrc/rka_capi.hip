@@ -88,12 +88,12 @@ StackLayout stack_layout(int L, int B, int T, int I, int H) {
 
 struct BwdLayout {
     size_t g, rec, part_hh, part_ih, total;
-    int ks_hh, ks_ih;  // split-K slices
+    PairPlan pair;  // the weight gradients: dW_hh, dW_ih
 };
 BwdLayout bwd_layout(int B, int T, int I, int H) {
     BwdLayout l{};
     const int K = B * T;
-    choose_pair_ksplit(3 * H, H, I, K, &l.ks_hh, &l.ks_ih);
+    l.pair = plan_pair(3 * H, H, I, K);
     int most_hh = 0, most_ih = 0;
     pair_ksplit_bound(3 * H, H, I, K, &most_hh, &most_ih);
     l.g = 0;
@@ -285,16 +285,16 @@ int rka_gru_backward(const float* x, const float* h0, const float* w_ih, const f
     // dW_ih = G_i^T X, G_i = g[:, H:4H] in (r, z, n) order.  One launch.
     {
         const SplitProduct hh{3 * H, H, K, GemmOperand{g, 4 * H, 1, 0, nullptr}, GemmOperand{y, H, 1, T, h0},
-                              dw_hh, H, db_hh, H, reinterpret_cast<float*>(ws + l.part_hh), l.ks_hh};
+                              dw_hh, H, db_hh, H, reinterpret_cast<float*>(ws + l.part_hh), l.pair.ks0};
         const SplitProduct ih{3 * H, I, K, GemmOperand{g + H, 4 * H, 1, 0, nullptr}, GemmOperand{x, I, 1, 0, nullptr},
-                              dw_ih, I, db_ih, 0, reinterpret_cast<float*>(ws + l.part_ih), l.ks_ih};
+                              dw_ih, I, db_ih, 0, reinterpret_cast<float*>(ws + l.part_ih), l.pair.ks1};
         {
             StageScope scope(3, s);
-            RKA_RETURN_IF_ERR(gemm_splitk_pair_partials(hh, ih, s));
+            RKA_RETURN_IF_ERR(gemm_splitk_pair_partials(hh, ih, l.pair, s));
         }
         if (!dx) {
             StageScope scope(4, s);
-            return splitk_reduce_pair(hh, ih, s);
+            return splitk_reduce_pair(hh, ih, l.pair, s);
         }
         // dX = G_i W_ih: A(m=bt, k=j) = g[bt, H+j]; B(n=i, k=j) = W_ih[j, i].
         // One launch with the reductions, which run beside its tiles (stage
@@ -302,7 +302,7 @@ int rka_gru_backward(const float* x, const float* h0, const float* w_ih, const f
         GemmOperand ga{g + H, 4 * H, 0, 0, nullptr};
         GemmOperand wk{w_ih, I, 1, 0, nullptr};
         StageScope scope(5, s);
-        return gemm_direct_reduce_pair(K, I, 3 * H, ga, wk, dx, I, hh, ih, s);
+        return gemm_direct_reduce_pair(K, I, 3 * H, ga, wk, dx, I, hh, ih, l.pair, s);
     }
     return 0;
 }

@@ -101,30 +101,37 @@ struct SplitProduct {
     float* partial;
     int ksplit;
 };
+// How the weight-gradient pair of a backward call runs.  Taken once per call
+// (plan_pair reads the tile mode of rka_set_gemm_tiles, which another thread may
+// change meanwhile) and handed to the pair's launch and to its reduction.
+enum PairForm { PAIR_RING, PAIR_64, PAIR_128x64, PAIR_SPLIT };
+struct PairPlan {
+    PairForm form;
+    int ks0, ks1;  // k-slices of the two products
+    bool direct;   // the launch writes the results itself: nothing to reduce
+};
+// m rows, n0 and n1 columns.
+PairPlan plan_pair(int m, int n0, int n1, int k);
+// The most slices over every tile mode, which sizes the workspace.
+void pair_ksplit_bound(int m, int n0, int n1, int k, int* ks0, int* ks1);
 // The partial products of two split-K products in one launch (all slices
-// of each; reduce each with splitk_reduce); only p0's B operand may carry
-// the row remap.  With the reductions, the same results as two gemm_splitk
-// calls with the same slices.
-int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, hipStream_t stream);
+// of each, or the results); only p0's B operand may carry the row remap.
+int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan,
+                              hipStream_t stream);
 int splitk_reduce(const SplitProduct& p, hipStream_t stream);
 // Both products' reductions in one launch (the same results as two
 // splitk_reduce calls).
-int splitk_reduce_pair(const SplitProduct& p0, const SplitProduct& p1, hipStream_t stream);
+int splitk_reduce_pair(const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan, hipStream_t stream);
 // gemm_direct (no bias) and splitk_reduce_pair(p0, p1) in one launch: the
 // same results as the two calls.
 int gemm_direct_reduce_pair(int m, int n, int k, const GemmOperand& a, const GemmOperand& b, float* c, int ldc,
-                            const SplitProduct& p0, const SplitProduct& p1, hipStream_t stream);
+                            const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan, hipStream_t stream);
 // rka_set_gemm_tiles (RKA_GEMM_TILES_AUTO or RKA_GEMM_TILES_128).
 int set_gemm_tiles(int mode);
 // Slices for a split-K product of about wgs_per_cu workgroups per CU
 // (0: half a workgroup per CU, for products that share the GPU with a
 // concurrently running recurrence); a multiple of 8 from 8 up.
 int choose_ksplit(int m, int n, int k, int num_cus, int wgs_per_cu);
-// Slices of the weight-gradient pair's products (m rows, n0 and n1 columns) at
-// the current tile choice, and the most over every choice (rka_set_gemm_tiles),
-// which sizes the workspace.
-void choose_pair_ksplit(int m, int n0, int n1, int k, int* ks0, int* ks1);
-void pair_ksplit_bound(int m, int n0, int n1, int k, int* ks0, int* ks1);
 
 // ----------------------------------------------------------- recurrence ---
 enum RecKind { REC_AUTO = 0, REC_TILED = 1, REC_REGISTER = 2 };

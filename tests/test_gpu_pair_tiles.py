@@ -4,6 +4,8 @@ one slice (the results written by the products' own launch), few, and a
 multiple of 8; sequences shorter than a 16-deep stage and of one step (the
 [h0 ; y[:, :-1]] rows); a last slice shorter than the others; aligned and
 unaligned rows; 64x64 and 128x64 tiles and the ring."""
+import threading
+
 import pytest
 import torch
 
@@ -64,3 +66,55 @@ def test_weight_gradients_match_float64(gpu, hip_lib, B, T, I, H, need_dx):
         ref = (g_ih @ w_ih.double()).view(B, T, I)
         mag = (g_ih.abs() @ w_ih.double().abs()).view(B, T, I)
         assert bool(((dx.double() - ref).abs() <= 3 * H * 2.0 ** -24 * mag + 1e-30).all())
+
+
+def test_tile_mode_changed_by_another_thread(gpu, hip_lib):
+    """A call takes its plan once: with another thread switching the tile mode
+    all along, a pass with one slice per product (whose launch writes the
+    results itself, or leaves partial sums to a reduction) gives one mode's
+    weight gradients or the other's, never unwritten ones."""
+    from rnn_kernel_amd import _lib
+
+    B, T, I, H = 2, 8, 16, 16
+    gen = torch.Generator(device=gpu).manual_seed(4)
+
+    def randn(*shape):
+        return torch.randn(*shape, generator=gen, device=gpu)
+
+    x, h0, y, dy = randn(B, T, I), randn(B, H), torch.tanh(randn(B, T, H)), randn(B, T, H)
+    w_ih, w_hh, res = 0.1 * randn(3 * H, I), 0.1 * randn(3 * H, H), torch.sigmoid(randn(B, T, H, 4))
+    nb = hip_lib.rka_gru_backward_workspace_bytes(B, T, I, H)
+    dx, dh0, nan = torch.empty(B, T, I, device=gpu), torch.empty(B, H, device=gpu), float("nan")
+
+    def run():
+        ws = torch.full((nb,), 255, dtype=torch.uint8, device=gpu)  # (NaN where read as float)
+        out = [torch.full(s, nan, device=gpu) for s in ((3 * H, I), (3 * H, H), (3 * H,), (3 * H,))]
+        _lib.check(hip_lib.rka_gru_backward(x.data_ptr(), h0.data_ptr(), w_ih.data_ptr(), w_hh.data_ptr(), y.data_ptr(),
+                                            res.data_ptr(), dy.data_ptr(), None, dx.data_ptr(), dh0.data_ptr(),
+                                            *[o.data_ptr() for o in out], ws.data_ptr(), nb, B, T, I, H,
+                                            torch.cuda.current_stream().cuda_stream), "backward")
+        return torch.cat([o.flatten() for o in out])
+
+    stop = threading.Event()
+
+    def switch():
+        mode = 0
+        while not stop.is_set():
+            mode ^= 1
+            hip_lib.rka_set_gemm_tiles(mode)
+
+    thread = threading.Thread(target=switch)
+    try:
+        want = []
+        for mode in (0, 1):
+            _lib.set_gemm_tiles(mode)
+            want.append(run())
+        assert torch.isfinite(want[0]).all() and torch.allclose(want[0], want[1], rtol=1e-5, atol=1e-6)
+        thread.start()
+        got = [run() for _ in range(600)]
+    finally:
+        stop.set()
+        if thread.is_alive():
+            thread.join()
+        _lib.set_gemm_tiles(0)
+    assert all(any(torch.equal(g, w) for w in want) for g in got)
