@@ -32,9 +32,7 @@
 // Non-finite values: the pieces of an infinity are not finite sums, so an output
 // that comes out infinite or NaN is computed again as a plain float32 dot
 // product by the lane that stored it (split_redo); finite results are never
-// touched.  A piece, or a product of two, below 2^-126 counts as zero: what
-// underflows is 2^-17 of a value, so operands or products below some 1e-33 keep
-// fewer bits.
+// touched.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -45,8 +43,20 @@ constexpr int kSplitTile = 128;                  // tile edge
 constexpr int kPlane = kSplitTile * 8;           // dwords of a plane: 128 rows x 16 k of bf16
 constexpr int kSplitStage = 2 * 3 * kPlane;      // dwords of a stage
 
-// The three pieces of a and b, packed in pairs (a low).
+// Operands are multiplied by 2^23 before they are split, products by 2^-46 in the
+// end.  The smallest float32 is 2^-149, so that every piece is then at least
+// 2^-126, and a product of pieces that could be lost is below 2^-172: nothing
+// is lost that a float32 holds.  Without the scale the lower pieces of values
+// below some 1e-33 were: error of a product with one operand of 1e-36 2.7e-5
+// (2-norm, against 2.4e-7), of 1e-38 2.7e-3.  Operands from 2^105 or sums from 2^82
+// overflow, and are computed again as other results that are not finite.
+constexpr float kSplitScale = 8388608.f;                  // 2^23
+constexpr float kSplitUnscale = 1.f / kSplitScale / kSplitScale;
+
+// The three pieces of scaled a and b, packed in pairs (a low).
 __device__ __forceinline__ void split3(float a, float b, unsigned (&p)[3]) {
+    a *= kSplitScale;
+    b *= kSplitScale;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const bf16x2 v = {(__bf16)a, (__bf16)b};
@@ -366,7 +376,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = row_of(x, r);
-            const float v[2] = {acc[x][0][r] + bias[0], acc[x][1][r] + bias[1]};
+            const float v[2] = {fmaf(acc[x][0][r], kSplitUnscale, bias[0]), fmaf(acc[x][1][r], kSplitUnscale, bias[1])};
             odd = odd || !__builtin_isfinite(v[0]) || !__builtin_isfinite(v[1]);
             if (m >= p.m) continue;
             float* dst = dst_of(m);

@@ -50,6 +50,26 @@ def test_split_product_error(gpu, hip_lib, m, n, k, b_kmajor, scale):
     assert bool(((c.double() - ref).abs() <= (6 * stages + 4) * 2.0 ** -24 * mag + tiny).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(32768, 128, 16), (32641, 132, 20), (32701, 125, 5), (32768, 129, 387)])
+@pytest.mark.parametrize("b_kmajor", [0, 1])
+@pytest.mark.parametrize("sa,sb", [(1e-36, 1.0), (1.0, 1e-38), (1e-41, 1.0), (1.0, 1e-41), (1e-19, 1e-19), (1e-41, 1e36)])
+def test_split_product_of_small_magnitudes(gpu, hip_lib, m, n, k, b_kmajor, sa, sb):
+    """Operands and products down to the smallest float32 keep the bits that a
+    float32 product keeps."""
+    print(f"split m={m} n={n} k={k} b_kmajor={b_kmajor} sa={sa} sb={sb}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    a = sa * torch.randn(m, k, generator=g, device=gpu)
+    b = sb * torch.randn((k, n) if b_kmajor else (n, k), generator=g, device=gpu)
+    c = _product(gpu, hip_lib, a, b, b_kmajor)
+    bd = b.double() if b_kmajor else b.double().t().contiguous()
+    ref = a.double() @ bd
+    mag = a.double().abs() @ bd.abs()
+    # as in test_split_product_error, and one rounding of a result below the
+    # normal range (half of 2^-149)
+    stages = (k + 15) // 16
+    assert bool(((c.double() - ref).abs() <= (6 * stages + 4) * 2.0 ** -24 * mag + 2.0 ** -150).all())
+
+
 @pytest.mark.parametrize("b_kmajor", [0, 1])
 def test_split_product_non_finite(gpu, hip_lib, b_kmajor):
     """Rows with an infinity, a NaN, values that round past the largest bf16 and
