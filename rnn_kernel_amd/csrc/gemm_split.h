@@ -53,10 +53,21 @@ constexpr int kSplitStage = 2 * 3 * kPlane;      // dwords of a stage
 constexpr float kSplitScale = 8388608.f;                  // 2^23
 constexpr float kSplitUnscale = 1.f / kSplitScale / kSplitScale;
 
-// The three pieces of scaled a and b, packed in pairs (a low).
-__device__ __forceinline__ void split3(float a, float b, unsigned (&p)[3]) {
-    a *= kSplitScale;
-    b *= kSplitScale;
+// v_mfma_f32_32x32x16_bf16 rounds its sums towards minus infinity (what the
+// addends hold below the largest one's last bits is cut off): on average -2e-8 of
+// an output's mean magnitude at k = 256, -1.5e-7 at k = 2304, in every row alike.
+// What later sums over rows (the gradients of a stack's lower layers) adds that
+// up, where roundings to nearest cancel.  So A's odd rows are split with the
+// opposite sign and their sums negated in the end, which turns the direction of
+// their rounding: the mean over all rows is then below 3e-10, as on the fp32 matrix
+// cores.  In the split-K products odd slices change sign too, so that the error
+// cancels in the sum of the slices (k = 262144: 1.6e-6 -> 8.8e-7).
+
+// The three pieces of a and b times s (a scale of either sign), packed in pairs
+// (a low).
+__device__ __forceinline__ void split3(float a, float b, float s, unsigned (&p)[3]) {
+    a *= s;
+    b *= s;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const bf16x2 v = {(__bf16)a, (__bf16)b};
@@ -71,25 +82,27 @@ __device__ __forceinline__ void split3(float a, float b, unsigned (&p)[3]) {
 // LDS planes of an operand's stage.  Row-major: [row][16 k] (32 bytes a row;
 // thread x of a pass holds k 4 (x % 4) of row x / 4).  k-major: [k pair][row] of
 // dwords (thread: rows 4 (t % 32) .. + 3 at k 2 (t / 32) and the next).  Every
-// access of either is free of bank conflicts.
-template <int KMAJOR>
-__device__ __forceinline__ void split_store(unsigned* lds, int tid, const float4 (&v)[2]) {
+// access of either is free of bank conflicts.  s: the scale of the thread's rows
+// (ALT, k-major: of its even rows, odd ones take -s).
+template <int KMAJOR, bool ALT>
+__device__ __forceinline__ void split_store(unsigned* lds, int tid, float s, const float4 (&v)[2]) {
     if constexpr (KMAJOR == 0) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             unsigned p[3], q[3];
-            split3(v[j].x, v[j].y, p);
-            split3(v[j].z, v[j].w, q);
+            split3(v[j].x, v[j].y, s, p);
+            split3(v[j].z, v[j].w, s, q);
 #pragma unroll
             for (int c = 0; c < 3; ++c)
                 *reinterpret_cast<uintx2*>(lds + c * kPlane + (tid + NT * j) * 2) = uintx2{p[c], q[c]};
         }
     } else {
         unsigned p[4][3];
-        split3(v[0].x, v[1].x, p[0]);
-        split3(v[0].y, v[1].y, p[1]);
-        split3(v[0].z, v[1].z, p[2]);
-        split3(v[0].w, v[1].w, p[3]);
+        const float odd = ALT ? -s : s;
+        split3(v[0].x, v[1].x, s, p[0]);
+        split3(v[0].y, v[1].y, odd, p[1]);
+        split3(v[0].z, v[1].z, s, p[2]);
+        split3(v[0].w, v[1].w, odd, p[3]);
 #pragma unroll
         for (int c = 0; c < 3; ++c)
             *reinterpret_cast<uintx4*>(lds + c * kPlane + (tid / 32) * kSplitTile + 4 * (tid % 32)) =
@@ -263,6 +276,10 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
     const LA la(p.a, p.m, m0, kbeg, klen, tid);
     LB lb(p.b, p.n, n0, kbeg, klen, tid);
     float4 ra[2][2], rb[2][2];
+    // the sign of the tile's even rows; a thread's rows of a row-major A are tid /
+    // 4 and that plus 64, all odd or all even
+    const float sign = SPLIT && (bz & 1) ? -1.f : 1.f;
+    const float scale_a = kSplitScale * (AK ? sign : (tid / 4) % 2 ? -sign : sign);
     floatx16 acc[2][2];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
@@ -313,8 +330,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
                 cs.w += ra[ST][0].w + ra[ST][1].w;
             }
         }
-        split_store<AK>(as, tid, ra[ST]);
-        split_store<BKM>(bs, tid, rb[ST]);
+        split_store<AK, true>(as, tid, scale_a, ra[ST]);
+        split_store<BKM, false>(bs, tid, kSplitScale, rb[ST]);
         la.load(kb + 2, nkb, klen, tid, ra[ST]);
         lb.load(kb + 2, nkb, klen, tid, rb[ST]);
         __syncthreads();
@@ -370,13 +387,15 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
 #pragma unroll
         for (int y = 0; y < 2; ++y) bias[y] = p.bias[min(col_of(y), p.n - 1)];
     }
+    const float unscale = sign * kSplitUnscale;
     bool odd = false;  // an output that is not finite
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = row_of(x, r);
-            const float v[2] = {fmaf(acc[x][0][r], kSplitUnscale, bias[0]), fmaf(acc[x][1][r], kSplitUnscale, bias[1])};
+            const float u = (AK ? x : r) % 2 ? -unscale : unscale;  // m odd: the row's sums are negated
+            const float v[2] = {fmaf(acc[x][0][r], u, bias[0]), fmaf(acc[x][1][r], u, bias[1])};
             odd = odd || !__builtin_isfinite(v[0]) || !__builtin_isfinite(v[1]);
             if (m >= p.m) continue;
             float* dst = dst_of(m);

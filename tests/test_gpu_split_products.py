@@ -70,6 +70,24 @@ def test_split_product_of_small_magnitudes(gpu, hip_lib, m, n, k, b_kmajor, sa, 
     assert bool(((c.double() - ref).abs() <= (6 * stages + 4) * 2.0 ** -24 * mag + 2.0 ** -150).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(32768, 128, 256), (32768, 129, 387), (32768, 128, 2304)])
+@pytest.mark.parametrize("b_kmajor", [0, 1])
+def test_split_product_error_has_no_mean(gpu, hip_lib, m, n, k, b_kmajor):
+    """The errors cancel in a sum over the rows (a bias gradient of the layer
+    below sums thousands of them), as roundings to nearest do."""
+    print(f"split m={m} n={n} k={k} b_kmajor={b_kmajor}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g, device=gpu)
+    b = torch.randn((k, n) if b_kmajor else (n, k), generator=g, device=gpu)
+    ref = a.double() @ (b.double() if b_kmajor else b.double().t().contiguous())
+    mean = (_product(gpu, hip_lib, a, b, b_kmajor).double() - ref).mean() / ref.abs().mean()
+    # six roundings per 16-deep stage, each at most 2^-24 of an output's size and
+    # of either sign alike: six standard deviations of the mean of m n outputs
+    # (measured: below one)
+    stages = (k + 15) // 16
+    assert abs(mean.item()) <= 6 * 2.0 ** -24 * (6 * stages / (m * n)) ** 0.5
+
+
 @pytest.mark.parametrize("b_kmajor", [0, 1])
 def test_split_product_non_finite(gpu, hip_lib, b_kmajor):
     """Rows with an infinity, a NaN, values that round past the largest bf16 and
