@@ -1260,8 +1260,13 @@ int ring_ksplit(int m, int n, int k) { return choose_ksplit(m, n, k, 128, 3); }
 // columns, k = B T).  Both products take the same
 // slices, so that every workgroup has the same work; the candidates are
 // multiples of 8 (a slice's tiles then share an XCD, split_coords) and fewer
-// than 8, each slice at least four 16-deep stages and at most 4096 values long
-// (the length of a chain of float32 additions).  Taken is the least of
+// than 8, each slice at least four 16-deep stages and, up to k = 2^20 (256 slices
+// at most), at most 4096 values long.  No chain of float32 additions may round
+// more than the ring's slices do: the 64x64 form closes its sums every 128 values
+// (gemm_small.h), the 128x64 form takes at least the ring's slices (`ring`, the
+// finer of the two products), the split form, whose error over as many values is
+// 0.73 of theirs, at least 5/9 of them.  Error against the ring's over 119 sizes
+// (dW, db, 2-norm): 0.1 to 1.1 times (2.5 without this rule).  Taken is the least of
 //   workgroups per CU x (stages + 2) x (time of a stage at that many)
 //   + the partial sums, written and read again,
 // where up to four workgroups share a CU and a part of one counts whole.  A
@@ -1277,11 +1282,13 @@ PairPlan make_pair_plan(int m, int n0, int n1, int k) {
     constexpr int kMaxSlices = 256;
     constexpr double kStage[4] = {0.75, 0.5, 0.38, 0.35};
     const int most = std::min(kMaxSlices, std::max(1, k / (4 * kSplitBK)));
-    const int least = std::min(most, (k + 4095) / 4096);
+    const int ring = std::max(ring_ksplit(m, n0, k), ring_ksplit(m, n1, k));
     double least_cost = 1e30;
     for (const PairForm form : {PAIR_64, PAIR_128x64, PAIR_SPLIT}) {
         if (form == PAIR_SPLIT && !(split_takes(m, n0, k) && split_takes(m, n1, k))) continue;
         const int tm = form == PAIR_64 ? 64 : 128, tn = form == PAIR_SPLIT ? 128 : 64;
+        const int fine = form == PAIR_64 ? 1 : form == PAIR_128x64 ? ring : (5 * ring + 8) / 9;
+        const int least = std::min(most, std::max((k + 4095) / 4096, fine));
         const double unit = form == PAIR_64 ? 1.0 : form == PAIR_128x64 ? 1.85 : 2.1;
         const double tiles = (double)((m + tm - 1) / tm) * ((n0 + tn - 1) / tn + (n1 + tn - 1) / tn);
         for (int ks = 1; ks <= most; ks += ks < 8 ? 1 : 8) {

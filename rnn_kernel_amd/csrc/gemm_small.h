@@ -228,6 +228,16 @@ __device__ __forceinline__ void small_frag(const float* lds, int row0, int k, in
     }
 }
 
+// A weight gradient sums thousands of time steps: the 64x64 form closes its
+// float32 sums every kFoldStages stages (128 values) and adds those up apart, so
+// that a slice may be as long as the launch wants it and no chain of additions is
+// longer than in the ring's shortest slices.  Error against float64 (2-norm) at
+// batch 16, 256 steps, I = H = 256 in eight slices: 4.1e-7 -> 2.1e-7 (the ring, 32
+// slices: 2.1e-7); time of the backward's products 69 -> 71 us.  The 128x64
+// form would lose a workgroup per CU to the second set of sums (235 -> 276 us at
+// 75, 258, 3, 308); its slices are kept as short as the ring's (make_pair_plan).
+constexpr int kFoldStages = 8;
+
 // One tile (bx, by); SPLIT: the partial products of k slice bz, with the column
 // sums of A (the bias gradients) in the first column of tiles.
 template <int AK, int BKM, typename S, bool VEC, bool SPLIT = false, bool BSHIFT = false>
@@ -307,11 +317,42 @@ __device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, in
         load(0, 0);
         load(1, 1);
         int kb = 0;
-        for (; kb + 1 < nkb; kb += 2) {
-            stage(kb, std::integral_constant<int, 0>{});
-            stage(kb + 1, std::integral_constant<int, 1>{});
+        auto run = [&](int end) {
+            for (; kb + 1 < end; kb += 2) {
+                stage(kb, std::integral_constant<int, 0>{});
+                stage(kb + 1, std::integral_constant<int, 1>{});
+            }
+        };
+        if constexpr (SPLIT && TM == 64) {
+            floatx4 sum[MB][NB];
+            float csum = 0.f;
+#pragma unroll
+            for (int x = 0; x < MB; ++x)
+#pragma unroll
+                for (int y = 0; y < NB; ++y) sum[x][y] = floatx4{0.f, 0.f, 0.f, 0.f};
+            while (kb + kFoldStages < nkb) {
+                run(kb + kFoldStages);
+#pragma unroll
+                for (int x = 0; x < MB; ++x)
+#pragma unroll
+                    for (int y = 0; y < NB; ++y) {
+                        sum[x][y] += acc[x][y];
+                        acc[x][y] = floatx4{0.f, 0.f, 0.f, 0.f};
+                    }
+                csum += cs;
+                cs = 0.f;
+            }
+            run(nkb);
+            if (kb < nkb) stage(kb, std::integral_constant<int, 0>{});
+#pragma unroll
+            for (int x = 0; x < MB; ++x)
+#pragma unroll
+                for (int y = 0; y < NB; ++y) acc[x][y] += sum[x][y];
+            cs += csum;
+        } else {
+            run(nkb);
+            if (kb < nkb) stage(kb, std::integral_constant<int, 0>{});
         }
-        if (kb < nkb) stage(kb, std::integral_constant<int, 0>{});
     }
     // through LDS: the wavefronts that split k are added in order, and rows of C
     // are written whole

@@ -68,6 +68,54 @@ def test_weight_gradients_match_float64(gpu, hip_lib, B, T, I, H, need_dx):
         assert bool(((dx.double() - ref).abs() <= 3 * H * 2.0 ** -24 * mag + 1e-30).all())
 
 
+# sizes whose few long slices had chains of up to 4096 additions; B, T, I, H
+@pytest.mark.parametrize("B,T,I,H", [(16, 256, 256, 256), (236, 19, 12, 412), (6, 549, 2, 389), (115, 155, 1, 242),
+                                     (164, 51, 51, 130), (75, 258, 3, 308), (6, 1622, 12, 653)])
+def test_weight_gradients_are_no_further_off_than_the_ring(gpu, hip_lib, B, T, I, H):
+    """Error against float64 (2-norm) of the chosen form at most that of the
+    128x128 ring's short slices (one fifth more: two samples of rounding)."""
+    from rnn_kernel_amd import _lib
+
+    print(f"pair B={B} T={T} I={I} H={H}", flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(B + T + I + H)
+
+    def randn(*shape):
+        return torch.randn(*shape, generator=gen, device=gpu)
+
+    x, h0, y, dy = randn(B, T, I), randn(B, H), torch.tanh(randn(B, T, H)), randn(B, T, H)
+    w_ih, w_hh, res = 0.1 * randn(3 * H, I), 0.1 / H ** 0.5 * randn(3 * H, H), torch.sigmoid(randn(B, T, H, 4))
+    stream = torch.cuda.current_stream().cuda_stream
+    g, dh0 = torch.empty(B, T, 4, H, device=gpu), torch.empty(B, H, device=gpu)
+    nb = hip_lib.rka_gru_recurrence_workspace_bytes(B, H)
+    ws = torch.empty(nb, dtype=torch.uint8, device=gpu)
+    _lib.check(hip_lib.rka_gru_recurrence_backward(dy.data_ptr(), None, res.data_ptr(), h0.data_ptr(), y.data_ptr(),
+                                                   w_hh.data_ptr(), g.data_ptr(), dh0.data_ptr(), ws.data_ptr(), nb, B,
+                                                   T, H, stream), "recurrence_backward")
+    G = g.double().view(B * T, 4 * H)
+    g_ih, g_hh = G[:, H:], torch.cat([G[:, H:3 * H], G[:, :H]], dim=1)
+    hprev = torch.cat([h0[:, None], y[:, :-1]], dim=1).double().reshape(B * T, H)
+    refs = (g_ih.t().contiguous() @ x.double().reshape(B * T, I), g_hh.t().contiguous() @ hprev)
+    nb = hip_lib.rka_gru_backward_workspace_bytes(B, T, I, H)
+    ws = torch.empty(nb, dtype=torch.uint8, device=gpu)
+
+    def errors(mode):
+        # (a pair that the split form takes runs in it in either mode: then
+        # unaligned sizes of the same slices are compared with themselves)
+        _lib.set_gemm_tiles(mode)
+        out = [torch.empty(*s, device=gpu) for s in ((3 * H, I), (3 * H, H), (3 * H,), (3 * H,))]
+        _lib.check(hip_lib.rka_gru_backward(x.data_ptr(), h0.data_ptr(), w_ih.data_ptr(), w_hh.data_ptr(), y.data_ptr(),
+                                            res.data_ptr(), dy.data_ptr(), None, None, dh0.data_ptr(),
+                                            *[o.data_ptr() for o in out], ws.data_ptr(), nb, B, T, I, H, stream),
+                   "backward")
+        return [((o.double() - r).norm() / r.norm()).item() for o, r in zip(out, refs)]
+
+    try:
+        ring, own = errors(1), errors(0)
+    finally:
+        _lib.set_gemm_tiles(0)
+    assert all(e <= 1.2 * r for e, r in zip(own, ring)), (own, ring)
+
+
 def test_tile_mode_changed_by_another_thread(gpu, hip_lib):
     """A call takes its plan once: with another thread switching the tile mode
     all along, a pass with one slice per product (whose launch writes the
