@@ -239,8 +239,9 @@ __device__ __forceinline__ void small_frag(const float* lds, int row0, int k, in
 constexpr int kFoldStages = 8;
 
 // One tile (bx, by); SPLIT: the partial products of k slice bz, with the column
-// sums of A (the bias gradients) in the first column of tiles.
-template <int AK, int BKM, typename S, bool VEC, bool SPLIT = false, bool BSHIFT = false>
+// sums of A (the bias gradients) in the first column of tiles.  REDO: only outputs
+// that are not finite are replaced (gemm_split.h), and no column sums formed.
+template <int AK, int BKM, typename S, bool VEC, bool SPLIT = false, bool BSHIFT = false, bool REDO = false>
 __device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, int bz, float* smem) {
     static_assert(!SPLIT || (AK == 1 && BKM == 1 && S::WK == 1), "split-K products take k-major operands");
     constexpr int TM = S::TM, TN = S::TN, BK = S::BK, MB = S::MB, NB = S::NB;
@@ -255,7 +256,7 @@ __device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, in
     const int kbeg = SPLIT ? bz * p.kchunk : 0;
     const int klen = SPLIT ? max(0, min(p.k - kbeg, p.kchunk)) : p.k;
     const int nkb = (klen + BK - 1) / BK;
-    const bool colsum = SPLIT && p.want_colsum && by == 0;
+    const bool colsum = SPLIT && !REDO && p.want_colsum && by == 0;
     float cs = 0.f;
     // the columns a thread stores are the same in every row it stores
     static_assert(NT % (TN / 4) == 0, "a thread's columns");
@@ -392,7 +393,13 @@ __device__ __forceinline__ void small_tile(const GemmArgs& p, int bx, int by, in
         } else {
             dst = p.c + (size_t)m * p.ldc + sn;
         }
-        if (p.c_vec && sn + 3 < p.n) {
+        if constexpr (REDO) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)  // (stored by other lanes: read past the L1)
+                if (sn + q < p.n &&
+                    !__builtin_isfinite(__hip_atomic_load(dst + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+                    dst[q] = c[q];
+        } else if (p.c_vec && sn + 3 < p.n) {
             *reinterpret_cast<float4*>(dst) = make_float4(c[0], c[1], c[2], c[3]);
         } else {
 #pragma unroll

@@ -29,10 +29,13 @@
 // 129, k = 387: 58 -> 46; 19200 x 1533, k = 511: 308 -> 190; the pair 387 x (129 +
 // 129), k = 32768: 155 -> 115; 993 x (331 + 331), k = 8192: 152 -> 83.
 //
-// Non-finite values: the pieces of an infinity are not finite sums, so an output
-// that comes out infinite or NaN is computed again as a plain float32 dot
-// product by the lane that stored it (split_redo); finite results are never
-// touched.
+// Non-finite values: the pieces of an infinity are not finite sums, so a workgroup
+// one of whose outputs comes out infinite or NaN computes its tile again in 64x64
+// fp32 tiles (gemm_small.h) and replaces those outputs; finite results are never
+// touched.  Where every output is NaN (after a diverged step, or an aborted
+// recurrence) a product takes both forms' time: 32768 x 768, k = 256 256 us
+// against 86; a training pass at batch 64, 512 steps, I = H = 256 1.26 ms against
+// 1.15 (11.4 and 17.4 ms when each lane went over its outputs one by one).
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -245,14 +248,19 @@ struct SplitShiftLoader {
     static __device__ __forceinline__ int kshift(int, int) { return 0; }
 };
 
-// An output as a plain float32 dot product over k in [kbeg, kbeg + klen).
-template <int AK, int BKM, bool SHIFT>
-__device__ __forceinline__ float split_dot(const GemmArgs& p, int m, int n, int kbeg, int klen) {
-    float s = 0.f;
+// The tile (bx, by) again in fp32, for the outputs that are not finite.
+template <int AK, int BKM, bool SPLIT, bool SHIFT, bool UA>
+__device__ __forceinline__ void split_redo(const GemmArgs& p, int bx, int by, int bz, unsigned* smem) {
+    using S = SmallTile<64, 64, 32, 32, 16>;
+    static_assert(S::smem<AK, BKM>() <= 2 * kSplitStage, "fits the stages' memory");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wavefront's outputs are stored
 #pragma unroll 1
-    for (int k = kbeg; k < kbeg + klen; ++k)
-        s = fmaf(*elem_ptr<AK, false, false>(p.a, m, k), *elem_ptr<BKM, SHIFT, false>(p.b, n, k), s);
-    return s;
+    for (int q = 0; q < 4; ++q) {
+        __syncthreads();
+        const int sx = 2 * bx + (q & 1), sy = 2 * by + (q >> 1);
+        if (S::TM * sx < p.m && S::TN * sy < p.n)
+            small_tile<AK, BKM, S, !UA, SPLIT, SHIFT, true>(p, sx, sy, bz, reinterpret_cast<float*>(smem));
+    }
 }
 
 // One 128x128 tile (bx, by); SPLIT: the partial products of k slice bz, with the
@@ -269,6 +277,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
     const int klen = SPLIT ? max(0, min(p.k - kbeg, p.kchunk)) : p.k;
     const int nkb = (klen + 15) / 16;
     const bool colsum = SPLIT && p.want_colsum && by == 0;
+    __shared__ int s_odd;  // an output is not finite
+    if (tid == 0) s_odd = 0;
     float4 cs = make_float4(0.f, 0.f, 0.f, 0.f);
 
     using LA = SplitLoader<AK, UA>;
@@ -417,20 +427,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
                 }
             }
         }
-    if (__builtin_expect(__any(odd), 0)) {
-        // the lane reads back what it stored (past the L1) and replaces what is
-        // not finite
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll 1
-        for (int e = 0; e < 64; ++e) {
-            const int m = row_of(e >> 5, (e >> 1) & 15), n = col_of(e & 1);
-            if (m >= p.m || n >= p.n) continue;
-            float* at = dst_of(m) + n;
-            const float old = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (!__builtin_isfinite(old))
-                *at = split_dot<AK, BKM, SHIFT>(p, m, n, kbeg, klen) + (!SPLIT && p.bias ? p.bias[n] : 0.f);
-        }
-    }
+    if (__any(odd) && lane == 0) s_odd = 1;
     if constexpr (SPLIT) {
         if (colsum) {
             // rows 4 (tid % 32) .. + 3 from the eight threads that share them
@@ -450,6 +447,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
             }
         }
     }
+    __syncthreads();
+    if (__builtin_expect(s_odd != 0, 0)) split_redo<AK, BKM, SPLIT, SHIFT, UA>(p, bx, by, bz, smem);
 }
 
 template <int BKM, bool UA>
