@@ -79,8 +79,9 @@ int rka_gru_forward(const float* x, const float* h0,
  * Inference through a stack of layers (layer 0 takes x, each later one the
  * previous layer's output): rka_gru_forward without a gate cache, layer by
  * layer, with one workspace.  h0 and hn are [num_layers,B,H], y the last
- * layer's output [B,T,H]; weights holds w_ih, w_hh, b_ih, b_hh of each layer
- * in order (4 num_layers pointers, read on the host during the call).
+ * layer's output [B,T,H] (earlier layers' outputs pass through it too); weights
+ * holds w_ih, w_hh, b_ih, b_hh of each layer in order (4 num_layers pointers,
+ * read on the host during the call).
  */
 size_t rka_gru_stack_forward_workspace_bytes(int num_layers, int batch, int seq_len, int input_size, int hidden_size);
 int rka_gru_stack_forward(int num_layers, const float* x, const float* h0, const float* const* weights,

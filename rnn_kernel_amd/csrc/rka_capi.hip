@@ -71,18 +71,16 @@ FwdLayout fwd_layout(int B, int T, int I, int H) {
     return l;
 }
 
-// Workspace of a stack: the layers' own (shared), then the outputs of the
-// layers before the last, two in turn.
+// Workspace of a stack: the layers' own (shared), then one layer output: the
+// layers write to it and to the call's own output in turn, the last one to that.
 struct StackLayout {
-    size_t layer, y[2], total;
+    size_t layer, y, total;
 };
 StackLayout stack_layout(int L, int B, int T, int I, int H) {
     StackLayout l{};
     l.layer = fwd_layout(B, T, I, H).total;
-    const size_t y = align_up((size_t)B * T * H * sizeof(float), 256);
-    l.y[0] = align_up(l.layer, 256);
-    l.y[1] = l.y[0] + y;
-    l.total = l.y[0] + (size_t)std::min(L - 1, 2) * y;
+    l.y = align_up(l.layer, 256);
+    l.total = l.y + (L > 1 ? align_up((size_t)B * T * H * sizeof(float), 256) : 0);
     return l;
 }
 
@@ -248,7 +246,7 @@ int rka_gru_stack_forward(int num_layers, const float* x, const float* h0, const
     const size_t state = (size_t)batch * hidden_size;
     const float* in = x;
     for (int k = 0; k < num_layers; ++k) {
-        float* out = k + 1 == num_layers ? y : reinterpret_cast<float*>(ws + l.y[k & 1]);
+        float* out = (num_layers - 1 - k) % 2 == 0 ? y : reinterpret_cast<float*>(ws + l.y);
         const float* const* w = weights + 4 * k;
         RKA_RETURN_IF_ERR(rka_gru_forward(in, h0 + k * state, w[0], w[1], w[2], w[3], out, hn + k * state, nullptr, ws,
                                           l.layer, batch, seq_len, k == 0 ? input_size : hidden_size, hidden_size,

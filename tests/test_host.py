@@ -95,6 +95,16 @@ def test_backward_workspace_holds_gate_gradients_exchange_and_partials(hip_lib):
     assert need > g_bytes + hip_lib.rka_gru_recurrence_workspace_bytes(B, H) + 2 * 3 * H * H * 4
 
 
+@pytest.mark.parametrize("layers", [1, 2, 3, 4, 7])
+def test_stack_workspace_holds_one_layer_output(hip_lib, layers):
+    """Inference through a stack takes, beside the call's own output, what two
+    layers called one after the other take: a layer's workspace and one output."""
+    B, T, I, H = 32, 100, 48, 64
+    need = hip_lib.rka_gru_stack_forward_workspace_bytes(layers, B, T, I, H)
+    output = B * T * H * 4 if layers > 1 else 0
+    assert need <= hip_lib.rka_gru_forward_workspace_bytes(B, T, I, H) + output + 2 * 256
+
+
 def test_module_construction_and_validation_messages():
     from rnn_kernel_amd import GRU, MAX_HIDDEN_SIZE
 
