@@ -3,6 +3,7 @@
 // in rec_reg_kernels.h).
 #include "rec_reg_kernels.h"
 
+#include <algorithm>
 #include <atomic>
 
 namespace rka {
@@ -76,7 +77,7 @@ int block_threads(int dir, int rows, int slices) {
 // The local-slice kernels: S slices, 1, 2 or 4 batch rows per workgroup.
 // full: H = 64 * slices (the one-row forward has instances for it); stage:
 // the forward reads W_hh through LDS.
-const void* kernel_ptr(int dir, int cap, int rows, int slices, bool full = false, bool stage = true) {
+const void* kernel_ptr(int dir, int cap, int rows, int slices, bool full, bool stage) {
     (void)cap;
     const bool io = uses_io(dir, rows, slices);
     switch (slices) {
@@ -87,19 +88,24 @@ const void* kernel_ptr(int dir, int cap, int rows, int slices, bool full = false
     }
 }
 
-// Workgroups of the kernel that a CU holds (-1: the query failed), asked once
-// per device and kernel (a query takes about a microsecond of every call).
+// Workgroups that a CU holds of any instance that reg_launch may take for these
+// rows and slices (-1: a query failed), asked once per device (a query takes about
+// a microsecond of every call).
 int blocks_per_cu(int device, int dir, int cap, int rows, int slices) {
     static std::atomic<int> known[16][2][3][4];  // the answer + 1
     std::atomic<int>* k =
         device >= 0 && device < 16 ? &known[device][dir][rows == 1 ? 0 : rows == 2 ? 1 : 2][slices - 1] : nullptr;
     if (k != nullptr && k->load(std::memory_order_relaxed) > 0) return k->load(std::memory_order_relaxed) - 1;
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel_ptr(dir, cap, rows, slices),
-                                                     block_threads(dir, rows, slices), 0) != hipSuccess)
-        return -1;
-    if (k != nullptr) k->store(per_cu + 1, std::memory_order_relaxed);
-    return per_cu;
+    int least = 0;
+    for (int form = 0; form < 4; ++form) {
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel_ptr(dir, cap, rows, slices, form & 1, form & 2),
+                                                         block_threads(dir, rows, slices), 0) != hipSuccess)
+            return -1;
+        least = form == 0 ? per_cu : std::min(least, per_cu);
+    }
+    if (k != nullptr) k->store(least + 1, std::memory_order_relaxed);
+    return least;
 }
 
 // Units per workgroup and whether the register-resident kernels hold H.
