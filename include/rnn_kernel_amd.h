@@ -189,6 +189,21 @@ int rka_gru_recurrence_backward(const float* dy, const float* dhn,
 #define RKA_GEMM_TILES_128 1
 int rka_set_gemm_tiles(int mode);
 
+/* The form that products take in the present tile mode (host only: no GPU is
+ * asked), for tests and tuning.  rka_describe_gemm: a rka_gemm_f32 call of this
+ * size, `aligned` telling whether the contiguous dimension of both operands is
+ * whole aligned float4.  rka_describe_weight_gradients: the pair dW_hh, dW_ih of
+ * rka_gru_backward; writes the first min(n_out, 4) of {form, k-slices of dW_hh, of
+ * dW_ih, 1 if its launch writes the results itself}.  No counterpart in the
+ * reference (its products are cuBLAS calls). */
+#define RKA_GEMM_FORM_RING 0   /* 128x128 tiles, fp32 matrix cores */
+#define RKA_GEMM_FORM_SPLIT 1  /* 128x128 tiles, three bf16 pieces per value */
+#define RKA_GEMM_FORM_128X64 2 /* register-staged tiles, fp32 matrix cores */
+#define RKA_GEMM_FORM_64X64 3
+#define RKA_GEMM_FORM_32X32 4
+int rka_describe_gemm(int m, int n, int k, int a_kmajor, int aligned, int* form);
+int rka_describe_weight_gradients(int batch, int seq_len, int input_size, int hidden_size, int* out, int n_out);
+
 /* Poll rounds a recurrence kernel's wait for another workgroup's words
  * makes before it gives up (0 = the default, 2^24 rounds, about 2 s at the
  * fastest poll rate; at most 2^30).  Every recurrence grid is resident, so
@@ -243,8 +258,9 @@ int rka_recurrence_abort_count(unsigned long long* count);
  * 1 backward); affects later calls on all threads.  For tuning and tests.
  * kind 0: automatic (register-resident kernel when hidden_size <= 256, with
  *         the fewest batch rows per workgroup whose grid is resident, else
- *         four rows and one resident launch per batch slice; LDS-tiled
- *         above 256);
+ *         four rows and one resident launch per batch slice; four rows and 32
+ *         units per workgroup for 257 to 768, likewise; LDS-tiled above, or
+ *         where the others' grid is not resident);
  * kind 1: LDS-tiled; units = hidden units per workgroup (a divisor of 64,
  *         0 = auto), param = wavefronts holding (row, unit) pairs (1, 2, 4,
  *         0 = auto);

@@ -38,6 +38,8 @@ SIGNATURES = {
     "rka_set_recurrence_config": (_I, [_I, _I, _I, _I]),
     "rka_set_spin_limit": (_I, [_I]),
     "rka_set_gemm_tiles": (_I, [_I]),
+    "rka_describe_gemm": (_I, [_I, _I, _I, _I, _I, ctypes.POINTER(_I)]),
+    "rka_describe_weight_gradients": (_I, [_I, _I, _I, _I, ctypes.POINTER(_I), _I]),
     "rka_set_exchange_stores": (_I, [_I]),
     "rka_recurrence_abort_count": (_I, [ctypes.POINTER(ctypes.c_ulonglong)]),
     "rka_set_stall_block": (_I, [_I]),
@@ -179,6 +181,26 @@ def set_gemm_tiles(mode: int) -> None:
     """GEMM tile families: 0 = automatic (smaller tiles where 128x128
     would fill the CUs unevenly), 1 = 128x128 everywhere; see rka_set_gemm_tiles."""
     check(load().rka_set_gemm_tiles(mode), "rka_set_gemm_tiles")
+
+
+GEMM_FORMS = {0: "ring", 1: "split", 2: "128x64", 3: "64x64", 4: "32x32"}
+
+
+def describe_gemm(m: int, n: int, k: int, aligned: bool, a_kmajor: bool = False) -> str:
+    """Form a product of this size takes in the present tile mode; see
+    rka_describe_gemm."""
+    form = ctypes.c_int(0)
+    check(load().rka_describe_gemm(m, n, k, int(a_kmajor), int(aligned), ctypes.byref(form)), "rka_describe_gemm")
+    return GEMM_FORMS[form.value]
+
+
+def describe_weight_gradients(batch: int, seq_len: int, input_size: int, hidden: int) -> dict:
+    """Form and k-slices of a backward's weight-gradient pair in the present
+    tile mode; see rka_describe_weight_gradients."""
+    out = (ctypes.c_int * 4)()
+    check(load().rka_describe_weight_gradients(batch, seq_len, input_size, hidden, out, 4),
+          "rka_describe_weight_gradients")
+    return dict(form=GEMM_FORMS[out[0]], slices_hh=out[1], slices_ih=out[2], direct=bool(out[3]))
 
 
 def set_exchange_stores(mode: int) -> None:

@@ -1106,7 +1106,13 @@ std::atomic<int> g_gemm_tiles{RKA_GEMM_TILES_AUTO};
 bool split_takes(int m, int n, int k) { return m >= 4 && n >= 4 && k >= 4; }
 
 // Tiles a direct product runs in.
-enum DirectTile { TILE_128, TILE_SPLIT, TILE_128x64, TILE_64, TILE_32 };
+enum DirectTile {
+    TILE_128 = RKA_GEMM_FORM_RING,
+    TILE_SPLIT = RKA_GEMM_FORM_SPLIT,
+    TILE_128x64 = RKA_GEMM_FORM_128X64,
+    TILE_64 = RKA_GEMM_FORM_64X64,
+    TILE_32 = RKA_GEMM_FORM_32X32
+};
 using Tile128x64 = SmallTile<128, 64, 64, 32, 16>;
 using Tile64 = SmallTile<64, 64, 32, 32, 16>;
 using Tile32 = SmallTile<32, 32, 32, 32, 64>;
@@ -1215,6 +1221,16 @@ int set_gemm_tiles(int mode) {
         return fail(RKA_ERR_INVALID_ARGUMENT, "rka_set_gemm_tiles: mode must be 0 or 1");
     g_gemm_tiles.store(mode);
     return 0;
+}
+
+int describe_direct(int m, int n, int k, bool a_kmajor, bool aligned) {
+    GemmArgs args{};
+    args.a.kmajor = a_kmajor ? 1 : 0;
+    args.a_vec = args.b_vec = aligned ? 1 : 0;
+    args.m = m;
+    args.n = n;
+    args.k = k;
+    return direct_tile(args);
 }
 
 int gemm_direct(int m, int n, int k, const GemmOperand& a, const GemmOperand& b,

@@ -382,6 +382,24 @@ int rka_set_gemm_tiles(int mode) {
     return set_gemm_tiles(mode);
 }
 
+int rka_describe_gemm(int m, int n, int k, int a_kmajor, int aligned, int* form) {
+    clear_error();
+    if (m <= 0 || n <= 0 || k < 0 || !form)
+        return fail(RKA_ERR_INVALID_ARGUMENT, "rka_describe_gemm: m and n must be positive, form non-NULL");
+    *form = describe_direct(m, n, k, a_kmajor != 0, aligned != 0);
+    return 0;
+}
+
+int rka_describe_weight_gradients(int batch, int seq_len, int input_size, int hidden_size, int* out, int n_out) {
+    clear_error();
+    if (!out || n_out < 1) return fail(RKA_ERR_INVALID_ARGUMENT, "out must be non-NULL and n_out >= 1");
+    RKA_RETURN_IF_ERR(check_dims(batch, seq_len, input_size, hidden_size));
+    const PairPlan p = plan_pair(3 * hidden_size, hidden_size, input_size, batch * seq_len);
+    const int v[4] = {p.form, p.ks0, p.ks1, p.direct ? 1 : 0};
+    for (int i = 0; i < 4 && i < n_out; ++i) out[i] = v[i];
+    return 0;
+}
+
 int rka_set_spin_limit(int polls) {
     clear_error();
     if (polls < 0 || polls > kMaxSpinPolls)

@@ -104,7 +104,12 @@ struct SplitProduct {
 // How the weight-gradient pair of a backward call runs.  Taken once per call
 // (plan_pair reads the tile mode of rka_set_gemm_tiles, which another thread may
 // change meanwhile) and handed to the pair's launch and to its reduction.
-enum PairForm { PAIR_RING, PAIR_64, PAIR_128x64, PAIR_SPLIT };
+enum PairForm {
+    PAIR_RING = RKA_GEMM_FORM_RING,
+    PAIR_SPLIT = RKA_GEMM_FORM_SPLIT,
+    PAIR_128x64 = RKA_GEMM_FORM_128X64,
+    PAIR_64 = RKA_GEMM_FORM_64X64
+};
 struct PairPlan {
     PairForm form;
     int ks0, ks1;  // k-slices of the two products
@@ -128,6 +133,8 @@ int gemm_direct_reduce_pair(int m, int n, int k, const GemmOperand& a, const Gem
                             const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan, hipStream_t stream);
 // rka_set_gemm_tiles (RKA_GEMM_TILES_AUTO or RKA_GEMM_TILES_128).
 int set_gemm_tiles(int mode);
+// The form (RKA_GEMM_FORM_...) a direct product takes in the present tile mode.
+int describe_direct(int m, int n, int k, bool a_kmajor, bool aligned);
 // Slices for a split-K product of about wgs_per_cu workgroups per CU
 // (0: half a workgroup per CU, for products that share the GPU with a
 // concurrently running recurrence); a multiple of 8 from 8 up.

@@ -1,14 +1,14 @@
-"""The direct products' tile forms (128x128 ring, 128x64, 64x64 and 32x32
-register-staged tiles) against float64 at the edges of each, and the rule
-between them on aligned and unaligned storage."""
+"""The direct products' fp32 tile forms (128x128 ring, 128x64, 64x64 and 32x32
+register-staged tiles) against float64 at the edges of each, on aligned and
+unaligned storage.  The ring takes row-major products under
+RKA_GEMM_TILES_128 only."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
-# m, n, k: 32x32 tiles with one row, partial tiles, k below, at and past one
-# and two 64-deep stages; 64x64 and 128x64 tiles (more than one tile per CU, the
-# last ones partial; k of one, two, three and a partial 16-deep stage)
+# m, n, k: 32x32 tiles (one row, partial tiles, k below, at and past one and two
+# 64-deep stages, several tiles per CU) and, at (8200, 192, 32), 128x64 ones
 SHAPES = [(1, 768, 256), (1, 1, 3), (33, 31, 64), (31, 65, 65), (200, 96, 128), (64, 100, 130), (50, 40, 4),
           (8192, 130, 16), (8200, 192, 32), (8192, 188, 52), (16500, 129, 17), (33000, 65, 33)]
 
@@ -17,6 +17,34 @@ SHAPES = [(1, 768, 256), (1, 1, 3), (33, 31, 64), (31, 65, 65), (200, 96, 128), 
 @pytest.mark.parametrize("b_kmajor", [0, 1])
 @pytest.mark.parametrize("pad", [0, 1])  # floats between rows and before the first: not 16-byte aligned
 def test_direct_product_tiles_match_float64(gpu, hip_lib, m, n, k, b_kmajor, pad):
+    _check_direct(gpu, hip_lib, m, n, k, b_kmajor, pad)
+
+
+# tile mode, form, floats between rows and before the first, m, n, k: the last
+# tiles partial along m and n; k of less than one 16-deep stage, of one, two, a part
+# more and of many
+FORMS = [(0, "64x64", 0, 12600, 36, 4), (0, "64x64", 0, 16400, 252, 36), (0, "64x64", 0, 8300, 512, 256),
+         (0, "64x64", 1, 13657, 33, 1), (0, "64x64", 1, 16385, 255, 34), (0, "64x64", 1, 8200, 513, 387),
+         (0, "128x64", 0, 24612, 36, 4), (0, "128x64", 0, 8200, 192, 32), (0, "128x64", 0, 8196, 188, 260),
+         (0, "128x64", 1, 26747, 35, 1), (0, "128x64", 1, 24613, 37, 33),
+         (1, "ring", 0, 1, 4, 4), (1, "ring", 0, 300, 200, 52), (1, "ring", 0, 1028, 388, 16),
+         (1, "ring", 1, 31, 65, 65), (1, "ring", 1, 1000, 390, 70), (1, "ring", 1, 129, 1, 3)]
+
+
+@pytest.mark.parametrize("mode,form,pad,m,n,k", FORMS)
+@pytest.mark.parametrize("b_kmajor", [0, 1])
+def test_direct_product_forms_match_float64(gpu, hip_lib, mode, form, pad, m, n, k, b_kmajor):
+    from rnn_kernel_amd import _lib
+
+    try:
+        _lib.set_gemm_tiles(mode)
+        assert _lib.describe_gemm(m, n, k, aligned=pad == 0) == form
+        _check_direct(gpu, hip_lib, m, n, k, b_kmajor, pad)
+    finally:
+        _lib.set_gemm_tiles(0)
+
+
+def _check_direct(gpu, hip_lib, m, n, k, b_kmajor, pad):
     from rnn_kernel_amd import _lib
 
     print(f"direct m={m} n={n} k={k} b_kmajor={b_kmajor} pad={pad}", flush=True)

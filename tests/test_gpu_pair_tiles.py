@@ -1,9 +1,10 @@
-"""The weight-gradient products where their tile or number of slices changes,
+"""The weight-gradient products where their form or number of slices changes,
 against float64 sums of the gate gradients that the library itself returns:
 one slice (the results written by the products' own launch), few, and a
 multiple of 8; sequences shorter than a 16-deep stage and of one step (the
 [h0 ; y[:, :-1]] rows); a last slice shorter than the others; aligned and
-unaligned rows; 64x64 and 128x64 tiles and the ring."""
+unaligned rows; 64x64, 128x64 and split tiles, and under RKA_GEMM_TILES_128 the
+ring with its narrow last columns."""
 import threading
 
 import pytest
@@ -19,6 +20,35 @@ SHAPES = [(1, 1, 1, 1), (2, 3, 5, 7), (127, 1, 16, 20), (128, 1, 12, 64), (9, 14
 @pytest.mark.parametrize("B,T,I,H", SHAPES)
 @pytest.mark.parametrize("need_dx", [True, False])
 def test_weight_gradients_match_float64(gpu, hip_lib, B, T, I, H, need_dx):
+    _check_pair(gpu, hip_lib, B, T, I, H, need_dx)
+
+
+# tile mode, form, whether one launch writes the results, B, T, I, H.  The ring: one
+# tile, several, 5, 7 and 8 last columns summed apart (in 32 slices and in one), the
+# remainder just too wide for that
+FORMS = [(0, "64x64", True, 3, 5, 4, 4), (0, "64x64", False, 21, 25, 36, 68), (0, "64x64", False, 23, 47, 35, 67),
+         (0, "128x64", False, 99, 376, 2, 66), (0, "split", False, 16, 129, 204, 584),
+         (0, "split", False, 15, 52, 595, 342), (0, "split", False, 121, 149, 5, 65),
+         (1, "ring", False, 3, 5, 4, 4), (1, "ring", False, 9, 14, 33, 65), (1, "ring", False, 40, 25, 64, 128),
+         (1, "ring", False, 8, 512, 135, 133), (1, "ring", False, 2, 70, 136, 136), (1, "ring", False, 3, 50, 137, 140),
+         (1, "ring", False, 7, 300, 129, 129)]
+
+
+@pytest.mark.parametrize("mode,form,direct,B,T,I,H", FORMS)
+@pytest.mark.parametrize("need_dx", [True, False])
+def test_weight_gradient_forms_match_float64(gpu, hip_lib, mode, form, direct, B, T, I, H, need_dx):
+    from rnn_kernel_amd import _lib
+
+    try:
+        _lib.set_gemm_tiles(mode)
+        d = _lib.describe_weight_gradients(B, T, I, H)
+        assert (d["form"], d["direct"]) == (form, direct)
+        _check_pair(gpu, hip_lib, B, T, I, H, need_dx)
+    finally:
+        _lib.set_gemm_tiles(0)
+
+
+def _check_pair(gpu, hip_lib, B, T, I, H, need_dx):
     from rnn_kernel_amd import _lib
 
     print(f"pair B={B} T={T} I={I} H={H} dx={need_dx}", flush=True)
@@ -52,8 +82,8 @@ def test_weight_gradients_match_float64(gpu, hip_lib, B, T, I, H, need_dx):
     g_ih = G[:, H:]
     g_hh = torch.cat([G[:, H:3 * H], G[:, :H]], dim=1)
     hprev = torch.cat([h0[:, None], y[:, :-1]], dim=1).double().reshape(B * T, H)
-    # a float32 sum of n products, in chains of at most 4096 and their sum, is
-    # within (4096 + 256) 2^-24 of the sum of the products' magnitudes
+    # a float32 sum of n products, in chains of at most 4096 (to n = 2^20) and their
+    # sum, is within (4096 + 256) 2^-24 of the sum of the products' magnitudes
     n = min(B * T, 4352)
     for name, out, a, b in (("dw_ih", dw_ih, g_ih, x.double().reshape(B * T, I)), ("dw_hh", dw_hh, g_hh, hprev),
                             ("db_ih", db_ih, g_ih, None), ("db_hh", db_hh, g_hh, None)):

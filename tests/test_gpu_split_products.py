@@ -6,10 +6,11 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# m, n, k (enough 128x128 tiles that this form is taken): partial tiles along m and
-# n, k of a part of a stage, one, two and many; then the same without aligned
-# float4 rows, where loads that would cross an operand's end start earlier: a last
-# tile of one to three columns, last stages of one to three and more k
+# m, n, k: partial tiles along m and n, k of a part of a stage, one, two and many;
+# then the same without aligned float4 rows, where loads that would cross an
+# operand's end start earlier.  (16400, 252, 36), (8300, 512, 256), (16385, 255, 34),
+# (8300, 510, 129) and (8200, 513, 387) take fp32 64x64 tiles; SPLIT_SHAPES below are
+# all of this form
 SHAPES = [(32700, 124, 4), (32768, 128, 16), (32641, 132, 20), (16400, 252, 36), (8300, 512, 256), (16384, 256, 772),
           (32701, 125, 5), (32641, 127, 17), (16385, 255, 34), (8300, 510, 129), (8200, 513, 387), (8257, 643, 63)]
 
@@ -33,6 +34,26 @@ def _product(gpu, hip_lib, a, b, b_kmajor, bias=None):
 @pytest.mark.parametrize("b_kmajor", [0, 1])
 @pytest.mark.parametrize("scale", [1.0, 1e-30, 1e15])
 def test_split_product_error(gpu, hip_lib, m, n, k, b_kmajor, scale):
+    _check_error(gpu, hip_lib, m, n, k, b_kmajor, scale)
+
+
+# aligned: two columns of tiles, the last of 4 to 132 columns; unaligned: a last
+# tile of one, two, three and more columns (and rows), k of many stages that end with
+# one, two, three and more values
+SPLIT_SHAPES = [(32641, 132, 772), (16384, 388, 260), (32765, 128, 1028),
+                (32641, 129, 257), (32642, 130, 242), (32643, 131, 243), (32767, 257, 401), (32765, 387, 513)]
+
+
+@pytest.mark.parametrize("m,n,k", SPLIT_SHAPES)
+@pytest.mark.parametrize("b_kmajor", [0, 1])
+def test_split_product_edges(gpu, hip_lib, m, n, k, b_kmajor):
+    from rnn_kernel_amd import _lib
+
+    assert _lib.describe_gemm(m, n, k, aligned=n % 4 == 0 and k % 4 == 0) == "split"
+    _check_error(gpu, hip_lib, m, n, k, b_kmajor, 1.0)
+
+
+def _check_error(gpu, hip_lib, m, n, k, b_kmajor, scale):
     print(f"split m={m} n={n} k={k} b_kmajor={b_kmajor} scale={scale}", flush=True)
     g = torch.Generator(device=gpu).manual_seed(m + n + k)
     a = scale * torch.randn(m, k, generator=g, device=gpu)
@@ -43,8 +64,9 @@ def test_split_product_error(gpu, hip_lib, m, n, k, b_kmajor, scale):
     bd = b.double() if b_kmajor else b.double().t().contiguous()
     ref = a.double() @ bd + bias.double()
     mag = a.double().abs() @ bd.abs() + bias.double().abs()
-    # six float32 roundings per 16-deep stage and the left-out 2^-25; a piece or a
-    # product of two below the normal range (2^-126) may count as zero
+    # six float32 roundings per 16-deep stage and the left-out products of pieces
+    # (2^-24); the least normal value for each product and operand besides (looser
+    # than need be, see test_split_product_of_small_magnitudes)
     stages = (k + 15) // 16
     tiny = 2.0 ** -126 * (6 * k + a.double().abs().sum(1, keepdim=True) + bd.abs().sum(0))
     assert bool(((c.double() - ref).abs() <= (6 * stages + 4) * 2.0 ** -24 * mag + tiny).all())

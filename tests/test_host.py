@@ -105,6 +105,35 @@ def test_stack_workspace_holds_one_layer_output(hip_lib, layers):
     assert need <= hip_lib.rka_gru_forward_workspace_bytes(B, T, I, H) + output + 2 * 256
 
 
+def test_listed_products_take_the_forms_they_are_listed_for(hip_lib):
+    """The GPU tests' products by form, and every form among them."""
+    import test_gpu_gemm_tiles as direct
+    import test_gpu_pair_tiles as pairs
+    import test_gpu_split_products as split
+    from rnn_kernel_amd import _lib
+
+    try:
+        for mode, form, pad, m, n, k in direct.FORMS:
+            _lib.set_gemm_tiles(mode)
+            assert _lib.describe_gemm(m, n, k, aligned=pad == 0) == form, (m, n, k)
+        for mode, form, one_launch, *size in pairs.FORMS:
+            _lib.set_gemm_tiles(mode)
+            d = _lib.describe_weight_gradients(*size)
+            assert (d["form"], d["direct"]) == (form, one_launch), size
+    finally:
+        _lib.set_gemm_tiles(0)
+    for m, n, k in split.SPLIT_SHAPES:
+        assert _lib.describe_gemm(m, n, k, aligned=n % 4 == 0 and k % 4 == 0) == "split", (m, n, k)
+    assert all(_lib.describe_gemm(m, n, k, aligned=False) == "32x32" for m, n, k in direct.SHAPES if n != 192)
+    assert {f[1] for f in direct.FORMS} == {"ring", "128x64", "64x64"}
+    assert {f[1] for f in pairs.FORMS} == {"ring", "split", "128x64", "64x64"}
+    form = ctypes.c_int(0)
+    assert hip_lib.rka_describe_gemm(0, 1, 1, 0, 0, ctypes.byref(form)) == 1001
+    assert hip_lib.rka_describe_gemm(1, 1, 1, 0, 0, None) == 1001
+    assert hip_lib.rka_describe_weight_gradients(1, 1, 1, 0, ctypes.byref(form), 1) == 1001
+    assert hip_lib.rka_describe_weight_gradients(1, 1, 1, 1, ctypes.byref(form), 0) == 1001
+
+
 def test_module_construction_and_validation_messages():
     from rnn_kernel_amd import GRU, MAX_HIDDEN_SIZE
 
