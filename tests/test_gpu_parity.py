@@ -244,7 +244,7 @@ LAYER_SHAPES = [
     (300, 3, 8, 256),    # B x 4 workgroups not resident: four rows per workgroup, two batch-slice launches
     (130, 4, 6, 130),    # three slices, two rows per workgroup
     (400, 5, 4, 160),    # three slices at four rows not resident: batch-slice launches of 80 groups
-    (1, 3, 4, 768),      # the largest hidden size at one batch row (LDS-tiled, one unit per workgroup)
+    (1, 3, 4, 768),      # the largest hidden size at one batch row
     (8, 512, 135, 133),  # weight gradients in several partial 64x64 tiles and slices, unaligned
     (2, 70, 136, 136),   # ... aligned, k = 140
 ]
@@ -307,7 +307,7 @@ def agent_stores(hip_lib):
     _lib.set_exchange_stores(0)
 
 
-# register (H <= 256) and tiled (H = 512) recurrences; G = 1, 3, 4, 5 and 64 groups
+# register (H <= 256) and wide (H = 512) recurrences; G = 1, 2, 3, 4 and 64 groups
 AGENT_SHAPES = [(1, 5, 8, 256), (3, 5, 7, 130), (4, 6, 8, 256), (5, 4, 8, 512), (64, 4, 16, 256)]
 
 
@@ -316,6 +316,20 @@ def test_layer_with_agent_scope_exchange_matches_oracle(gpu, oracle, agent_store
     """Every launch publishes with agent-scope stores (the path a group whose
     workgroups span XCDs takes): the layer still matches the oracle."""
     _check_layer_against_oracle(gpu, oracle, agent_stores, B, T, I, H)
+
+
+def test_tiled_layer_with_agent_scope_exchange_matches_oracle(gpu, oracle, agent_stores):
+    """The same for the LDS-tiled kernels, which the automatic choice leaves to
+    grids the others cannot hold resident."""
+    from rnn_kernel_amd import _lib
+
+    try:
+        for d in (0, 1):
+            _lib.set_recurrence_config(d, 1, 0, 0)
+        _check_layer_against_oracle(gpu, oracle, agent_stores, 5, 4, 8, 512)
+    finally:
+        for d in (0, 1):
+            _lib.set_recurrence_config(d, 0, 0, 0)
 
 
 @pytest.mark.parametrize("B,T,I,H", AGENT_SHAPES)

@@ -33,7 +33,7 @@ def _ptr(t):
 #   c2-like one-row launch, then a small odd shape;
 #   at the static limit (B H = 262144): B = 1024 at H = 256 runs the register
 #   kernel as several batch-slice launches (the last slice's words end at the
-#   array's end), H = 512 the LDS-tiled kernel; then the small odd shape
+#   array's end), H = 512 the wide kernel; then the small odd shape
 SEQUENCES = [
     ((64, 40, 256, 1), (5, 7, 130, 2)),
     ((1024, 6, 256, 3), (512, 5, 512, 4), (5, 7, 130, 5)),
@@ -43,6 +43,20 @@ SEQUENCES = [
 @pytest.mark.parametrize("with_reserve", [True, False])
 @pytest.mark.parametrize("sequence", SEQUENCES)
 def test_noalloc_forward_matches_workspace_forward(gpu, hip_lib, with_reserve, sequence):
+    _check_sequence(gpu, hip_lib, with_reserve, sequence)
+
+
+def test_noalloc_tiled_forward_matches_workspace_forward(gpu, hip_lib):
+    from rnn_kernel_amd import _lib
+
+    try:
+        _lib.set_recurrence_config(0, 1, 0, 0)  # LDS-tiled
+        _check_sequence(gpu, hip_lib, True, ((512, 5, 512, 4), (5, 7, 130, 5)))
+    finally:
+        _lib.set_recurrence_config(0, 0, 0, 0)
+
+
+def _check_sequence(gpu, hip_lib, with_reserve, sequence):
     from rnn_kernel_amd import _lib
 
     stream = torch.cuda.current_stream().cuda_stream
