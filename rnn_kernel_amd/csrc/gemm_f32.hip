@@ -3,7 +3,8 @@
 //   large products: 128x128 tiles, each value in three bf16 pieces (gemm_split.h);
 //   those that would fill the CUs unevenly: register-staged tiles of 32x32 to
 //   128x64 on v_mfma_f32_16x16x4_f32 (gemm_small.h);
-//   the rest: the 128x128 ring below.
+//   products of a k-major A, and under RKA_GEMM_TILES_128 every product that the
+//   rule gives no split tiles: the 128x128 ring below.
 //
 // The products of a layer are
 //   input projection  Gx  = X W_ih^T + b_ih        (A row-major, B row-major)
@@ -55,40 +56,15 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // Address of element (row r, k) of an operand whose layout is fixed at
 // compile time: KMAJOR 0 = element (r,k) at ptr[r*ld+k], 1 = at ptr[k*ld+r].
 // SHIFT: the [h0 ; y[:, :-1]] row remap of the dW_hh B operand (k = b*T + t
-// reads row k-1 for t > 0 and row b of shift_first for t == 0).  SEG: the
-// products of one backward time chunk (SegMap rows).  Compiled per layout so
-// that no product carries the others' address arithmetic or branches.
-template <bool SEG>
-__device__ __forceinline__ int seg_map(const SegMap& s, int i) {
-    if constexpr (!SEG) return i;
-    return s.len ? (i / s.len) * s.stride + s.off + i % s.len : i;
-}
-
-__device__ __forceinline__ const float* uniform_ptr(const float* p) {
-    const unsigned long long v = reinterpret_cast<uintptr_t>(p);
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
-    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-    return reinterpret_cast<const float*>(((unsigned long long)hi << 32) | lo);
-}
-
-template <int KMAJOR, bool SHIFT, bool SEG>
+// reads row k-1 for t > 0 and row b of shift_first for t == 0).  Compiled per
+// layout so that no product carries the others' address arithmetic or branches.
+template <int KMAJOR, bool SHIFT>
 __device__ __forceinline__ const float* elem_ptr(const GemmOperand& op, int r, int k) {
     if constexpr (KMAJOR == 0) {
-        return op.ptr + (size_t)seg_map<SEG>(op.seg, r) * op.ld + k;
+        return op.ptr + (size_t)r * op.ld + k;
     } else {
-        k = seg_map<SEG>(op.seg, k);
         if constexpr (SHIFT) {
-            const int t = k % op.shift_T;
-            if constexpr (SEG) {
-                // The chunked products pick the base from the two pointers
-                // read as wave-uniform values: picking between the two fields
-                // made the compiler copy both into a private array indexed
-                // per lane (scratch loads).
-                const float* first = uniform_ptr(op.shift_first);
-                const float* rest = uniform_ptr(op.ptr);
-                return t == 0 ? first + (size_t)(k / op.shift_T) * op.ld + r : rest + (size_t)(k - 1) * op.ld + r;
-            }
-            if (t == 0) return op.shift_first + (size_t)(k / op.shift_T) * op.ld + r;
+            if (k % op.shift_T == 0) return op.shift_first + (size_t)(k / op.shift_T) * op.ld + r;
             return op.ptr + (size_t)(k - 1) * op.ld + r;
         } else {
             return op.ptr + (size_t)k * op.ld + r;
@@ -128,13 +104,13 @@ constexpr int kDirectBK = 16;
 constexpr int kSplitBK = 16;
 static_assert(BM == 128 && BN == 128 && NT == 256, "tile staging layout");
 
-template <int KMAJOR, bool SHIFT, bool SEG, int BK, int NV4 = BM * BK / (4 * NT), int KQ = BK / 4>
+template <int KMAJOR, bool SHIFT, int BK, int NV4 = BM * BK / (4 * NT), int KQ = BK / 4>
 __device__ __forceinline__ void load_tile(const GemmOperand& op, bool vec, int rows, int kend, int r0, int k0,
                                           int tid, float4 (&v)[NV4]) {
     if (vec && r0 + BM <= rows && k0 + BK <= kend) {
         // interior tile of a vector-capable operand (the common case; the
         // test is uniform): no per-lane bounds checks
-        if constexpr (KMAJOR == 1 && SHIFT && !SEG) {
+        if constexpr (KMAJOR == 1 && SHIFT) {
             // the [h0 ; y[:, :-1]] remap with one division per tile: the
             // thread's rows k, k + NT/32, ... advance t and wrap into the next
             // sequence at t == T
@@ -159,7 +135,7 @@ __device__ __forceinline__ void load_tile(const GemmOperand& op, bool vec, int r
         for (int i = 0; i < NV4; ++i) {
             const int r = KMAJOR == 0 ? r0 + tid / KQ + (NT / KQ) * i : r0 + 4 * (tid % 32);
             const int k = KMAJOR == 0 ? k0 + 4 * (tid % KQ) : k0 + tid / 32 + (NT / 32) * i;
-            v[i] = *reinterpret_cast<const float4*>(elem_ptr<KMAJOR, SHIFT, SEG>(op, r, k));
+            v[i] = *reinterpret_cast<const float4*>(elem_ptr<KMAJOR, SHIFT>(op, r, k));
         }
         return;
     }
@@ -172,7 +148,7 @@ __device__ __forceinline__ void load_tile(const GemmOperand& op, bool vec, int r
         // of four rows).  store_tile writes it back in the same order.  (The
         // float4 order below read four floats 16 bytes apart per lane:
         // 2.3-3x slower GEMMs at hidden size 129.)
-        if constexpr (!SHIFT && !SEG) {
+        if constexpr (!SHIFT) {
             // Element x's address is a wave-uniform base (the element's row or
             // k offset, x / NT, is the same in every lane) plus the lane's
             // offset, which is the same for every element: one VGPR of
@@ -204,13 +180,13 @@ __device__ __forceinline__ void load_tile(const GemmOperand& op, bool vec, int r
                 const int x = (4 * i + c) * NT + tid;
                 const int r = r0 + (KMAJOR == 1 ? x % BM : x / BK);
                 const int k = k0 + (KMAJOR == 1 ? x / BM : x % BK);
-                e[c] = (r < rows && k < kend) ? *elem_ptr<KMAJOR, SHIFT, SEG>(op, r, k) : 0.f;
+                e[c] = (r < rows && k < kend) ? *elem_ptr<KMAJOR, SHIFT>(op, r, k) : 0.f;
             }
             v[i] = make_float4(e[0], e[1], e[2], e[3]);
         }
         return;
     }
-    if constexpr (!SHIFT && !SEG) {
+    if constexpr (!SHIFT) {
         // edge tile of a vector-capable operand: a float4 is entirely in or
         // out (the contiguous extent is a multiple of 4)
         const int lr = KMAJOR == 0 ? tid / KQ : 4 * (tid % 32);
@@ -239,7 +215,7 @@ __device__ __forceinline__ void load_tile(const GemmOperand& op, bool vec, int r
         // The contiguous extent is a multiple of 4 and rows are 16-byte
         // aligned, so a float4 is entirely in or out.
         const bool in = (r < rows) && (k < kend);
-        v[i] = in ? *reinterpret_cast<const float4*>(elem_ptr<KMAJOR, SHIFT, SEG>(op, r, k))
+        v[i] = in ? *reinterpret_cast<const float4*>(elem_ptr<KMAJOR, SHIFT>(op, r, k))
                   : make_float4(0.f, 0.f, 0.f, 0.f);
     }
 }
@@ -310,7 +286,6 @@ struct GemmArgs {
     int tiles_m, tiles;    // output tiles along m, in total
     int ksplit;            // split mode: slices of this launch
     int z_off, ksplit_total;  // split mode: first slice, slices in the buffer
-    SegMap c_seg;          // direct mode: output row map
     unsigned long long* zero;  // direct mode: words cleared on the side (nullable)
     size_t zero_words;
     int rot;               // split mode with c set (one slice): row rotation of c and colsum
@@ -441,7 +416,7 @@ __device__ __forceinline__ void mma_tile(const float* as, const float* bs, int l
 // otherwise both operands take the float4 loads, and the one-float-per-lane
 // code, whose addresses would hold ~40 more VGPRs and cost the aligned
 // kernels their third workgroup per CU, is not compiled in.
-template <int AK, int BKM, bool BSHIFT, bool SEG, int BK, bool UA, bool IDLE = false>
+template <int AK, int BKM, bool BSHIFT, int BK, bool UA, bool IDLE = false>
 __device__ __forceinline__ void mainloop(const GemmArgs& p, int m0, int n0, int kbeg, int kend, int nkb,
                                                  int tid, int lane, int wm, int wn, bool colsum, float& cs,
                                                  float* As0, float* As1, float* Bs0, float* Bs1,
@@ -450,8 +425,8 @@ __device__ __forceinline__ void mainloop(const GemmArgs& p, int m0, int n0, int 
     const bool av = !UA || p.a_vec != 0, bv = !UA || p.b_vec != 0;
     float4 ra[NV4], rb[NV4];
     if (nkb > 0) {
-        load_tile<AK, false, SEG, BK>(p.a, av, p.m, kend, m0, kbeg, tid, ra);
-        load_tile<BKM, BSHIFT, SEG, BK>(p.b, bv, p.n, kend, n0, kbeg, tid, rb);
+        load_tile<AK, false, BK>(p.a, av, p.m, kend, m0, kbeg, tid, ra);
+        load_tile<BKM, BSHIFT, BK>(p.b, bv, p.n, kend, n0, kbeg, tid, rb);
         store_tile<AK, AK, BK>(As0, tid, av, ra);
         store_tile<BKM, 1, BK>(Bs0, tid, bv, rb);
     }
@@ -463,8 +438,8 @@ __device__ __forceinline__ void mainloop(const GemmArgs& p, int m0, int n0, int 
         float* bs_n = (kb & 1) ? Bs0 : Bs1;
         const bool more = kb + 1 < nkb;
         if (more) {
-            load_tile<AK, false, SEG, BK>(p.a, av, p.m, kend, m0, kbeg + (kb + 1) * BK, tid, ra);
-            load_tile<BKM, BSHIFT, SEG, BK>(p.b, bv, p.n, kend, n0, kbeg + (kb + 1) * BK, tid, rb);
+            load_tile<AK, false, BK>(p.a, av, p.m, kend, m0, kbeg + (kb + 1) * BK, tid, ra);
+            load_tile<BKM, BSHIFT, BK>(p.b, bv, p.n, kend, n0, kbeg + (kb + 1) * BK, tid, rb);
         }
         if constexpr (!IDLE) mma_tile<AK, BK>(as, bs, lane, wm, wn, tid, colsum, cs, acc);
         if (more) {
@@ -522,19 +497,19 @@ constexpr int kDmaTile = 16 * BM;  // floats per operand tile
 // the last four, `rows` being a multiple of 4 there), so every load stays
 // inside the operand; the products of those rows land in outputs that are
 // not stored.
-template <int KMAJOR, bool SHIFT, bool SEG, bool ROT, int R = BM, bool CLAMP = false>
+template <int KMAJOR, bool SHIFT, bool ROT, int R = BM, bool CLAMP = false>
 __device__ __forceinline__ const float* dma_src(const GemmOperand& op, int r0, int k0, int s, int rows = 0) {
     if constexpr (KMAJOR == 1) {
         int r = r0 + 4 * (s % (R / 4));
         if constexpr (CLAMP) r = min(r, rows - 4);
-        return elem_ptr<1, SHIFT, SEG>(op, r, k0 + s / (R / 4));
+        return elem_ptr<1, SHIFT>(op, r, k0 + s / (R / 4));
     } else {
         const int t = s >> 2;
         const int kq = (s & 3) ^ ((t >> 2) & 3);
         const int row = ROT ? (t & ~63) | ((t & 15) << 2) | ((t >> 4) & 3) : t;
         int r = r0 + row;
         if constexpr (CLAMP) r = min(r, rows - 1);
-        return elem_ptr<0, false, SEG>(op, r, k0 + 4 * kq);
+        return elem_ptr<0, false>(op, r, k0 + 4 * kq);
     }
 }
 
@@ -569,7 +544,7 @@ __device__ __forceinline__ void wait_vmcnt(int n) {
 // the same MFMA code.  Edge tiles clamp their loads (dma_src).  IDLE: a
 // wavefront whose 64x64 quadrant holds no output issues its share of the
 // loads and the barriers but no MFMAs.
-template <int AK, int BKM, bool BSHIFT, bool SEG, bool IDLE = false>
+template <int AK, int BKM, bool BSHIFT, bool IDLE = false>
 __device__ __forceinline__ void mainloop_dma(const GemmArgs& p, int m0, int n0, int kbeg, int kend, int tid, int lane,
                                              int wm, int wn, bool colsum, float& cs, float* smem,
                                              floatx4 (&acc)[4][4]) {
@@ -584,9 +559,9 @@ __device__ __forceinline__ void mainloop_dma(const GemmArgs& p, int m0, int n0, 
 #pragma unroll
             for (int d = 0; d < 2; ++d) {
                 const int s0 = 64 * (2 * wave + d);  // first chunk of this wave's 1 KB block
-                lds_dma16(dma_src<AK, false, SEG, false, BM, true>(p.a, m0, k0, s0 + lane, p.m),
+                lds_dma16(dma_src<AK, false, false, BM, true>(p.a, m0, k0, s0 + lane, p.m),
                           a_stage(st) + 4 * s0);
-                lds_dma16(dma_src<BKM, BSHIFT, SEG, true, BM, true>(p.b, n0, k0, s0 + lane, p.n),
+                lds_dma16(dma_src<BKM, BSHIFT, true, BM, true>(p.b, n0, k0, s0 + lane, p.n),
                           b_stage(st) + 4 * s0);
             }
             return;
@@ -601,10 +576,10 @@ __device__ __forceinline__ void mainloop_dma(const GemmArgs& p, int m0, int n0, 
             const int ka = AK == 1 ? k0 + sc / 32 : k0 + 4 * ((sc & 3) ^ ((sc >> 4) & 3));
             const int kb2 = BKM == 1 ? k0 + sc / 32 : k0 + 4 * ((sc & 3) ^ ((sc >> 4) & 3));
             v[2 * d] = ka < kend ? *reinterpret_cast<const float4*>(
-                                       dma_src<AK, false, SEG, false, BM, true>(p.a, m0, k0, sc, p.m))
+                                       dma_src<AK, false, false, BM, true>(p.a, m0, k0, sc, p.m))
                                  : make_float4(0.f, 0.f, 0.f, 0.f);
             v[2 * d + 1] = kb2 < kend ? *reinterpret_cast<const float4*>(
-                                            dma_src<BKM, BSHIFT, SEG, true, BM, true>(p.b, n0, k0, sc, p.n))
+                                            dma_src<BKM, BSHIFT, true, BM, true>(p.b, n0, k0, sc, p.n))
                                       : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         // the ring's DMA loads are counted on the same counter: wait for all
@@ -655,7 +630,7 @@ constexpr int gemm_smem_floats() {
 // Epilogue of one output tile: acc[a][b][r] is C(row(a, 4 g + r), n0 + 64 wn
 // + 4 c + b); a lane's four b values are one float4 of a C row (a partial
 // row of slice bz in split mode).
-template <int AK, bool SPLIT, bool SEG>
+template <int AK, bool SPLIT>
 __device__ __forceinline__ void store_c(const GemmArgs& p, int m0, int n0, int bz, int wm, int wn, int lane,
                                         const floatx4 (&acc)[4][4]) {
     const int c = lane & 15, g = lane >> 4;
@@ -687,7 +662,7 @@ __device__ __forceinline__ void store_c(const GemmArgs& p, int m0, int n0, int b
                 v.y += bias4.y;
                 v.z += bias4.z;
                 v.w += bias4.w;
-                dst = p.c + (size_t)seg_map<SEG>(p.c_seg, m) * p.ldc + n;
+                dst = p.c + (size_t)m * p.ldc + n;
             }
             if (vec_store) {
                 if (!SPLIT) {
@@ -709,7 +684,7 @@ __device__ __forceinline__ void store_c(const GemmArgs& p, int m0, int n0, int b
 }
 
 // One output tile (bx, by) of k-chunk bz.
-template <int AK, int BKM, bool BSHIFT, bool SPLIT, bool SEG, int BK, bool UA>
+template <int AK, int BKM, bool BSHIFT, bool SPLIT, int BK, bool UA>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bx, int by, int bz, float* smem) {
     constexpr int AF = lds_tile_floats<AK, BK>();
     constexpr int BF = lds_tile_floats<1, BK>();
@@ -744,38 +719,33 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& p, int bx, int by, int
     if (kDma && (!UA || (p.a_vec && p.b_vec))) {
         // both operands float4-capable (always so in the aligned instances)
         if (idle) {
-            mainloop_dma<AK, BKM, BSHIFT, SEG, true>(p, m0, n0, kbeg, kend, tid, lane, wm, wn, false, cs, smem, acc);
+            mainloop_dma<AK, BKM, BSHIFT, true>(p, m0, n0, kbeg, kend, tid, lane, wm, wn, false, cs, smem, acc);
             return;
         }
-        mainloop_dma<AK, BKM, BSHIFT, SEG>(p, m0, n0, kbeg, kend, tid, lane, wm, wn, colsum, cs, smem, acc);
+        mainloop_dma<AK, BKM, BSHIFT>(p, m0, n0, kbeg, kend, tid, lane, wm, wn, colsum, cs, smem, acc);
     } else {
         if (idle) {
-            mainloop<AK, BKM, BSHIFT, SEG, BK, UA, true>(p, m0, n0, kbeg, kend, nkb, tid, lane, wm, wn, false, cs, As0,
+            mainloop<AK, BKM, BSHIFT, BK, UA, true>(p, m0, n0, kbeg, kend, nkb, tid, lane, wm, wn, false, cs, As0,
                                                          As1, Bs0, Bs1, acc);
             return;
         }
-        mainloop<AK, BKM, BSHIFT, SEG, BK, UA>(p, m0, n0, kbeg, kend, nkb, tid, lane, wm, wn, colsum, cs, As0, As1, Bs0,
+        mainloop<AK, BKM, BSHIFT, BK, UA>(p, m0, n0, kbeg, kend, nkb, tid, lane, wm, wn, colsum, cs, As0, As1, Bs0,
                                            Bs1, acc);
     }
-    store_c<AK, SPLIT, SEG>(p, m0, n0, bz, wm, wn, lane, acc);
+    store_c<AK, SPLIT>(p, m0, n0, bz, wm, wn, lane, acc);
     if (colsum && tid < BM && m0 + tid < p.m) {
         float* cpart = p.partial + (size_t)p.ksplit_total * p.m * p.n;
         cpart[(size_t)(p.z_off + bz) * p.m + m0 + tid] = cs;
     }
 }
 
-template <int AK, int BKM, bool BSHIFT, bool SPLIT, bool SEG, bool UA, int BK = SPLIT ? kSplitBK : kDirectBK>
+template <int AK, int BKM, bool UA>
 __global__ __launch_bounds__(NT) void gemm_f32_kernel(GemmArgs p) {
-    __shared__ __attribute__((aligned(16))) float smem[gemm_smem_floats<AK, BK>()];
-    int bx, by, bz = 0;
-    if (SPLIT) {
-        split_coords(p, blockIdx.x, bx, by, bz);
-    } else {
-        direct_coords(p, blockIdx.x, bx, by);
-        for (size_t i = (size_t)blockIdx.x * NT + threadIdx.x; i < p.zero_words; i += (size_t)gridDim.x * NT)
-            p.zero[i] = 0ull;
-    }
-    gemm_tile<AK, BKM, BSHIFT, SPLIT, SEG, BK, UA>(p, bx, by, bz, smem);
+    __shared__ __attribute__((aligned(16))) float smem[gemm_smem_floats<AK, kDirectBK>()];
+    int bx, by;
+    direct_coords(p, blockIdx.x, bx, by);
+    for (size_t i = (size_t)blockIdx.x * NT + threadIdx.x; i < p.zero_words; i += (size_t)gridDim.x * NT) p.zero[i] = 0ull;
+    gemm_tile<AK, BKM, false, false, kDirectBK, UA>(p, bx, by, 0, smem);
 }
 
 // Two split-K products of k-major operands in one launch: workgroups
@@ -783,17 +753,17 @@ __global__ __launch_bounds__(NT) void gemm_f32_kernel(GemmArgs p) {
 // gradients dW_hh, whose B operand is row-remapped, and dW_ih).  One launch
 // of both at half the slices each keeps three workgroups per CU with half
 // the partial sums and one ramp-up and tail instead of two.
-template <bool SHIFT0, bool SEG, bool UA>
+template <bool UA>
 __global__ __launch_bounds__(NT) void gemm_f32_pair_kernel(GemmArgs p0, GemmArgs p1) {
     __shared__ __attribute__((aligned(16))) float smem[gemm_smem_floats<1, kSplitBK>()];
     const int blocks0 = p0.tiles * p0.ksplit;
     int bx, by, bz;
     if ((int)blockIdx.x < blocks0) {
         split_coords(p0, blockIdx.x, bx, by, bz);
-        gemm_tile<1, 1, SHIFT0, true, SEG, kSplitBK, UA>(p0, bx, by, bz, smem);
+        gemm_tile<1, 1, true, true, kSplitBK, UA>(p0, bx, by, bz, smem);
     } else {
         split_coords(p1, blockIdx.x - blocks0, bx, by, bz);
-        gemm_tile<1, 1, false, true, SEG, kSplitBK, UA>(p1, bx, by, bz, smem);
+        gemm_tile<1, 1, false, true, kSplitBK, UA>(p1, bx, by, bz, smem);
     }
 }
 
@@ -897,10 +867,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(ReduceJob j0, Reduce
 // its weight-gradient reductions are independent: the reductions stream
 // partial sums from HBM while the product keeps the matrix cores busy, on
 // the workgroup slots the product's tiles leave free.
-template <int AK, int BKM, bool UA>
+template <bool UA>
 __global__ __launch_bounds__(NT) void gemm_direct_reduce_kernel(GemmArgs p, ReduceJob j0, ReduceJob j1) {
     static_assert(NT == 256, "reduction teams assume 256-thread workgroups");
-    __shared__ __attribute__((aligned(16))) float smem[gemm_smem_floats<AK, kDirectBK>()];
+    __shared__ __attribute__((aligned(16))) float smem[gemm_smem_floats<0, kDirectBK>()];
     if ((int)blockIdx.x >= p.tiles) {
         // (large products: many slices)
         reduce_range_t<kTeam>(j0, j1, (int)blockIdx.x - p.tiles, (int)gridDim.x - p.tiles);
@@ -908,7 +878,7 @@ __global__ __launch_bounds__(NT) void gemm_direct_reduce_kernel(GemmArgs p, Redu
     }
     int bx, by;
     direct_coords(p, blockIdx.x, bx, by);
-    gemm_tile<AK, BKM, false, false, false, kDirectBK, UA>(p, bx, by, 0, smem);
+    gemm_tile<0, 1, false, false, kDirectBK, UA>(p, bx, by, 0, smem);
 }
 
 // ------------------------------------------------------- small products ---
@@ -953,7 +923,7 @@ __device__ __forceinline__ void narrow_block(const GemmArgs& p, int id, float* l
         for (int i = threadIdx.x; i < kNarrowSlab * kNarrowMax; i += 256) {
             const int kk = i / kNarrowMax, j = i % kNarrowMax;
             const int k = k0 + kk;
-            bs[kk][j] = (j < p.narrow && k < kend) ? *elem_ptr<1, BSHIFT, false>(p.b, n0 + j, k) : 0.f;
+            bs[kk][j] = (j < p.narrow && k < kend) ? *elem_ptr<1, BSHIFT>(p.b, n0 + j, k) : 0.f;
         }
         __syncthreads();
         const int kq = k0 + 64 * q;
@@ -987,12 +957,11 @@ __device__ __forceinline__ void narrow_block(const GemmArgs& p, int id, float* l
 
 constexpr int kNarrowSmemBytes = (kNarrowSlab + 4 * 64) * kNarrowMax * (int)sizeof(float);
 
-template <bool BSHIFT0>
 __global__ __launch_bounds__(256) void gemm_narrow_kernel(GemmArgs p0, GemmArgs p1, int blocks0) {
     __shared__ __attribute__((aligned(16))) float smem[kNarrowSmemBytes / sizeof(float)];
     const int id = (int)blockIdx.x;
     if (id < blocks0)
-        narrow_block<BSHIFT0>(p0, id, smem);
+        narrow_block<true>(p0, id, smem);
     else
         narrow_block<false>(p1, id - blocks0, smem);
 }
@@ -1026,7 +995,7 @@ int narrow_cols(int n) {
 }
 
 // The narrow columns of the weight-gradient pair (after the tiles' launch).
-int launch_narrow_pair(const GemmArgs& p0, const GemmArgs& p1, bool shift0, hipStream_t stream) {
+int launch_narrow_pair(const GemmArgs& p0, const GemmArgs& p1, hipStream_t stream) {
     auto blocks = [](const GemmArgs& p) -> long long {
         return p.narrow ? (long long)((p.m + 63) / 64) * p.ksplit : 0;
     };
@@ -1034,45 +1003,7 @@ int launch_narrow_pair(const GemmArgs& p0, const GemmArgs& p1, bool shift0, hipS
     if (b0 + b1 == 0) return 0;
     if (b0 + b1 > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
     const dim3 grid((unsigned)(b0 + b1));
-    if (shift0)
-        hipLaunchKernelGGL((gemm_narrow_kernel<true>), grid, dim3(256), 0, stream, p0, p1, (int)b0);
-    else
-        hipLaunchKernelGGL((gemm_narrow_kernel<false>), grid, dim3(256), 0, stream, p0, p1, (int)b0);
-    RKA_RETURN_IF_HIP(hipGetLastError());
-    return 0;
-}
-
-template <int AK, int BKM, bool BSHIFT, bool SPLIT, bool SEG>
-void launch_gemm_kernel(const GemmArgs& args, dim3 grid, hipStream_t stream) {
-    if (args.a_vec && args.b_vec)
-        hipLaunchKernelGGL((gemm_f32_kernel<AK, BKM, BSHIFT, SPLIT, SEG, false>), grid, dim3(NT), 0, stream, args);
-    else
-        hipLaunchKernelGGL((gemm_f32_kernel<AK, BKM, BSHIFT, SPLIT, SEG, true>), grid, dim3(NT), 0, stream, args);
-}
-
-template <bool SPLIT, bool SEG>
-int launch_gemm_t(const GemmArgs& args, dim3 grid, hipStream_t stream) {
-    const int ak = args.a.kmajor, bk = args.b.kmajor;
-    const bool shift = args.b.shift_T > 0;
-    if (shift && !bk) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: the row remap needs a k-major operand");
-    if (SPLIT) {
-        // the weight gradients: both operands k-major
-        if (!ak || !bk) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: split-K products take k-major operands");
-        if (shift)
-            launch_gemm_kernel<1, 1, true, true, SEG>(args, grid, stream);
-        else
-            launch_gemm_kernel<1, 1, false, true, SEG>(args, grid, stream);
-    } else {
-        if (shift) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: the row remap is for split-K products");
-        if (!ak && !bk)
-            launch_gemm_kernel<0, 0, false, false, SEG>(args, grid, stream);
-        else if (!ak)
-            launch_gemm_kernel<0, 1, false, false, SEG>(args, grid, stream);
-        else if (!bk)
-            launch_gemm_kernel<1, 0, false, false, SEG>(args, grid, stream);
-        else
-            launch_gemm_kernel<1, 1, false, false, SEG>(args, grid, stream);
-    }
+    hipLaunchKernelGGL(gemm_narrow_kernel, grid, dim3(256), 0, stream, p0, p1, (int)b0);
     RKA_RETURN_IF_HIP(hipGetLastError());
     return 0;
 }
@@ -1091,13 +1022,26 @@ void finish_args(GemmArgs& args, int ksplit, bool av, bool bv) {
     }
 }
 
-template <bool SPLIT>
-int launch_gemm(GemmArgs args, int ksplit, bool av, bool bv, hipStream_t stream) {
-    finish_args<SPLIT>(args, ksplit, av, bv);
-    const int tm = args.tiles_m, tn = args.tiles / args.tiles_m;
-    const dim3 grid(SPLIT ? tm * tn * ksplit : tm * tn);
-    const bool seg = args.a.seg.len || args.b.seg.len || args.c_seg.len;
-    return seg ? launch_gemm_t<SPLIT, true>(args, grid, stream) : launch_gemm_t<SPLIT, false>(args, grid, stream);
+// A direct product in the ring.
+int launch_ring(GemmArgs args, hipStream_t stream) {
+    finish_args<false>(args, 1, args.a_vec != 0, args.b_vec != 0);
+    auto with = [&](auto ak, auto bk) {
+        constexpr int A = decltype(ak)::value, B = decltype(bk)::value;
+        auto kern = args.a_vec && args.b_vec ? gemm_f32_kernel<A, B, false> : gemm_f32_kernel<A, B, true>;
+        hipLaunchKernelGGL(kern, dim3(args.tiles), dim3(NT), 0, stream, args);
+    };
+    const std::integral_constant<int, 0> rowm;
+    const std::integral_constant<int, 1> km;
+    if (!args.a.kmajor && !args.b.kmajor)
+        with(rowm, rowm);
+    else if (!args.a.kmajor)
+        with(rowm, km);
+    else if (!args.b.kmajor)
+        with(km, rowm);
+    else
+        with(km, km);
+    RKA_RETURN_IF_HIP(hipGetLastError());
+    return 0;
 }
 
 std::atomic<int> g_gemm_tiles{RKA_GEMM_TILES_AUTO};
@@ -1234,10 +1178,12 @@ int describe_direct(int m, int n, int k, bool a_kmajor, bool aligned) {
 }
 
 int gemm_direct(int m, int n, int k, const GemmOperand& a, const GemmOperand& b,
-                const float* bias, float* c, int ldc, hipStream_t stream, SegMap c_seg,
+                const float* bias, float* c, int ldc, hipStream_t stream,
                 unsigned long long* zero, size_t zero_words) {
     if (m <= 0 || n <= 0 || k < 0) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: m and n must be positive");
     if (!a.ptr || !b.ptr || !c) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: null operand");
+    if (a.shift_T > 0 || b.shift_T > 0)
+        return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: the row remap is for split-K products");
     if ((long long)((m + BM - 1) / BM) * ((n + BN - 1) / BN) > 0x7fffffff) return fail(RKA_ERR_UNSUPPORTED_SHAPE, "gemm: grid too large");
     RKA_RETURN_IF_ERR(check_ld(a, b));
     GemmArgs args{};
@@ -1251,16 +1197,12 @@ int gemm_direct(int m, int n, int k, const GemmOperand& a, const GemmOperand& b,
     args.c = c;
     args.ldc = ldc;
     args.c_vec = (ldc % 4 == 0 && aligned16(c)) ? 1 : 0;
-    args.c_seg = c_seg;
     args.zero = zero;
     args.zero_words = zero ? zero_words : 0;
-    if (!(a.seg.len || b.seg.len || c_seg.len || a.shift_T > 0 || b.shift_T > 0)) {
-        args.a_vec = vec_ok(a, m, k) ? 1 : 0;
-        args.b_vec = vec_ok(b, n, k) ? 1 : 0;
-        const DirectTile tile = direct_tile(args);
-        if (tile != TILE_128) return launch_small(tile, args, nullptr, nullptr, 0, stream);
-    }
-    return launch_gemm<false>(args, 1, vec_ok(a, m, k), vec_ok(b, n, k), stream);
+    args.a_vec = vec_ok(a, m, k) ? 1 : 0;
+    args.b_vec = vec_ok(b, n, k) ? 1 : 0;
+    const DirectTile tile = direct_tile(args);
+    return tile == TILE_128 ? launch_ring(args, stream) : launch_small(tile, args, nullptr, nullptr, 0, stream);
 }
 
 size_t splitk_partial_floats(int m, int n, int ksplit) {
@@ -1370,9 +1312,9 @@ int launch_small_pair(const SplitProduct& p0, const SplitProduct& p1, bool direc
                       const GemmArgs& a1, hipStream_t stream) {
     return launch_pair_tiles(p0, p1, direct, a0, a1, S::TM, S::TN, [&](dim3 grid, const GemmArgs& x, const GemmArgs& y) {
         if (a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec)
-            hipLaunchKernelGGL((gemm_small_pair_kernel<S, true, true>), grid, dim3(NT), 0, stream, x, y);
+            hipLaunchKernelGGL((gemm_small_pair_kernel<S, true>), grid, dim3(NT), 0, stream, x, y);
         else
-            hipLaunchKernelGGL((gemm_small_pair_kernel<S, true, false>), grid, dim3(NT), 0, stream, x, y);
+            hipLaunchKernelGGL((gemm_small_pair_kernel<S, false>), grid, dim3(NT), 0, stream, x, y);
     });
 }
 }  // namespace
@@ -1431,13 +1373,6 @@ int split_args(int m, int n, int k, const GemmOperand& a, const GemmOperand& b, 
 
 }  // namespace
 
-int gemm_splitk_partials(int m, int n, int k, const GemmOperand& a, const GemmOperand& b, bool want_colsum,
-                         float* partial, int ksplit, int z_off, int ksplit_total, hipStream_t stream) {
-    GemmArgs args;
-    RKA_RETURN_IF_ERR(split_args(m, n, k, a, b, want_colsum, partial, ksplit, z_off, ksplit_total, false, &args));
-    return launch_gemm<true>(args, ksplit, args.a_vec != 0, args.b_vec != 0, stream);
-}
-
 int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan,
                               hipStream_t stream) {
     GemmArgs a0, a1;
@@ -1445,15 +1380,13 @@ int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, co
                                  p0.ksplit, true, &a0));
     RKA_RETURN_IF_ERR(split_args(p1.m, p1.n, p1.k, p1.a, p1.b, p1.colsum != nullptr, p1.partial, p1.ksplit, 0,
                                  p1.ksplit, true, &a1));
-    if (p1.b.shift_T > 0) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: only the first product of a pair is remapped");
-    const bool seg = a0.a.seg.len || a0.b.seg.len || a1.a.seg.len || a1.b.seg.len;
-    if (seg) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: pair products take whole operands");
-    if (plan.form != PAIR_RING) {
-        if (p0.b.shift_T <= 0 || !p0.colsum || !p1.colsum || p0.ksplit != plan.ks0 || p1.ksplit != plan.ks1)
-            return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: not the pair of the plan");
-        if (plan.form == PAIR_64) return launch_small_pair<Tile64>(p0, p1, plan.direct, a0, a1, stream);
-        if (plan.form == PAIR_128x64) return launch_small_pair<Tile128x64>(p0, p1, plan.direct, a0, a1, stream);
-        const bool vec = a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec;
+    if (p0.b.shift_T <= 0 || p1.b.shift_T > 0 || !p0.colsum || !p1.colsum || p0.ksplit != plan.ks0 ||
+        p1.ksplit != plan.ks1)
+        return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: not the pair of the plan");
+    const bool vec = a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec;
+    if (plan.form == PAIR_64) return launch_small_pair<Tile64>(p0, p1, plan.direct, a0, a1, stream);
+    if (plan.form == PAIR_128x64) return launch_small_pair<Tile128x64>(p0, p1, plan.direct, a0, a1, stream);
+    if (plan.form == PAIR_SPLIT) {
         auto kern = vec ? gemm_split_pair_kernel<false> : gemm_split_pair_kernel<true>;
         return launch_pair_tiles(p0, p1, plan.direct, a0, a1, kSplitTile, kSplitTile,
                                  [&](dim3 grid, const GemmArgs& x, const GemmArgs& y) {
@@ -1461,20 +1394,10 @@ int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, co
                                  });
     }
     const dim3 grid(a0.tiles * a0.ksplit + a1.tiles * a1.ksplit);
-    const bool ua = !(a0.a_vec && a0.b_vec && a1.a_vec && a1.b_vec);
-    if (p0.b.shift_T > 0) {
-        if (ua)
-            hipLaunchKernelGGL((gemm_f32_pair_kernel<true, false, true>), grid, dim3(NT), 0, stream, a0, a1);
-        else
-            hipLaunchKernelGGL((gemm_f32_pair_kernel<true, false, false>), grid, dim3(NT), 0, stream, a0, a1);
-    } else {
-        if (ua)
-            hipLaunchKernelGGL((gemm_f32_pair_kernel<false, false, true>), grid, dim3(NT), 0, stream, a0, a1);
-        else
-            hipLaunchKernelGGL((gemm_f32_pair_kernel<false, false, false>), grid, dim3(NT), 0, stream, a0, a1);
-    }
+    auto kern = vec ? gemm_f32_pair_kernel<false> : gemm_f32_pair_kernel<true>;
+    hipLaunchKernelGGL(kern, grid, dim3(NT), 0, stream, a0, a1);
     RKA_RETURN_IF_HIP(hipGetLastError());
-    return launch_narrow_pair(a0, a1, p0.b.shift_T > 0, stream);
+    return launch_narrow_pair(a0, a1, stream);
 }
 
 namespace {
@@ -1508,35 +1431,18 @@ ReduceJob reduce_job(const SplitProduct& p) {
 }
 }  // namespace
 
-int splitk_reduce(const SplitProduct& p, hipStream_t stream) {
-    return launch_reduce(reduce_job(p), ReduceJob{}, stream);
-}
-
 int splitk_reduce_pair(const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan, hipStream_t stream) {
     if (plan.direct) return 0;
     return launch_reduce(reduce_job(p0), reduce_job(p1), stream);
 }
-
-namespace {
-template <int AK, int BKM>
-void launch_direct_reduce(const GemmArgs& args, const ReduceJob& j0, const ReduceJob& j1, dim3 grid,
-                          hipStream_t stream) {
-    if (args.a_vec && args.b_vec)
-        hipLaunchKernelGGL((gemm_direct_reduce_kernel<AK, BKM, false>), grid, dim3(NT), 0, stream, args, j0, j1);
-    else
-        hipLaunchKernelGGL((gemm_direct_reduce_kernel<AK, BKM, true>), grid, dim3(NT), 0, stream, args, j0, j1);
-}
-}  // namespace
 
 int gemm_direct_reduce_pair(int m, int n, int k, const GemmOperand& a, const GemmOperand& b, float* c, int ldc,
                             const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan, hipStream_t stream) {
     if (m <= 0 || n <= 0 || k < 0) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: m and n must be positive");
     if (!a.ptr || !b.ptr || !c) return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: null operand");
     RKA_RETURN_IF_ERR(check_ld(a, b));
-    if (a.seg.len || b.seg.len || b.shift_T > 0) {
-        RKA_RETURN_IF_ERR(splitk_reduce_pair(p0, p1, plan, stream));
-        return gemm_direct(m, n, k, a, b, nullptr, c, ldc, stream);
-    }
+    if (a.kmajor || !b.kmajor || a.shift_T > 0 || b.shift_T > 0)
+        return fail(RKA_ERR_INVALID_ARGUMENT, "gemm: the input gradient takes a row-major and a k-major operand");
     const DeviceInfo* dev = nullptr;
     RKA_RETURN_IF_ERR(current_device_info(&dev));
     GemmArgs args{};
@@ -1564,21 +1470,10 @@ int gemm_direct_reduce_pair(int m, int n, int k, const GemmOperand& a, const Gem
         const long most = (tile == TILE_SPLIT ? 1 : 4) * reducers;
         return launch_small(tile, args, &j0, &j1, (long)std::min<size_t>(want, most), stream);
     }
-    if (!a.kmajor && !b.kmajor)
-        launch_direct_reduce<0, 0>(args, j0, j1, grid, stream);
-    else if (!a.kmajor)
-        launch_direct_reduce<0, 1>(args, j0, j1, grid, stream);
-    else if (!b.kmajor)
-        launch_direct_reduce<1, 0>(args, j0, j1, grid, stream);
-    else
-        launch_direct_reduce<1, 1>(args, j0, j1, grid, stream);
+    auto kern = args.a_vec && args.b_vec ? gemm_direct_reduce_kernel<false> : gemm_direct_reduce_kernel<true>;
+    hipLaunchKernelGGL(kern, grid, dim3(NT), 0, stream, args, j0, j1);
     RKA_RETURN_IF_HIP(hipGetLastError());
     return 0;
-}
-
-int splitk_reduce(int m, int n, const float* partial, int ksplit_total, int rot, float* c, int ldc,
-                  float* colsum, hipStream_t stream) {
-    return launch_reduce(reduce_job(m, n, partial, ksplit_total, rot, c, ldc, colsum), ReduceJob{}, stream);
 }
 
 }  // namespace rka

@@ -442,14 +442,14 @@ __global__ __launch_bounds__(NT) void gemm_small_reduce_kernel(GemmArgs p, Reduc
 }
 
 // The two split-K weight-gradient products in one launch (gemm_f32_pair_kernel).
-template <typename S, bool SHIFT0, bool VEC>
+template <typename S, bool VEC>
 __global__ __launch_bounds__(NT, S::TM == 64 ? 4 : 2) void gemm_small_pair_kernel(GemmArgs p0, GemmArgs p1) {
     __shared__ __attribute__((aligned(16))) float smem[S::template smem<1, 1>()];
     const int blocks0 = p0.tiles * p0.ksplit;
     int bx, by, bz;
     if ((int)blockIdx.x < blocks0) {
         split_coords(p0, blockIdx.x, bx, by, bz);
-        small_tile<1, 1, S, VEC, true, SHIFT0>(p0, bx, by, bz, smem);
+        small_tile<1, 1, S, VEC, true, true>(p0, bx, by, bz, smem);
     } else {
         split_coords(p1, blockIdx.x - blocks0, bx, by, bz);
         small_tile<1, 1, S, VEC, true, false>(p1, bx, by, bz, smem);

@@ -218,7 +218,7 @@ int rka_gru_forward(const float* x, const float* h0, const float* w_ih, const fl
     const size_t rec_words = (rec_workspace_bytes(0, B, H) - rec_off) / sizeof(unsigned long long);
     {
         StageScope scope(0, s);
-        RKA_RETURN_IF_ERR(gemm_direct(B * T, 3 * H, I, a, b, b_ih, gx, 3 * H, s, SegMap{}, rec_state, rec_words));
+        RKA_RETURN_IF_ERR(gemm_direct(B * T, 3 * H, I, a, b, b_ih, gx, 3 * H, s, rec_state, rec_words));
     }
     StageScope scope(1, s);
     return launch_rec_forward(gx, h0, w_hh, b_hh, y, hn, reserve, ws + l.rec, l.total - l.rec, B, T, H, s,

@@ -47,14 +47,6 @@ int current_device_info(const DeviceInfo** out);
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // ----------------------------------------------------------------- GEMM ---
-// Segment map of a row index i of the underlying 2-D array:
-// len == 0: i; else (i / len) * stride + off + i % len.  With len = L,
-// stride = T, off = t0 it selects rows (b, t0 .. t0+L-1) of a [B, T, .]
-// tensor, i.e. one time chunk of every sequence.
-struct SegMap {
-    int len = 0, stride = 0, off = 0;
-};
-
 struct GemmOperand {
     const float* ptr = nullptr;
     int ld = 0;
@@ -65,25 +57,14 @@ struct GemmOperand {
     // [h0 ; y[:, :-1]] without materialising them.
     int shift_T = 0;
     const float* shift_first = nullptr;
-    // applied first to the underlying row (k if kmajor, else r)
-    SegMap seg{};
 };
 
-// C[m,n] = sum_k A(m,k) B(n,k) + bias[n]; direct store (row m of C at
-// c_seg(m)).
+// C[m,n] = sum_k A(m,k) B(n,k) + bias[n].
 // zero / zero_words: a buffer of 64-bit words the launch also clears (the
 // next kernel's exchange state, so that it needs no fill launch of its own).
 int gemm_direct(int m, int n, int k, const GemmOperand& a, const GemmOperand& b,
-                const float* bias, float* c, int ldc, hipStream_t stream, SegMap c_seg = SegMap{},
+                const float* bias, float* c, int ldc, hipStream_t stream,
                 unsigned long long* zero = nullptr, size_t zero_words = 0);
-
-// Split-K partial products only: slices [z_off, z_off + ksplit) of a
-// partial buffer holding ksplit_total slices (layout as gemm_splitk).
-int gemm_splitk_partials(int m, int n, int k, const GemmOperand& a, const GemmOperand& b, bool want_colsum,
-                         float* partial, int ksplit, int z_off, int ksplit_total, hipStream_t stream);
-// out[o] = sum of the ksplit_total slices at row (o + rot) % m; colsum likewise.
-int splitk_reduce(int m, int n, const float* partial, int ksplit_total, int rot, float* c, int ldc,
-                  float* colsum, hipStream_t stream);
 
 // Split-K products reduce deterministically.  Output rows are rotated:
 // out[o] = C[(o + rot) % m] (rot = 0: no rotation).  colsum (nullable)
@@ -120,12 +101,10 @@ PairPlan plan_pair(int m, int n0, int n1, int k);
 // The most slices over every tile mode, which sizes the workspace.
 void pair_ksplit_bound(int m, int n0, int n1, int k, int* ks0, int* ks1);
 // The partial products of two split-K products in one launch (all slices
-// of each, or the results); only p0's B operand may carry the row remap.
+// of each, or the results); p0's B operand carries the row remap.
 int gemm_splitk_pair_partials(const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan,
                               hipStream_t stream);
-int splitk_reduce(const SplitProduct& p, hipStream_t stream);
-// Both products' reductions in one launch (the same results as two
-// splitk_reduce calls).
+// Both products' reductions in one launch.
 int splitk_reduce_pair(const SplitProduct& p0, const SplitProduct& p1, const PairPlan& plan, hipStream_t stream);
 // gemm_direct (no bias) and splitk_reduce_pair(p0, p1) in one launch: the
 // same results as the two calls.
