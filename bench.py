@@ -52,7 +52,7 @@ MFMA_FP32_PEAK_TFLOPS = 157.3
 # independent FMA chains), and valu_frac and the step floor use that rate.
 HBM_PEAK_GBS = 8000.0
 RECURRENCES = ("forward_recurrence", "backward_recurrence")
-CPU_THREAD_CAP = 16  # the GPU box's CPU share for one GPU, whatever os.cpu_count() reports
+CPU_THREAD_CAP = 16  # CPU share of one GPU of a node, whatever os.cpu_count() reports
 
 
 def flops_per_step(B, T, I, H):

@@ -43,8 +43,8 @@ def compile_flags() -> list:
         "-std=c++17",
         "-fPIC",
         f"--offload-arch={ARCH}",
-        # Packed fp32 VALU ops are kept off on this pool (known-bad forms);
-        # the hot dot products are written as scalar fmaf chains.
+        # Packed fp32 VALU ops are kept off (some of their forms have given wrong
+        # results); the hot dot products are written as scalar fmaf chains.
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
         "-Wall",
         "-Wno-unused-command-line-argument",

@@ -1,8 +1,8 @@
 // fp32 products on the bf16 matrix cores, for the large ones: a float32 is the
 // exact sum of three bf16 values (24 mantissa bits in three rounded pieces of 8,
 // x = p0 + p1 + p2), so a product of two is nine bf16 products, each exact in
-// float32.  The three smallest (p1 q2, p2 q1, p2 q2, together below 2^-25 of
-// the product) are left out, the other six go to v_mfma_f32_32x32x16_bf16,
+// float32.  The three smallest (p1 q2, p2 q1, p2 q2, together at most about 2^-24
+// of the product) are left out, the other six go to v_mfma_f32_32x32x16_bf16,
 // smallest first, into one float32 accumulator: six matrix instructions of 32
 // clocks per 32x32x16 block where the fp32 ones (32x32x2) take eight of 64.
 // Included by gemm_f32.hip, whose GemmArgs and tile orders it shares.

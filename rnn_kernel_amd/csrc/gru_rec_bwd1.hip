@@ -3,7 +3,7 @@
 // sixteen wavefronts, one batch row per workgroup), in a translation unit of
 // their own: the build compiles this file with LLVM's max-ilp machine
 // scheduler (-mllvm -amdgpu-sched-strategy=max-ilp), a per-translation-unit
-// option.  Measured on MI355X (same box, alternating pairs, backward per
+// option.  Measured on MI355X (same GPU, alternating pairs, backward per
 // launch): c2 (H = 256) 402.0-406.6 vs 409.6-414.9 us, H = 192 367.3-371.1
 // vs 373.1-375.4 us.  Where it measured no faster it is not used: two slices
 // (H = 128: 365 vs 347 us), H = 160 (three slices, not whole: 384 vs 381

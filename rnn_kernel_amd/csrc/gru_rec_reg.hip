@@ -13,7 +13,7 @@ namespace {
 // Compute wavefronts of the one-row forward: sixteen at four slices (every
 // wave has half the FMAs of eight, and the owner stores its own outputs: a
 // workgroup holds at most 1024 threads), else eight plus the I/O wavefront.
-// Measured on MI355X (same box, alternating runs, forward per launch): c2
+// Measured on MI355X (same GPU, alternating runs, forward per launch): c2
 // 434-437 vs 443 us; at one to three slices the I/O wavefront wins (H = 64,
 // 128, 192: 359 / 365 / 403 vs 370 / 389 / 427 us).
 constexpr int fwd_waves1(int S) { return S == 4 ? 16 : 8; }

@@ -261,7 +261,7 @@ __device__ __forceinline__ bool group_on_one_xcd(unsigned long long* words, int 
 // its reader has passed the step, so ready lanes reload the same value).
 // Otherwise each lane leaves the loop when its own words are in, which
 // costs some thirty scalar instructions of exec-mask bookkeeping per round.
-// Measured at c2 (same box, alternating pairs, µs per launch): forward (one
+// Measured at c2 (same GPU, alternating pairs, µs per launch): forward (one
 // word per lane) 445.6-446.4 uniform vs 451.8-453.2 per lane; the backward
 // (several words per lane) 453.5 / 454.7 uniform vs 448.4 / 450.1, and the
 // four-row forward spills with it, so both keep the per-lane loop.

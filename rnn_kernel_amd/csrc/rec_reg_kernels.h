@@ -10,7 +10,7 @@
 // group exchange one word per value and step (h_t forward, G_h,t backward)
 // and sit on one XCD when the group count allows.
 //
-// Measured on MI355X (same box, alternating runs) against the designs this
+// Measured on MI355X (same GPU, alternating runs) against the designs this
 // one replaced:
 //   * wavefronts holding contiguous k (j) chunks with the exchanged words
 //     replicated into 16-lane rows (v_permlane16/32_swap) and broadcast into
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(IO ? NWF * 64 + 64 : NWF * 64) void gru_fwd_local_k
     // kind: 1 = step 0 (its h values come from h0; it runs before the loop,
     // so no later step tests t), 3 = a step with at least one more after it
     // (its tests of t + 1 < T fold away), 0 = tested at run time (the last
-    // steps).  Measured on MI355X (same box, three alternating pairs):
+    // steps).  Measured on MI355X (same GPU, three alternating pairs):
     // without the run-time tests in the bulk of the steps, c2 forward 401 ->
     // 393 us per launch, c5 7.70 -> 7.61 ms, H = 128 and 192 -5.5 and -3 us.
     auto step = [&](auto kind, int t, const float (&cur)[3], float (&nxt)[3]) -> bool {
@@ -1275,7 +1275,7 @@ __global__ __launch_bounds__(64 * NWB) void gru_bwd_local_kernel(
             // streaming stores: G is read once, by the gradient GEMMs after
             // this kernel, so it need not take MALL space from the reserve,
             // y and dy this kernel still has to read (backward 0.449 vs
-            // 0.467 ms per c2 launch, same-box A/B)
+            // 0.467 ms per c2 launch, same-GPU A/B)
             float* op = g_r + 4 * (unsigned)t * (unsigned)H;  // wave-uniform
             __builtin_nontemporal_store(o_dan, op + u);
             __builtin_nontemporal_store(o_drh, op + H + u);
@@ -1436,7 +1436,7 @@ __global__ __launch_bounds__(64 * NWB) void gru_bwd_local_kernel(
         using Any = std::integral_constant<int, 0>;
         // Steps followed by at least two more run without the run-time tests
         // of the next step and of the loads two steps ahead (the last steps
-        // keep them).  Measured on MI355X (same box, three alternating
+        // keep them).  Measured on MI355X (same GPU, three alternating
         // pairs): c5 backward 3326-3330 -> 3252-3255 us per launch, H = 128
         // 346-347 -> 338-340 us; the whole-slice instances at three and four
         // slices (built with max-ilp) measured slower with it (c2 +5 us) and

@@ -1,7 +1,7 @@
 """Parity of the HIP path (through the C ABI) with the CPU oracle and with
 torch.nn.GRU fp32 on the same GPU.
 
-Tolerances (stated by the north star): outputs and h_n within max-abs 1e-4;
+Tolerances: outputs and h_n within max-abs 1e-4;
 gradients within max|g - g_ref| / max|g_ref| <= 1e-3 per tensor.  Small shapes
 are checked against the float64 oracle; the BASELINE configurations are
 checked against torch.nn.GRU fp32 (TF32 off) on the same GPU and, for a
