@@ -206,3 +206,32 @@ def test_split_weight_gradients_non_finite(gpu):
         rows = torch.isfinite(p.grad.reshape(3 * H, -1)).all(dim=1)
         assert bool(rows[~bad].all())
         assert not bool(rows[bad].any())
+
+
+@pytest.mark.parametrize("H", [256, 129])  # aligned and unaligned rows
+def test_split_backward_non_finite_leaves_the_rest(gpu, H):
+    """The same with dx (in the launch that also reduces the partial sums): what
+    the infinity does not reach equals the pass without it, bit for bit."""
+    from rnn_kernel_amd import GRUFunction, _lib
+
+    B, T = 64, 512
+    assert _lib.describe_weight_gradients(B, T, H, H)["form"] == "split"
+    assert _lib.describe_gemm(B * T, H, 3 * H, aligned=H % 4 == 0) == "split"
+    g = torch.Generator(device=gpu).manual_seed(H)
+    w = [((torch.rand(*s, generator=g, device=gpu) * 2 - 1) / 16).requires_grad_(True)
+         for s in ((3 * H, H), (3 * H, H), (3 * H,), (3 * H,))]
+    x = torch.randn(B, T, H, generator=g, device=gpu).requires_grad_(True)
+    dy = torch.randn(B, T, H, generator=g, device=gpu)
+    grads = []
+    for value in (dy[3, 0, 17].item(), float("inf")):
+        dy[3, 0, 17] = value
+        y, _ = GRUFunction.apply(x, torch.zeros(B, H, device=gpu), *w)
+        grads.append(torch.autograd.grad(y, [x] + w, dy))
+    bad = torch.zeros(3 * H, dtype=torch.bool, device=gpu)
+    bad[[17, H + 17, 2 * H + 17]] = True
+    hit = torch.zeros(B, T, dtype=torch.bool, device=gpu)
+    hit[3, 0] = True
+    for k, (plain, odd) in enumerate(zip(*grads)):
+        mask = hit if k == 0 else bad
+        assert torch.equal(plain[~mask], odd[~mask])
+        assert not torch.isfinite(odd[mask].reshape(int(mask.sum()), -1)).all(dim=1).any()
