@@ -28,7 +28,7 @@
 // blocks are four adjacent output columns, stored as one float4 (a
 // streaming store for the direct products).  At I = H = 256, B T = 32768 inside
 // the training step (us, ring -> the split form now taken): input projection 119
-// -> 78, dx with the weight-gradient reductions 110 -> 81, the dW pair 233 -> 153.
+// -> 81, dx with the weight-gradient reductions 110 -> 85, the dW pair 233 -> 163.
 // Each operand layout is a
 // template instance, so no product carries another's address arithmetic.
 // The weight gradients (K = B*T rows) use split-K with a fixed-order

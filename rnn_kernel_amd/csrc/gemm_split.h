@@ -14,20 +14,23 @@
 // products brings 9e-8 at k = 256 but costs the third workgroup per CU (94 vs
 // 83 us), and is not used.
 //
-// What bounds it: the matrix cores and LDS about alike (a 16-deep stage of a
-// workgroup is 24 MFMAs per wavefront and 72 KB of LDS traffic).  128x128 tiles
+// What bounds it: nothing alone.  The matrix cores are busy 0.40 to 0.54 of the
+// cycles and the VALU issues on 0.11 to 0.16 of them; the wavefronts wait to issue
+// for 0.35 to 0.46 of theirs and on counters (the loads, LDS) for 0.2 to 0.33, one
+// barrier per 16-deep stage (24 MFMAs per wavefront, 72 KB of LDS traffic per
+// workgroup).  The clock falls to 1.8-1.9 GHz meanwhile.  128x128 tiles
 // of four wavefronts, 64x64 each; the operands are loaded as float32 two stages
 // ahead in registers, split there and written to LDS as three planes (48 KB for
 // two stages: three workgroups per CU).  Measured against the fp32
-// tiles they replace (us): 32768 x 768, k = 256: 113 -> 80; 8192 x 2304, k = 768:
-// 237 -> 166; 16384 x 1536, k = 512: 211 -> 141; the weight-gradient pair 768 x
-// (256 + 256), k = 32768: 229 -> 159, k = 262144: 1725 -> 1186.
+// tiles they replace (us): 32768 x 768, k = 256: 113 -> 81; 8192 x 2304, k = 768:
+// 237 -> 165; 16384 x 1536, k = 512: 211 -> 141; the weight-gradient pair 768 x
+// (256 + 256), k = 32768: 229 -> 162, k = 262144: 1725 -> 1245.
 //
 // Operands without aligned float4 rows (odd sizes; UA, any row length from 4) are
 // loaded in the same float4 from 4-byte-aligned addresses.  Against the fp32
 // register-staged tiles they replace (us): 32768 x 387, k = 129: 60 -> 40; 32768 x
 // 129, k = 387: 58 -> 46; 19200 x 1533, k = 511: 308 -> 190; the pair 387 x (129 +
-// 129), k = 32768: 155 -> 115; 993 x (331 + 331), k = 8192: 152 -> 83.
+// 129), k = 32768: 155 -> 117; 993 x (331 + 331), k = 8192: 152 -> 86.
 //
 // Non-finite values: the pieces of an infinity are not finite sums, so a workgroup
 // one of whose outputs comes out infinite or NaN computes its tile again in 64x64
@@ -52,7 +55,8 @@ constexpr int kSplitStage = 2 * 3 * kPlane;      // dwords of a stage
 // is lost that a float32 holds.  Without the scale the lower pieces of values
 // below some 1e-33 were: error of a product with one operand of 1e-36 2.7e-5
 // (2-norm, against 2.4e-7), of 1e-38 2.7e-3.  Operands from 2^105 or sums from 2^82
-// overflow, and are computed again as other results that are not finite.
+// overflow, and are computed again as other results that are not finite.  The
+// multiplication costs 1 to 3 % of a product (pair at k = 32768: 157 -> 161 us).
 constexpr float kSplitScale = 8388608.f;                  // 2^23
 constexpr float kSplitUnscale = 1.f / kSplitScale / kSplitScale;
 
@@ -84,8 +88,9 @@ __device__ __forceinline__ void split3(float a, float b, float s, unsigned (&p)[
 
 // LDS planes of an operand's stage.  Row-major: [row][16 k] (32 bytes a row;
 // thread x of a pass holds k 4 (x % 4) of row x / 4).  k-major: [k pair][row] of
-// dwords (thread: rows 4 (t % 32) .. + 3 at k 2 (t / 32) and the next).  Every
-// access of either is free of bank conflicts.  s: the scale of the thread's rows
+// dwords (thread: rows 4 (t % 32) .. + 3 at k 2 (t / 32) and the next).  Bank
+// conflicts counted per LDS instruction: 0 with both operands k-major, 1.2 with one,
+// 2.6 cycles with both row-major.  s: the scale of the thread's rows
 // (ALT, k-major: of its even rows, odd ones take -s).
 template <int KMAJOR, bool ALT>
 __device__ __forceinline__ void split_store(unsigned* lds, int tid, float s, const float4 (&v)[2]) {
