@@ -64,11 +64,14 @@ constexpr float kSplitUnscale = 1.f / kSplitScale / kSplitScale;
 // addends hold below the largest one's last bits is cut off): on average -2e-8 of
 // an output's mean magnitude at k = 256, -1.5e-7 at k = 2304, in every row alike.
 // What later sums over rows (the gradients of a stack's lower layers) adds that
-// up, where roundings to nearest cancel.  So A's odd rows are split with the
+// up, where roundings to nearest cancel.  So half of A's rows are split with the
 // opposite sign and their sums negated in the end, which turns the direction of
 // their rounding: the mean over all rows is then below 3e-10, as on the fp32 matrix
-// cores.  In the split-K products odd slices change sign too, so that the error
-// cancels in the sum of the slices (k = 262144: 1.6e-6 -> 8.8e-7).
+// cores.  Which rows is a hash of the row's own values (split_hash), not of its
+// place, so that equal sequences of a batch give equal results.  In the split-K
+// products, whose rows are the gate units, it is the odd rows; odd slices change sign
+// too, so that the error cancels in the sum of the slices (k = 262144: 1.6e-6 ->
+// 8.8e-7).  (Negating the sums every eight stages instead took 2 % of the pair.)
 
 // The three pieces of a and b times s (a scale of either sign), packed in pairs
 // (a low).
@@ -86,31 +89,39 @@ __device__ __forceinline__ void split3(float a, float b, float s, unsigned (&p)[
     }
 }
 
+// The parity of the bits of a row's first sixteen values (of what the first stage
+// loads for them; the four threads of the row hold four each).
+__device__ __forceinline__ bool split_hash(const float4& v) {
+    unsigned h = __float_as_uint(v.x) ^ __float_as_uint(v.y) ^ __float_as_uint(v.z) ^ __float_as_uint(v.w);
+    h ^= __shfl_xor(h, 1, 4);
+    h ^= __shfl_xor(h, 2, 4);
+    return __popc(h) & 1;
+}
+
 // LDS planes of an operand's stage.  Row-major: [row][16 k] (32 bytes a row;
 // thread x of a pass holds k 4 (x % 4) of row x / 4).  k-major: [k pair][row] of
 // dwords (thread: rows 4 (t % 32) .. + 3 at k 2 (t / 32) and the next).  Bank
 // conflicts counted per LDS instruction: 0 with both operands k-major, 1.2 with one,
-// 2.6 cycles with both row-major.  s: the scale of the thread's rows
-// (ALT, k-major: of its even rows, odd ones take -s).
-template <int KMAJOR, bool ALT>
-__device__ __forceinline__ void split_store(unsigned* lds, int tid, float s, const float4 (&v)[2]) {
+// 2.6 cycles with both row-major.  s: the scales of the thread's two rows
+// (row-major), or of its even and odd rows (k-major).
+template <int KMAJOR>
+__device__ __forceinline__ void split_store(unsigned* lds, int tid, const float (&s)[2], const float4 (&v)[2]) {
     if constexpr (KMAJOR == 0) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             unsigned p[3], q[3];
-            split3(v[j].x, v[j].y, s, p);
-            split3(v[j].z, v[j].w, s, q);
+            split3(v[j].x, v[j].y, s[j], p);
+            split3(v[j].z, v[j].w, s[j], q);
 #pragma unroll
             for (int c = 0; c < 3; ++c)
                 *reinterpret_cast<uintx2*>(lds + c * kPlane + (tid + NT * j) * 2) = uintx2{p[c], q[c]};
         }
     } else {
         unsigned p[4][3];
-        const float odd = ALT ? -s : s;
-        split3(v[0].x, v[1].x, s, p[0]);
-        split3(v[0].y, v[1].y, odd, p[1]);
-        split3(v[0].z, v[1].z, s, p[2]);
-        split3(v[0].w, v[1].w, odd, p[3]);
+        split3(v[0].x, v[1].x, s[0], p[0]);
+        split3(v[0].y, v[1].y, s[1], p[1]);
+        split3(v[0].z, v[1].z, s[0], p[2]);
+        split3(v[0].w, v[1].w, s[1], p[3]);
 #pragma unroll
         for (int c = 0; c < 3; ++c)
             *reinterpret_cast<uintx4*>(lds + c * kPlane + (tid / 32) * kSplitTile + 4 * (tid % 32)) =
@@ -291,10 +302,10 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
     const LA la(p.a, p.m, m0, kbeg, klen, tid);
     LB lb(p.b, p.n, n0, kbeg, klen, tid);
     float4 ra[2][2], rb[2][2];
-    // the sign of the tile's even rows; a thread's rows of a row-major A are tid /
-    // 4 and that plus 64, all odd or all even
-    const float sign = SPLIT && (bz & 1) ? -1.f : 1.f;
-    const float scale_a = kSplitScale * (AK ? sign : (tid / 4) % 2 ? -sign : sign);
+    const float sign = SPLIT && (bz & 1) ? -1.f : 1.f;  // of the tile's even rows (k-major A)
+    float scale_a[2] = {sign * kSplitScale, -sign * kSplitScale};
+    const float scale_b[2] = {kSplitScale, kSplitScale};
+    __shared__ __attribute__((aligned(16))) float s_unscale[AK ? 4 : kSplitTile];  // of each row of a row-major A
     floatx16 acc[2][2];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
@@ -345,8 +356,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
                 cs.w += ra[ST][0].w + ra[ST][1].w;
             }
         }
-        split_store<AK, true>(as, tid, scale_a, ra[ST]);
-        split_store<BKM, false>(bs, tid, kSplitScale, rb[ST]);
+        split_store<AK>(as, tid, scale_a, ra[ST]);
+        split_store<BKM>(bs, tid, scale_b, rb[ST]);
         la.load(kb + 2, nkb, klen, tid, ra[ST]);
         lb.load(kb + 2, nkb, klen, tid, rb[ST]);
         __syncthreads();
@@ -373,6 +384,15 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
         lb.load(0, nkb, klen, tid, rb[0]);
         la.load(1, nkb, klen, tid, ra[1]);
         lb.load(1, nkb, klen, tid, rb[1]);
+        if constexpr (!AK) {
+            // (read behind the loop's barriers)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const bool neg = split_hash(ra[0][j]);
+                scale_a[j] = neg ? -kSplitScale : kSplitScale;
+                if (tid % 4 == 0) s_unscale[tid / 4 + 64 * j] = neg ? -kSplitUnscale : kSplitUnscale;
+            }
+        }
         int kb = 0;
         for (; kb + 1 < nkb; kb += 2) {
             stage(kb, std::integral_constant<int, 0>{});
@@ -402,14 +422,14 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int bx, int by, in
 #pragma unroll
         for (int y = 0; y < 2; ++y) bias[y] = p.bias[min(col_of(y), p.n - 1)];
     }
-    const float unscale = sign * kSplitUnscale;
     bool odd = false;  // an output that is not finite
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = row_of(x, r);
-            const float u = (AK ? x : r) % 2 ? -unscale : unscale;  // m odd: the row's sums are negated
+            const float u = AK ? (x ? -sign : sign) * kSplitUnscale  // (m odd: x is 1)
+                               : s_unscale[64 * wm + 32 * x + 8 * (r / 4) + 4 * h + r % 4];
             const float v[2] = {fmaf(acc[x][0][r], u, bias[0]), fmaf(acc[x][1][r], u, bias[1])};
             odd = odd || !__builtin_isfinite(v[0]) || !__builtin_isfinite(v[1]);
             if (m >= p.m) continue;

@@ -110,6 +110,20 @@ def test_split_product_error_has_no_mean(gpu, hip_lib, m, n, k, b_kmajor):
     assert abs(mean.item()) <= 6 * 2.0 ** -24 * (6 * stages / (m * n)) ** 0.5
 
 
+@pytest.mark.parametrize("m,n,k", [(32768, 128, 16), (32768, 128, 256), (32641, 129, 387)])
+@pytest.mark.parametrize("b_kmajor", [0, 1])
+def test_split_product_rows_do_not_depend_on_their_place(gpu, hip_lib, m, n, k, b_kmajor):
+    """Equal sequences of a batch give equal results: a row's result is the same
+    bit for bit wherever the row stands."""
+    print(f"split m={m} n={n} k={k} b_kmajor={b_kmajor}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    a = torch.randn(m, k, generator=g, device=gpu)
+    b = torch.randn((k, n) if b_kmajor else (n, k), generator=g, device=gpu)
+    c = _product(gpu, hip_lib, a, b, b_kmajor)
+    for shift in (1, 37):
+        assert torch.equal(_product(gpu, hip_lib, a.roll(shift, 0).contiguous(), b, b_kmajor), c.roll(shift, 0))
+
+
 @pytest.mark.parametrize("b_kmajor", [0, 1])
 def test_split_product_non_finite(gpu, hip_lib, b_kmajor):
     """Rows with an infinity, a NaN, values that round past the largest bf16 and
